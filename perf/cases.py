@@ -179,3 +179,47 @@ def tolerance(case):
     if case["act"] == "relu" and case["mode"] == "train":
         rel = max(rel, 3e-3)
     return {"rel": rel}
+
+
+def _act64(name, t):
+    if name == "identity":
+        return t
+    if name == "relu":
+        return torch.relu(t)
+    if name == "silu":
+        return torch.nn.functional.silu(t)
+    return torch.nn.functional.gelu(t, approximate="tanh" if name == "gelu_tanh" else "none")
+
+
+def exact(case, seed):
+    """The same outputs in float64 by plain torch, one sample at a time; dweight and dbias are summed over the samples."""
+    state = prepare(case, seed)
+    m, x = state["module"], state["x"].detach()
+    C, G, N = case["C"], case["G"], case["N"]
+    channels = (1, C) + (1,) * (x.dim() - 2)
+    weight, bias = m.weight.detach().double().requires_grad_(True), m.bias.detach().double().requires_grad_(True)
+    rows = {}
+
+    def put(name, n, value):
+        rows.setdefault(name, torch.empty(x.shape, dtype=torch.float64, device=x.device))[n:n + 1] = value
+
+    dweight, dbias = torch.zeros_like(weight), torch.zeros_like(bias)
+    for n in range(N):
+        xn = x[n:n + 1].double()
+        if case["add"]:
+            xn = xn + state["residual"][n:n + 1].double() + state["channel_bias"][n].double().view(channels)
+            put("sum", n, xn)
+        xn.requires_grad_(case["mode"] == "train")
+        with torch.set_grad_enabled(case["mode"] == "train"):
+            groups = xn.reshape(1, G, -1)
+            centred = groups - groups.mean(2, keepdim=True)
+            xhat = (centred * torch.rsqrt(centred.square().mean(2, keepdim=True) + m.eps)).reshape(xn.shape)
+            y = _act64(case["act"], xhat * weight.view(channels) + bias.view(channels))
+        put("y", n, y.detach())
+        if case["mode"] == "train":
+            dx, dw, db = torch.autograd.grad(y, (xn, weight, bias), state["dy"][n:n + 1].double())
+            put("dx", n, dx)
+            dweight, dbias = dweight + dw, dbias + db
+    if case["mode"] == "train":
+        return {"y": rows["y"], "dx": rows["dx"], "dweight": dweight, "dbias": dbias}
+    return rows
