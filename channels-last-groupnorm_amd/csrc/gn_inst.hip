@@ -9,14 +9,16 @@
 #ifndef GN_INST_DTYPE
 #error "compile with -DGN_INST_DTYPE=<0|1|2|3>"
 #endif
-// One data type's kernels are spread over three translation units so that they compile in parallel:
-// part 0 the forward, part 1 the backward, part 2 the forward with fused additions (single-launch variants).
+// One data type's kernels are spread over four translation units so that they compile in parallel: the single-launch
+// kernels of the forward (part 0), the backward (part 1) and the forward with fused additions (part 2); the streaming
+// kernels of both directions and the choice between the families (part 3).
 #ifndef GN_INST_PART
-#error "compile with -DGN_INST_PART=<0|1|2>"
+#error "compile with -DGN_INST_PART=<0|1|2|3>"
 #endif
 #define GN_PART_FWD (GN_INST_PART == 0)
 #define GN_PART_BWD (GN_INST_PART == 1)
 #define GN_PART_ADD (GN_INST_PART == 2)
+#define GN_PART_STREAM (GN_INST_PART == 3)
 
 namespace gn {
 
@@ -41,6 +43,11 @@ typedef float wide_param_t;
 #define GN_CAT2(a, b) a##b
 #define GN_CAT(a, b) GN_CAT2(a, b)
 
+// The single-launch families (parts 0 to 2): true if the call was launched, false if it does not fit one.
+bool GN_CAT(try_resident_fwd_, GN_SUFFIX)(const FwdArgs &a);
+bool GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(const FwdArgs &a);
+bool GN_CAT(try_resident_bwd_, GN_SUFFIX)(const BwdArgs &a);
+
 namespace {
 
 typedef acc_t<elem_t> A;
@@ -50,7 +57,10 @@ dim3 tile_grid(const Plan &p, int extra_x) {
   return dim3((unsigned)(p.tiles + extra_x), (unsigned)p.nchunk, (unsigned)(p.N < 65535 ? p.N : 65535));
 }
 
-#if GN_PART_FWD
+// dy stored in a 16-bit type while the data are float (only the float instantiation has such kernels)
+[[maybe_unused]] constexpr bool kHasDy16 = GN_INST_DTYPE == 0;
+
+#if GN_PART_STREAM
 template <typename PT, int VEC, int ACT> void launch_apply(const FwdArgs &a, const A *part, const PartialGeo &q) {
   const Plan &p = a.plan;
   launch(kKindFwdApply, (apply_kernel<elem_t, PT, VEC, ACT>), tile_grid(p, 0), dim3(kBlock), a.stream, (const elem_t *)a.x,
@@ -65,7 +75,7 @@ template <typename PT, int VEC> void launch_apply_act(const FwdArgs &a, const A 
     default: launch_apply<PT, VEC, GN_ACT_GELU_TANH>(a, part, q); break;
   }
 }
-#endif  // GN_PART_FWD
+#else  // single-launch families
 
 // ---- resident (single-launch) path ----------------------------------------------------------------
 // Workgroups that can be resident at once for a kernel: occupancy reported by the runtime times the CUs.
@@ -163,7 +173,7 @@ int worthwhile_batches(const Plan &p, bool backward) {
 }
 size_t stat_size(int sdtype) { return sdtype == GN_F32 ? 4 : sdtype == GN_F64 ? 8 : 2; }
 
-#if !GN_PART_BWD
+#if GN_PART_FWD || GN_PART_ADD
 // One NV variant, the tensor cut into `batches` launches over consecutive samples (1: the whole tensor).
 template <typename PT, int ACT, int NV, int ADD> bool try_resident_fwd_nv(const FwdArgs &a, int batches) {
   if (NV < resident_min_rows()) return false;
@@ -235,27 +245,14 @@ template <typename PT> bool try_resident_fwd_pt(const FwdArgs &a) {
     default: return try_resident_fwd_act<PT, GN_ACT_GELU_TANH>(a);
   }
 }
-}  // namespace
-// the single-launch forward with fused additions lives in part 2
-bool GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(const FwdArgs &a);
-namespace {
 bool try_resident_fwd(const FwdArgs &a) {
-  if constexpr (sizeof(A) != 4) {
-    return false;  // no single-launch kernels for 64-bit data
-  } else {
-    if (!resident_enabled() || a.plan.vec == 1) return false;
-#if GN_PART_FWD
-    if (a.has_add()) return GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(a);
-#endif
-    return a.pdtype == GN_INST_DTYPE ? try_resident_fwd_pt<elem_t>(a) : try_resident_fwd_pt<wide_param_t>(a);
-  }
+  if (!resident_enabled() || a.plan.vec != kVec) return false;
+  return a.pdtype == GN_INST_DTYPE ? try_resident_fwd_pt<elem_t>(a) : try_resident_fwd_pt<wide_param_t>(a);
 }
 
-#endif  // !GN_PART_BWD
+#endif  // GN_PART_FWD || GN_PART_ADD
 
 #if GN_PART_BWD
-// dy stored in a 16-bit type while the data are float (only the float instantiation has such kernels)
-constexpr bool kHasDy16 = GN_INST_DTYPE == 0;
 template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, int batches);
 template <typename PT, int ACT, int NV, int XW = 0, int XL = 0> bool try_resident_bwd_nv(const BwdArgs &a, int batches) {
   if (a.dydtype != GN_INST_DTYPE) {
@@ -343,19 +340,25 @@ template <typename PT> bool try_resident_bwd_pt(const BwdArgs &a) {
   }
 }
 bool try_resident_bwd(const BwdArgs &a) {
-  if constexpr (sizeof(A) != 4) {
-    return false;
-  } else {
-    if (!resident_enabled() || a.plan.vec == 1) return false;
-    return a.pdtype == GN_INST_DTYPE ? try_resident_bwd_pt<elem_t>(a) : try_resident_bwd_pt<wide_param_t>(a);
-  }
+  if (!resident_enabled() || a.plan.vec != kVec) return false;
+  return a.pdtype == GN_INST_DTYPE ? try_resident_bwd_pt<elem_t>(a) : try_resident_bwd_pt<wide_param_t>(a);
 }
 
 #endif  // GN_PART_BWD
+#endif  // GN_PART_STREAM
 
-#if GN_PART_FWD
+#if GN_PART_STREAM
+// The single-launch kernel if the call fits one (64-bit data has none).
+bool try_resident(const BwdArgs &a) {
+  if constexpr (sizeof(A) != 4) return false;
+  else return GN_CAT(try_resident_bwd_, GN_SUFFIX)(a);
+}
+bool try_resident(const FwdArgs &a) {
+  if constexpr (sizeof(A) != 4) return false;
+  else return a.has_add() ? GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(a) : GN_CAT(try_resident_fwd_, GN_SUFFIX)(a);
+}
 template <int VEC> hipError_t fwd_impl(const FwdArgs &a) {
-  if (VEC != 1 && !a.streaming_only && try_resident_fwd(a)) return hipGetLastError();
+  if (VEC != 1 && !a.streaming_only && try_resident(a)) return hipGetLastError();
   note_streaming_call();
   if (a.has_add()) {
     // multi-launch form: materialise the sum (in sum_out, or in y when the caller does not want it), then
@@ -400,9 +403,14 @@ template <int VEC> hipError_t fwd_impl(const FwdArgs &a) {
   return hipGetLastError();
 }
 
-#endif  // GN_PART_FWD
-
-#if GN_PART_BWD
+// Channels a workgroup of the dgamma / dbeta sums takes (a power of two; kBlock / columns lanes share a channel's
+// `entries` tile sums): 32, a 256-byte line per entry, while that leaves a lane at most two rounds of four loads, fewer
+// for more entries down to 8, a 64-byte sector.
+int dwdb_columns(int64_t entries) {
+  int cols = 32;
+  while (cols > 8 && entries > 8 * (kBlock / cols)) cols >>= 1;
+  return cols;
+}
 template <typename PT, int VEC, int ACT, bool DY16> void launch_bwd_act(const BwdArgs &a) {
   const Plan &p = a.plan;
   const BwdWorkspace ws = bwd_workspace(p);
@@ -426,9 +434,13 @@ template <typename PT, int VEC, int ACT, bool DY16> void launch_bwd_act(const Bw
     srcG = compactG;
   }
   {
-    launch(kKindBwdDx, (bwd_dx_kernel<elem_t, PT, VEC, ACT, DY16>), tile_grid(p, 1), dim3(kBlock), a.stream,
+    const int dcols = dwdb_columns(p.N * q.tiles);
+    const int pieces = (p.lpr * p.vec + dcols - 1) / dcols;  // per chunk, handed out over the samples of the grid
+    const int samples = (int)(p.N < 65535 ? p.N : 65535);
+    const int extra = a.dw || a.db ? (pieces + samples - 1) / samples : 0;
+    launch(kKindBwdDx, (bwd_dx_kernel<elem_t, PT, VEC, ACT, DY16>), tile_grid(p, extra), dim3(kBlock), a.stream,
                        (const elem_t *)a.x, (const elem_t *)a.dy, (elem_t *)a.dx, a.mean, a.rstd, a.sdtype, a.w, a.b, srcC,
-                       srcG, q, a.dw, a.db, p, a.dydtype);
+                       srcG, q, a.dw, a.db, p, a.dydtype, dcols);
   }
 }
 template <typename PT, int VEC, bool DY16> void bwd_act_dy(const BwdArgs &a) {
@@ -447,25 +459,28 @@ template <typename PT, int VEC> void bwd_act(const BwdArgs &a) {
   bwd_act_dy<PT, VEC, false>(a);
 }
 template <int VEC> hipError_t bwd_impl(const BwdArgs &a) {
-  if (VEC != 1 && try_resident_bwd(a)) return hipGetLastError();
+  if (VEC != 1 && try_resident(a)) return hipGetLastError();
   note_streaming_call();
   if (a.pdtype == GN_INST_DTYPE) bwd_act<elem_t, VEC>(a);
   else bwd_act<wide_param_t, VEC>(a);
   return hipGetLastError();
 }
 
-#endif  // GN_PART_BWD
+#endif  // GN_PART_STREAM
 
 }  // namespace
 
-#if GN_PART_FWD
+#if GN_PART_STREAM
 hipError_t GN_CAT(launch_fwd_, GN_SUFFIX)(const FwdArgs &a) {
   return a.plan.vec == 1 ? fwd_impl<1>(a) : fwd_impl<kVec>(a);
 }
-#elif GN_PART_BWD
 hipError_t GN_CAT(launch_bwd_, GN_SUFFIX)(const BwdArgs &a) {
   return a.plan.vec == 1 ? bwd_impl<1>(a) : bwd_impl<kVec>(a);
 }
+#elif GN_PART_FWD
+bool GN_CAT(try_resident_fwd_, GN_SUFFIX)(const FwdArgs &a) { return try_resident_fwd(a); }
+#elif GN_PART_BWD
+bool GN_CAT(try_resident_bwd_, GN_SUFFIX)(const BwdArgs &a) { return try_resident_bwd(a); }
 #else
 bool GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(const FwdArgs &a) { return try_resident_fwd(a); }
 #endif

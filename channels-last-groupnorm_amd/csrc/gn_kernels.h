@@ -1055,14 +1055,17 @@ __global__ __launch_bounds__(kBlock) void bwd_compact_kernel(const A *__restrict
 // Backward pass 2: sum the tile partials A, B of the chunk's groups, s = 1 / (D R),
 //   coef1 = (mean B - A) s rstd^3, coef2 = -mean coef1 - B s rstd      (gn_kernel.cu:798-800)
 //   dx = a g + coef1 x + coef2, g recomputed as in pass 1                (dx_elem_kernel, gn_kernel.cu:803-905)
-// One extra column of workgroups (blockIdx.x == tiles, sample 0 only) produces, for the channels of its
-// chunk, dgamma_c = sum_n (S1 - mean S2) rstd and dbeta_c = sum_n S2 (compute_dweight_dbias, gn_kernel.cu:695-728).
+// The workgroups behind the last tile (blockIdx.x >= tiles, of every sample) share out the channels of their chunk,
+// dcols at a time (dwdb_columns), and produce dgamma_c = sum (S1 - mean S2) rstd and dbeta_c = sum S2 over the samples
+// and tiles (compute_dweight_dbias, gn_kernel.cu:695-728).  Those sums are a chain of dependent memory round trips, not
+// bandwidth: with one workgroup per chunk, which had one lane per channel where the chunk was a whole row of scalar
+// channels, (6, 140, 64, 64) bf16 took 196 us per launch; now 11.7, which dx alone fills.
 // ---------------------------------------------------------------------------------------------
 template <typename T, typename PT, int VEC, int ACT, bool DY16 = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void bwd_dx_kernel(
     const T *__restrict__ x, const T *__restrict__ dy, T *__restrict__ dx, const void *mean, const void *rstd, int sdtype,
     const void *w, const void *b, const acc_t<T> *__restrict__ partC, const acc_t<T> *__restrict__ partG, PartialGeo q,
-    void *dw, void *db, Plan p, int dydtype) {
+    void *dw, void *db, Plan p, int dydtype, int dcols) {
   using A = acc_t<T>;
   using LV = LaneVec<T, VEC>;
   constexpr int U = kUnrollBwd;
@@ -1071,42 +1074,52 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   __shared__ A sm_c2[kBlock * VEC];
   __shared__ A sm_mu[kBlock * VEC];
   __shared__ A sm_rs[kBlock * VEC];
-  if ((int)blockIdx.x == p.tiles) {
-    if (blockIdx.z != 0 || (!dw && !db)) return;
-    const int cstart = blockIdx.y * p.lpr * p.vec;
+  if ((int)blockIdx.x >= p.tiles) {
+    if (!dw && !db) return;
+    // N * tiles entries per channel, dcols channels per workgroup, kBlock / dcols lanes side by side on the entries of one
+    // channel (consecutive lanes read consecutive channels), four entries of a lane in flight
+    const int ts = threadIdx.x >> __builtin_ctz(dcols), cl = threadIdx.x & (dcols - 1);
+    const int nsl = kBlock >> __builtin_ctz(dcols);
+    const int64_t piece = (int64_t)((int)blockIdx.x - p.tiles) * gridDim.z + blockIdx.z;
     const int lanes_here = p.cv - (int)blockIdx.y * p.lpr < p.lpr ? p.cv - (int)blockIdx.y * p.lpr : p.lpr;
-    const int wch = lanes_here * p.vec;
-    // threads are laid out (tile slice, channel): consecutive threads read consecutive channels
-    const int cw = wch < kBlock ? wch : kBlock;  // channels handled per pass
-    const int nsl = kBlock / cw;                 // tile slices
-    const int cl = threadIdx.x % cw, ts = threadIdx.x / cw;
-    for (int cbase = 0; cbase < wch; cbase += cw) {
-      const int c = cstart + cbase + cl;
-      A t1 = (A)0, t2 = (A)0;
-      if (cbase + cl < wch && ts < nsl) {
-        const int g = div_by(c, p.by_D);
-        for (int64_t n = 0; n < p.N; ++n) {
-          A s1 = (A)0, s2 = (A)0;
-          for (int t = ts; t < q.tiles; t += nsl) {
-            const int64_t idx = ((n * q.tiles + t) * p.C + c) * 2;
-            s1 += partC[idx];
-            s2 += partC[idx + 1];
-          }
-          const A mu = load_scalar<A>(mean, n * p.G + g, sdtype);
-          const A rs = load_scalar<A>(rstd, n * p.G + g, sdtype);
-          t1 += (s1 - mu * s2) * rs;
-          t2 += s2;
-        }
+    const int cstart = blockIdx.y * p.lpr * p.vec, wch = lanes_here * p.vec;
+    if (piece * dcols >= wch) return;  // (uniform over the workgroup)
+    const bool valid = piece * dcols + cl < wch;
+    const int c = cstart + (int)piece * dcols + (valid ? cl : 0);
+    const int g = div_by(c, p.by_D);
+    const int64_t entries = p.N * q.tiles;
+    A t1 = (A)0, t2 = (A)0;
+    for (int64_t i0 = ts; i0 < entries; i0 += 4 * (int64_t)nsl) {
+      A s1[4], s2[4], mu[4], rs[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t i = i0 + u * nsl < entries ? i0 + u * nsl : i0;  // entry (n, t) = (i / tiles, i mod tiles)
+        const int64_t gidx = (int64_t)(unsigned)div_by((int)(unsigned)i, q.by_tiles) * p.G + g;
+        s1[u] = partC[(i * p.C + c) * 2];
+        s2[u] = partC[(i * p.C + c) * 2 + 1];
+        mu[u] = load_scalar_flat<A>(mean, gidx, sdtype, partC);
+        rs[u] = load_scalar_flat<A>(rstd, gidx, sdtype, partC);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = i0 + u * nsl < entries;
+        t1 += in ? (s1[u] - mu[u] * s2[u]) * rs[u] : (A)0;
+        t2 += in ? s2[u] : (A)0;
+      }
+    }
+    sm_c1[threadIdx.x] = t1;
+    sm_c2[threadIdx.x] = t2;
+    __syncthreads();
+    for (int h = nsl >> 1; h > 0; h >>= 1) {
+      if (ts < h) {
+        sm_c1[threadIdx.x] += sm_c1[threadIdx.x + h * dcols];
+        sm_c2[threadIdx.x] += sm_c2[threadIdx.x + h * dcols];
       }
       __syncthreads();
-      if (ts < nsl) { sm_c1[ts * cw + cl] = t1; sm_c2[ts * cw + cl] = t2; }
-      __syncthreads();
-      if (ts == 0 && cbase + cl < wch) {
-        A r1 = (A)0, r2 = (A)0;
-        for (int s = 0; s < nsl; ++s) { r1 += sm_c1[s * cw + cl]; r2 += sm_c2[s * cw + cl]; }
-        if (dw) store_param<PT, A>(dw, c, r1);
-        if (db) store_param<PT, A>(db, c, r2);
-      }
+    }
+    if (ts == 0 && valid) {
+      if (dw) store_param<PT, A>(dw, c, sm_c1[cl]);
+      if (db) store_param<PT, A>(db, c, sm_c2[cl]);
     }
     return;
   }

@@ -1,0 +1,42 @@
+"""GPU tests of the streaming kernels at the sizes where their work is cut differently: C ABI calls with the single-launch
+kernels switched off, against torch in float64 with the bars of tests/test_gpu_parity.py."""
+import pytest
+import torch
+
+from gnnhwc import _cabi
+from tests.gpu_harness import cabi_bwd, cabi_fwd
+from tests.test_gpu_parity import _check_against_torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def streaming_only():
+    before = _cabi.set_resident(False)
+    yield
+    _cabi.set_resident(before)
+
+
+# dgamma / dbeta are summed over N * tiles entries by 32, 16 or 8 channels per workgroup (up to 64, 128, more entries), the
+# pieces of a chunk handed out over the samples: channel counts below, at and beside those widths, chunks that are one piece
+# and many, more samples than pieces and fewer, entries below the lanes of a channel.
+@pytest.mark.parametrize("N,R,C,G", [(1, 7, 3, 1), (1, 40, 31, 1), (2, 65, 33, 3), (1, 300, 7, 7), (5, 1000, 35, 5),
+                                     (6, 4096, 140, 4), (1, 30000, 70, 2), (3, 9000, 257, 1), (40, 9, 66, 2), (4, 3000, 64, 8),
+                                     (1, 20000, 320, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_parameter_gradients_of_the_streaming_backward(N, R, C, G, dtype, device):
+    print("streaming", N, R, C, G, dtype, flush=True)
+    _check_against_torch(N, R, C, G, "silu", dtype, device)
+    assert _cabi.last_launch() == "multi-launch"
+
+
+@pytest.mark.parametrize("want_dw,want_db", [(True, False), (False, True), (False, False)])
+def test_parameter_gradients_not_asked_for(want_dw, want_db, device):
+    x, dy = torch.randn(3, 500, 35, device=device), torch.randn(3, 500, 35, device=device)
+    w, b = torch.rand(35, device=device) + 0.5, torch.randn(35, device=device)
+    _, mean, rstd = cabi_fwd(x, w, b, 5, 1e-5, 2)
+    dx, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, 5, 2)
+    dx2, dw2, db2 = cabi_bwd(dy, x, w, b, mean, rstd, 5, 2, want_dw=want_dw, want_db=want_db)
+    assert torch.equal(dx, dx2)
+    assert torch.equal(dw, dw2) if want_dw else dw2 is None
+    assert torch.equal(db, db2) if want_db else db2 is None
