@@ -108,6 +108,13 @@ def _load():
 
 
 lib = _load()
+try:
+    from . import _native  # csrc/gn_torch.cpp: the eager calls of GN_NHWC and group_norm_nhwc
+except ImportError as exc:
+    raise ImportError("gnnhwc: the _native extension is not built or does not load (make -C %s): %s" % (_CSRC, exc)) from exc
+_native.bind(*[ctypes.cast(getattr(lib, "gnnhwc_" + name), ctypes.c_void_p).value
+               for name in ("last_error", "fwd_workspace_bytes", "bwd_workspace_bytes", "nchw_workspace_bytes", "fwd_cast",
+                            "bwd_cast", "fwd_add", "fwd_nchw", "bwd_nchw")])
 
 
 def last_error():

@@ -13,7 +13,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _cabi
+from . import _cabi, _native
 
 _DTYPE_CODE = {
     torch.float32: _cabi.F32,
@@ -530,6 +530,11 @@ def group_norm_nhwc(x, weight, bias, num_groups, eps=1e-5, activation="identity"
     weight / bias may then be None.  Not combined with the fused additions."""
     if x.stride(1) != 1:
         raise RuntimeError("group_norm_nhwc expects channels-last input (stride 1 along dim 1)")
+    if weight is not None and not torch.compiler.is_compiling():
+        out = _native.group_norm(x, weight, bias, num_groups, eps, ACTIVATION_CODES[activation], out_dtype, residual, channel_bias,
+                                 return_sum)
+        if out is not NotImplemented:
+            return out
     nd = x.dim()
     x = x.permute(0, *range(2, nd), 1).contiguous()  # (N, *spatial, C), a no-op copy-wise for channels-last input
     shape = x.shape
@@ -638,6 +643,13 @@ class GN_NHWC(nn.GroupNorm):
         self.out_dtype = out_dtype
 
     def forward(self, x):
+        if not torch.compiler.is_compiling():
+            # an ordinary eager call: checks, kernels and autograd node in native code (csrc/gn_torch.cpp), which declines
+            # whatever it does not take -- the Python implementation below serves those calls, and their errors
+            y = _native.group_norm(x, self.weight, self.bias, self.num_groups, self.eps, self.act_code, self.out_dtype, None, None,
+                                   False)
+            if y is not NotImplemented:
+                return y
         if self.out_dtype is not None and self.out_dtype != x.dtype:
             if (x.is_cuda and x.dtype == torch.float32 and x.stride(1) == 1
                     and self.out_dtype in (torch.float16, torch.bfloat16)):
