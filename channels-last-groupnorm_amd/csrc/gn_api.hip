@@ -116,11 +116,7 @@ Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int streams)
   p.tiles = (int)((R + p.tile_rows - 1) / p.tile_rows);
   p.nblocks = N * p.tiles * p.nchunk;
   set_divisors(p);
-  {
-    const int chunk_channels = p.lpr * vec;
-    const int64_t g = (chunk_channels + p.D - 2) / p.D + 1;  // groups a window of chunk_channels can touch
-    p.gmax = (int)(g < G ? g : G);
-  }
+  set_gmax(p);
   static const int debug = env_int("GNNHWC_DEBUG_PLAN", 0);
   if (debug)
     fprintf(stderr, "[gnnhwc] plan(%s) N=%lld R=%lld C=%lld G=%d D=%d vec=%d cv=%d lpr=%d nchunk=%d rpi=%d tile_rows=%d tiles=%d nblocks=%lld\n",
@@ -164,9 +160,10 @@ size_t fwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, bool 
   size_t need = fwd_workspace(make_plan(N, R, C, G, 1, 1)).total;
   size_t resident = 0;
   if (C % vec == 0) {
-    const size_t v = fwd_workspace(make_plan(N, R, C, G, vec, 1)).total;
+    const Plan pv = make_plan(N, R, C, G, vec, 1);
+    const size_t v = fwd_workspace(pv).total;
     if (v > need) need = v;
-    resident = dtype == GN_F64 || streaming_only ? 0 : resident_fwd_bytes(G);
+    resident = dtype == GN_F64 || streaming_only ? 0 : resident_fwd_bytes(pv);
   }
   return max_size(kWorkspaceHeader + need * acc_size(dtype), resident);
 }

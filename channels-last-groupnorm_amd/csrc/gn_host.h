@@ -108,11 +108,43 @@ inline BwdWorkspace bwd_workspace(const Plan &p) {
 constexpr size_t kWorkspaceHeader = 256;
 // The resident kernels keep their partial results and one flag per workgroup in the same workspace.
 constexpr int kMaxResidentBlocks = 4 * kNumCU;
+constexpr size_t kRollingRecordBytes = (size_t)32 << 20;
 inline size_t resident_rec_bytes(int64_t G) { return (size_t)16 * G * kMaxResidentBlocks; }
 // Final records of the two-level exchange, one per (sample, group) of a launch: a launch has at most kMaxResidentBlocks samples.
 inline size_t resident_frec_bytes(int64_t G) { return (size_t)16 * G * kMaxResidentBlocks; }
-inline size_t resident_fwd_bytes(int64_t G) {
-  return kWorkspaceHeader + align_up(resident_rec_bytes(G), 256) + align_up(resident_frec_bytes(G), 256);
+// A forward too large to be resident as a whole still runs as ONE launch ("rolling") if every set of workgroups that
+// exchange records with each other is: workgroups are dispatched in linear order (row tiles, then chunks, then samples),
+// they publish before they wait, and a set's workgroups wait for nobody behind the set -- so the sets in front always
+// finish and make room, and while one set stores its results the next one's rows are already arriving.  (Should the
+// order ever be another, waits expire and are recovered from like any other.)
+// The set of a workgroup: the chunks from its own to the last one that a group of its chunk reaches into.
+inline int64_t exchange_chunks(const Plan &p) {
+  const int64_t cc = (int64_t)p.lpr * p.vec;
+  const int64_t ahead = cc % p.D == 0 ? 0 : p.D % cc == 0 ? p.D / cc - 1 : (p.D - 1 + cc - 1) / cc;
+  return 1 + ahead < p.nchunk ? 1 + ahead : p.nchunk;
+}
+constexpr int kRollingRows = 16;  // fewest rows per lane of a rolling launch
+struct FwdRecords {
+  size_t rec, frec;  // bytes of the tile records and of the final records
+  bool rolling;      // a rolling launch is allowed
+};
+inline FwdRecords resident_fwd_records(const Plan &p) {
+  FwdRecords r = {align_up(resident_rec_bytes(p.G), 256), align_up(resident_frec_bytes(p.G), 256), false};
+  const int64_t rows = (int64_t)kRollingRows * p.rpi;
+  const int64_t columns = p.N * p.nchunk, tiles = (p.R + rows - 1) / rows;
+  // full tiles only, and record indices within the kernels' 24-bit multiplies
+  if (p.N > 65535 || p.R < rows || columns * p.G >= (1 << 23) || tiles >= (1 << 23)) return r;
+  const size_t rec = (size_t)16 * p.G * columns * tiles;
+  if (rec > kRollingRecordBytes) return r;
+  r.rolling = true;
+  if (rec > r.rec) r.rec = align_up(rec, 256);
+  const size_t frec = (size_t)16 * p.G * p.N;
+  if (frec > r.frec) r.frec = align_up(frec, 256);
+  return r;
+}
+inline size_t resident_fwd_bytes(const Plan &p) {
+  const FwdRecords r = resident_fwd_records(p);
+  return kWorkspaceHeader + r.rec + r.frec;
 }
 // All-to-all or two-level exchange: records a workgroup would poll in the all-to-all form (tiles x chunks per group x
 // groups per chunk); beyond this bound the polling traffic of the whole launch rivals the tensor itself.

@@ -96,15 +96,17 @@ template <typename K> int resident_slots(K kernel) {
 
 // Row tiling of a resident launch with a register capacity of nv rows per lane: tiles of exactly nv rows per
 // lane (all loads useful; only the last tile of a sample may be short), every workgroup resident.
-// Returns false if it does not fit.
-bool resident_tiling(const Plan &base, int64_t samples, int nv, int slots, Plan &out) {
+// Returns false if it does not fit.  `rolling`: only the workgroups that exchange records have to be resident together.
+bool resident_tiling(const Plan &base, int64_t samples, int nv, int slots, Plan &out, bool rolling = false) {
   const int64_t columns = samples * base.nchunk;
-  if (slots <= 0 || columns > slots || samples > 65535) return false;
+  if (slots <= 0 || samples > 65535) return false;
+  const int64_t together = rolling ? exchange_chunks(base) : columns;
+  if (together > slots) return false;
   if (base.G > 8192 || base.C >= (1 << 23)) return false;  // the kernels index their records with 24-bit multiplies
   if ((base.lpr & (base.lpr - 1)) != 0) return false;  // ... and find a lane's row and column by shifts
   const int64_t rows = (int64_t)nv * base.rpi;
   const int64_t tiles = (base.R + rows - 1) / rows;
-  if (columns * tiles > slots) return false;
+  if (together * tiles > slots) return false;
   out = base;
   out.N = samples;
   out.tile_rows = (int)rows;
@@ -123,13 +125,13 @@ void arm_generation(ResidentWorkspace &r, const CapturedEpoch &c) {
   r.sync.generation = c.generation;
   if (c.generation) r.sync.epoch = c.next_sequence();
 }
-ResidentWorkspace resident_fwd_ws(void *ws, const Plan &p) {
+ResidentWorkspace resident_fwd_ws(void *ws, const Plan &p, const FwdRecords &records) {
   ResidentWorkspace r;
   char *base = (char *)ws + kWorkspaceHeader;
   r.sync.area = base;
-  r.sync.area_bytes = (unsigned)(resident_fwd_bytes(p.G) - kWorkspaceHeader);
+  r.sync.area_bytes = (unsigned)(records.rec + records.frec);
   r.sync.rec_first = 0;
-  r.sync.frec_first = (unsigned)(align_up(resident_rec_bytes(p.G), 256) / 16);
+  r.sync.frec_first = (unsigned)(records.rec / 16);
   r.sync.crec_first = 0;  // (no channel records in the forward)
   r.sync.two_level = two_level_exchange(p) ? 1 : 0;
   r.sync.status = resident_status();
@@ -159,13 +161,11 @@ ResidentWorkspace resident_bwd_ws(void *ws, const Plan &p) {
   return r;
 }
 
-// How many consecutive single-launch kernels over groups of samples still beat the streaming pair.  Each launch
-// pays a fixed latency of roughly 9 microseconds in the backward but moves 3 S bytes instead of the pair's 5 S
-// (about 5.4 bytes per nanosecond either way, and about 14 us fixed for the pair); measured on (N, 320, 128, 128)
-// bf16: two launches equal the pair at N = 4 and beat it by 14 % at N = 6, three launches by 6 % at N = 8.
-// In the forward the pair only moves 3 S against 2 S, and two launches measured 5 % slower than the pair: never split.
-int worthwhile_batches(const Plan &p, bool backward) {
-  if (!backward) return 1;
+// How many consecutive single-launch kernels over groups of samples still beat the streaming pair in the backward.  Each
+// launch pays a fixed latency of roughly 9 microseconds but moves 3 S bytes instead of the pair's 5 S (about 5.4 bytes
+// per nanosecond either way, and about 14 us fixed for the pair); measured on (N, 320, 128, 128) bf16: two launches
+// equal the pair at N = 4 and beat it by 14 % at N = 6, three launches by 6 % at N = 8.
+int worthwhile_batches(const Plan &p) {
   const double s_mb = (double)p.N * p.R * p.C * sizeof(elem_t) / 1e6;
   const double k = (14.0 + 0.405 * s_mb) / 9.0;
   const int kk = k < 1.0 ? 1 : (int)k;
@@ -174,59 +174,56 @@ int worthwhile_batches(const Plan &p, bool backward) {
 size_t stat_size(int sdtype) { return sdtype == GN_F32 ? 4 : sdtype == GN_F64 ? 8 : 2; }
 
 #if GN_PART_FWD || GN_PART_ADD
-// One NV variant, the tensor cut into `batches` launches over consecutive samples (1: the whole tensor).
-template <typename PT, int ACT, int NV, int ADD> bool try_resident_fwd_nv(const FwdArgs &a, int batches) {
+// One NV variant: the tensor resident as a whole, or (rolling) set by set.  A rolling launch reads x once where the streaming
+// pair reads it twice, and its sets overlap each other's loads, exchanges and stores: bf16 (8 / 12 / 16, 320, 128, 128)
+// 47.7 / 72.1 / 100.2 -> 35.8 / 48.6 / 78.7 us (cold tensors), float32 (2, 256, 256, 256) 67.6 -> 49.4 = 5.4 TB/s, float16
+// (1, 256, 512, 1024) 143.6 -> 133.9; with a residual and the sum written, (16, 320, 128, 128) 185 -> 146.  One sample of a
+// chunk has to fit the device: 524288 rows of 128 bytes (chunks of half the width, which would fit twice the rows, are
+// slower than the streaming pair: 371 against 343 us for (1, 256, 1024, 1024) float16).
+template <typename PT, int ACT, int NV, int ADD>
+bool try_resident_fwd_nv(const FwdArgs &a, const FwdRecords &records, bool rolling) {
   if (NV < resident_min_rows()) return false;
   auto kernel_all = fused_fwd_kernel<elem_t, PT, kVec, ACT, NV, ADD, false>;  // every workgroup polls every tile
   auto kernel_two = fused_fwd_kernel<elem_t, PT, kVec, ACT, NV, ADD, true>;   // two-level exchange (many tiles)
   static const int slots = std::min(resident_slots(kernel_all), resident_slots(kernel_two));
-  const int64_t per = (a.plan.N + batches - 1) / batches;
   Plan p;
-  if (!resident_tiling(a.plan, per, NV, slots, p)) return false;
+  if (!resident_tiling(a.plan, a.plan.N, NV, slots, p, rolling)) return false;
+  // A rolling launch works with 16 rows per lane while a set is at most an eighth of what is resident -- several sets are
+  // then in every phase at any time -- and with 32 beyond that, where a set's exchange weighs more: bf16 (8, 320, 128, 128)
+  // 35.8 us with 16 rows against 38.2 with 32, (3, 640, 200, 200) 77.9 against 72.4, float32 (2, 256, 256, 256) 57.2 / 49.5.
+  if (rolling && NV < 32 && exchange_chunks(p) * p.tiles > slots / 8) return false;
   if (!resident_status()) return false;
   CapturedEpoch cap;
   if (!captured_epoch(a.stream, cap)) return false;
   ResidentOrder order(a.stream, cap.generation != nullptr);
   mark_resident_launch();
-  const int64_t sample = a.plan.R * a.plan.C;
-  for (int64_t n0 = 0; n0 < a.plan.N; n0 += per) {
-    Plan pb = p;
-    if (a.plan.N - n0 < per) resident_tiling(a.plan, a.plan.N - n0, NV, slots, pb);  // the last, shorter group
-    ResidentWorkspace r = resident_fwd_ws(a.ws, pb);  // the launches follow each other on the stream: same records
-    arm_generation(r, cap);
-    AddArgs add = a.add;  // this group of samples' part of the addends
-    if (add.residual) add.residual = (const elem_t *)add.residual + n0 * sample;
-    if (add.sum_out) add.sum_out = (elem_t *)add.sum_out + n0 * sample;
-    if (add.channel_bias) add.channel_bias = (const char *)add.channel_bias + n0 * a.plan.C * stat_size(add.channel_bias_dtype);
-    FusedFwdParams k = {};
-    k.x = (const elem_t *)a.x + n0 * sample;
-    k.y = (char *)a.y + n0 * sample * stat_size(a.ydtype);
-    k.sync = r.sync;
-    k.w = a.w;
-    k.b = a.b;
-    k.mean_out = a.mean ? (char *)a.mean + n0 * a.plan.G * stat_size(a.sdtype) : nullptr;
-    k.rstd_out = a.rstd ? (char *)a.rstd + n0 * a.plan.G * stat_size(a.sdtype) : nullptr;
-    k.sdtype = a.sdtype;
-    k.ydtype = a.ydtype;
-    k.eps = (float)a.eps;
-    k.add = add;
-    k.p = pb;
-    launch(ADD != kAddNone ? kKindFusedFwdAdd : kKindFusedFwd, r.sync.two_level ? kernel_two : kernel_all, tile_grid(pb, 0),
-           dim3(kBlock), a.stream, k);
-    note_resident_launch(ADD != kAddNone ? kKindFusedFwdAdd : kKindFusedFwd, NV, 0, 0, r.sync.two_level, batches, pb.nblocks);
-  }
+  ResidentWorkspace r = resident_fwd_ws(a.ws, p, records);
+  arm_generation(r, cap);
+  FusedFwdParams k = {};
+  k.x = a.x;
+  k.y = a.y;
+  k.sync = r.sync;
+  k.w = a.w;
+  k.b = a.b;
+  k.mean_out = a.mean;
+  k.rstd_out = a.rstd;
+  k.sdtype = a.sdtype;
+  k.ydtype = a.ydtype;
+  k.eps = (float)a.eps;
+  k.add = a.add;
+  k.p = p;
+  launch(ADD != kAddNone ? kKindFusedFwdAdd : kKindFusedFwd, r.sync.two_level ? kernel_two : kernel_all, tile_grid(p, 0),
+         dim3(kBlock), a.stream, k);
+  note_resident_launch(ADD != kAddNone ? kKindFusedFwdAdd : kKindFusedFwd, NV, 0, 0, r.sync.two_level, 1, p.nblocks);
   return true;
 }
 template <typename PT, int ACT, int ADD> bool try_resident_fwd_add(const FwdArgs &a) {
-  // never cut into several launches: with a residual the alternative (an elementwise sum, then the plain forward)
-  // measured faster than two single-launch kernels
-  const int wb = worthwhile_batches(a.plan, false);
-  const int most = a.plan.N < wb ? (int)a.plan.N : wb;
-  for (int b = 1; b <= most; ++b)
-    if (try_resident_fwd_nv<PT, ACT, 4, ADD>(a, b) || try_resident_fwd_nv<PT, ACT, 8, ADD>(a, b) ||
-        try_resident_fwd_nv<PT, ACT, 16, ADD>(a, b) || try_resident_fwd_nv<PT, ACT, 32, ADD>(a, b))
-      return true;
-  return false;
+  const FwdRecords records = resident_fwd_records(a.plan);
+  if (try_resident_fwd_nv<PT, ACT, 4, ADD>(a, records, false) || try_resident_fwd_nv<PT, ACT, 8, ADD>(a, records, false) ||
+      try_resident_fwd_nv<PT, ACT, 16, ADD>(a, records, false) || try_resident_fwd_nv<PT, ACT, 32, ADD>(a, records, false))
+    return true;
+  return records.rolling &&
+         (try_resident_fwd_nv<PT, ACT, 16, ADD>(a, records, true) || try_resident_fwd_nv<PT, ACT, 32, ADD>(a, records, true));
 }
 template <typename PT, int ACT> bool try_resident_fwd_act(const FwdArgs &a) {
 #if GN_PART_ADD
@@ -314,7 +311,7 @@ template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resi
   return true;
 }
 template <typename PT, int ACT> bool try_resident_bwd_act(const BwdArgs &a) {
-  const int most = a.plan.N < worthwhile_batches(a.plan, true) ? (int)a.plan.N : worthwhile_batches(a.plan, true);
+  const int most = a.plan.N < worthwhile_batches(a.plan) ? (int)a.plan.N : worthwhile_batches(a.plan);
   for (int b = 1; b <= most; ++b) {
     if (try_resident_bwd_nv<PT, ACT, 4>(a, b) || try_resident_bwd_nv<PT, ACT, 8>(a, b) ||
         try_resident_bwd_nv<PT, ACT, 16>(a, b) || try_resident_bwd_nv<PT, ACT, 22>(a, b) ||

@@ -84,6 +84,11 @@ inline void set_divisors(Plan &p) {
   p.by_chunk = make_divisor((int64_t)p.lpr * p.vec, p.C + p.D);
 }
 
+inline void set_gmax(Plan &p) {
+  const int64_t g = ((int64_t)p.lpr * p.vec + p.D - 2) / p.D + 1;  // groups a window of lpr * vec channels can touch
+  p.gmax = (int)(g < p.G ? g : p.G);
+}
+
 // Pre-additions of the forward (fused-addition variant): the tensor that is normalised is s = x + residual + channel_bias[n][c],
 // rounded to T once (what an unfused elementwise addition in T would hand to the normalisation); s is written to
 // sum_out if that is given.  Any of the three pointers may be null.

@@ -1,0 +1,101 @@
+"""GPU tests of forward launches with more workgroups than fit the device at once: sets of workgroups that exchange records
+follow each other through it.  Against the streaming kernels on the same inputs (which tests/test_gpu_parity.py holds to
+the float64 oracle): statistics agree to float32 rounding, y to that or to one spacing of its 16-bit type."""
+import pytest
+import torch
+
+from gnnhwc import _cabi
+from tests.gpu_harness import cabi_fwd, cabi_fwd_add
+
+pytestmark = pytest.mark.gpu
+
+# N, R, C, G: sets of one chunk (groups inside a chunk; several in flight, and one that fills the device), of two and three
+# chunks (groups across chunk borders), of a whole sample (one group), a last tile of one row, of all but one, chunks of 32 bytes
+SHAPES = [(7, 16384, 320, 32), (1, 524288, 192, 12), (2, 65537, 256, 32), (3, 40000, 640, 8), (70, 513, 1280, 32), (2, 32767, 1088, 4),
+          (3, 65536, 256, 1), (9, 16384, 272, 17)]
+
+
+def _inputs(N, R, C, dtype, device):
+    gen = torch.Generator(device=device).manual_seed(N + R + C)
+    x = torch.empty((N, R, C), device=device, dtype=dtype).normal_(generator=gen).mul_(1.5).add_(
+        torch.randn((C,), device=device, generator=gen).to(dtype))
+    w = (torch.rand((C,), device=device, generator=gen) + 0.5).to(dtype)
+    b = (0.1 * torch.randn((C,), device=device, generator=gen)).to(dtype)
+    return x, w, b
+
+
+def _close(y, y0, mean, mean0, rstd, rstd0):
+    # float32 statistics of up to 1e8 elements, summed in two orders
+    assert (mean - mean0).abs().max() <= 2e-6
+    assert ((rstd - rstd0).abs() / rstd0).max() <= 2e-6
+    eps = torch.finfo(y.dtype).eps  # one spacing is eps |y| at most; a statistic's rounding moves y by about 1e-6
+    for n in range(y.shape[0]):
+        a, t = y[n].float(), y0[n].float()
+        assert ((a - t).abs() <= (eps if y.dtype != torch.float32 else 0) * t.abs() + 1e-5).all()
+
+
+def _streaming(fn):
+    before = _cabi.set_resident(False)
+    try:
+        return fn()
+    finally:
+        _cabi.set_resident(before)
+
+
+@pytest.mark.parametrize("N,R,C,G", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_against_the_streaming_kernels(N, R, C, G, dtype, device):
+    print("rolling", N, R, C, G, dtype, flush=True)
+    x, w, b = _inputs(N, R, C, dtype, device)
+    y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
+    assert _cabi.last_launch().startswith("fused_fwd"), _cabi.last_launch()
+    again = cabi_fwd(x, w, b, G, 1e-5, 2)
+    for s, t in zip((y, mean, rstd), again):
+        assert torch.equal(s, t)
+    del again
+    y0, mean0, rstd0 = _streaming(lambda: cabi_fwd(x, w, b, G, 1e-5, 2))
+    _close(y, y0, mean, mean0, rstd, rstd0)
+    inplace = cabi_fwd(x, w, b, G, 1e-5, 2, y=x)[0]
+    assert torch.equal(inplace, y)
+
+
+def test_with_fused_additions(device):
+    x, w, b = _inputs(9, 16384, 320, torch.bfloat16, device)
+    r, cb = torch.randn_like(x), torch.randn(9, 320, device=device).bfloat16()
+    y, s, mean, rstd = cabi_fwd_add(x, r, cb, w, b, 32, 1e-5, 2)
+    assert _cabi.last_launch().startswith("fused_fwd_add"), _cabi.last_launch()
+    y0, s0, mean0, rstd0 = _streaming(lambda: cabi_fwd_add(x, r, cb, w, b, 32, 1e-5, 2))
+    assert torch.equal(s, s0)
+    _close(y, y0, mean, mean0, rstd, rstd0)
+
+
+@pytest.mark.parametrize("spins", [-2, 0, 2])
+def test_expired_waits_are_recovered(spins, device):
+    x, w, b = _inputs(14, 16384, 160, torch.bfloat16, device)
+    y0, mean0, rstd0 = _streaming(lambda: cabi_fwd(x, w, b, 16, 1e-5, 2))
+    before = _cabi.lib.gnnhwc_debug_set_spin_limit(spins)
+    try:
+        y, mean, rstd = cabi_fwd(x, w, b, 16, 1e-5, 2)
+        torch.cuda.synchronize()
+    finally:
+        _cabi.lib.gnnhwc_debug_set_spin_limit(before)
+    _cabi.lib.gnnhwc_resident_status()
+    _close(y, y0, mean, mean0, rstd, rstd0)
+
+
+def test_replayed_graph(device):
+    x, w, b = _inputs(8, 16384, 320, torch.bfloat16, device)
+    ws = torch.empty((_cabi.lib.gnnhwc_fwd_workspace_bytes(8, 16384, 320, 32, 3),), dtype=torch.uint8, device=device)
+    y = torch.empty_like(x)
+    cabi_fwd(x, w, b, 32, 1e-5, 2, y=y, ws=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        cabi_fwd(x, w, b, 32, 1e-5, 2, y=y, ws=ws)
+    for i in range(3):
+        x.add_(i)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = cabi_fwd(x, w, b, 32, 1e-5, 2)[0]
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
