@@ -46,8 +46,8 @@ const char *dtype_name(int dtype) {
   return (dtype >= 0 && dtype < 4) ? names[dtype] : "?";
 }
 
-// Cut (N, R, C) into workgroup tiles.  `vec` is 16 / sizeof(T) for the 128-bit path or 1 for the
-// scalar path; `streams` is the number of activation-sized tensors a tile reads (1 forward, 2 backward).
+// Cut (N, R, C) into workgroup tiles.  `vec` is 16 / sizeof(T) for the 128-bit path, a smaller power of two for
+// narrower lane vectors, `esize` the bytes of an element; `streams` is the number of activation-sized tensors a tile reads (1 forward, 2 backward).
 //
 // Chunk width: a workgroup reads `lpr` lane vectors (lpr * 16 bytes) of each row.  Narrow chunks mean
 // tall tiles for the same number of workgroups, and the per-tile partial results (one entry per group
@@ -55,7 +55,7 @@ const char *dtype_name(int dtype) {
 // whole 128-byte lines, divides the row evenly and leaves no lane idle is preferred.
 // Rows per tile: chosen so that a large tensor yields about `target` workgroups and a small one still
 // yields as many workgroups as it has lane rows, down to one row per lane.
-Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int streams) {
+Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int esize, int streams) {
   static const int forced_lpr = env_int("GNNHWC_LPR", 0);
   static const int forced_fwd_steps = env_int("GNNHWC_FWD_STEPS", 0);
   static const int forced_bwd_steps = env_int("GNNHWC_BWD_STEPS", 0);
@@ -73,7 +73,7 @@ Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int streams)
   } else if (vec > 1) {
     static const int preferred[] = {8, 16, 32, 64, 128, 256, 4, 2};  // half and quarter lines only as a last resort
     for (int d : preferred)
-      if (p.cv % d == 0) { lpr = d; break; }
+      if (p.cv % d == 0 && (vec * esize == 16 || d * vec * esize >= 128)) { lpr = d; break; }
   }
   if (lpr == 0) {  // no even cut into whole cache lines: take the whole row, or equal-ish chunks of a long one
     const int nchunk = (p.cv + kBlock - 1) / kBlock;
@@ -153,29 +153,35 @@ int check_dtypes(int dtype, int pdtype, int sdtype) {
 }
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
+// Elements per lane vector: the widest power of two up to 16 bytes that divides C and every address (given as their
+// bitwise or: null pointers do not count).
+int lane_vector(int64_t C, int dtype, uintptr_t addresses) {
+  const int esize = elem_size(dtype);
+  int vec = 16 / esize;
+  while (vec > 1 && (C % vec != 0 || addresses % (uintptr_t)(vec * esize) != 0)) vec >>= 1;
+  return vec;
+}
+
 size_t acc_size(int dtype) { return dtype == GN_F64 ? 8 : 4; }
 size_t max_size(size_t a, size_t b) { return a > b ? a : b; }
+// (the width a call runs at depends on its addresses as well: the workspace serves every width C allows)
 size_t fwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, bool streaming_only = false) {
-  const int vec = 16 / elem_size(dtype);
-  size_t need = fwd_workspace(make_plan(N, R, C, G, 1, 1)).total;
-  size_t resident = 0;
-  if (C % vec == 0) {
-    const Plan pv = make_plan(N, R, C, G, vec, 1);
-    const size_t v = fwd_workspace(pv).total;
-    if (v > need) need = v;
-    resident = dtype == GN_F64 || streaming_only ? 0 : resident_fwd_bytes(pv);
+  const int esize = elem_size(dtype), full = 16 / esize;
+  size_t need = 0, resident = 0;
+  for (int vec = 1; vec <= full && C % vec == 0; vec *= 2) {
+    const Plan pv = make_plan(N, R, C, G, vec, esize, 1);
+    need = max_size(need, fwd_workspace(pv).total);
+    if (vec == full && dtype != GN_F64 && !streaming_only) resident = resident_fwd_bytes(pv);
   }
   return max_size(kWorkspaceHeader + need * acc_size(dtype), resident);
 }
 size_t bwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype) {
-  const int vec = 16 / elem_size(dtype);
-  size_t need = bwd_workspace(make_plan(N, R, C, G, 1, 2)).total;
-  size_t resident = 0;
-  if (C % vec == 0) {
-    const Plan pv = make_plan(N, R, C, G, vec, 2);
-    const size_t v = bwd_workspace(pv).total;
-    if (v > need) need = v;
-    resident = dtype == GN_F64 ? 0 : resident_bwd_bytes((int64_t)pv.lpr * vec, G);
+  const int esize = elem_size(dtype), full = 16 / esize;
+  size_t need = 0, resident = 0;
+  for (int vec = 1; vec <= full && C % vec == 0; vec *= 2) {
+    const Plan pv = make_plan(N, R, C, G, vec, esize, 2);
+    need = max_size(need, bwd_workspace(pv).total);
+    if (vec == full && dtype != GN_F64) resident = resident_bwd_bytes((int64_t)pv.lpr * vec, G);
   }
   return max_size(kWorkspaceHeader + need * acc_size(dtype), resident);
 }
@@ -546,15 +552,14 @@ static int forward(const void *x, const AddArgs &add, const void *weight, const 
   if (!workspace || !aligned16(workspace) || workspace_bytes < need)
     return fail(GNNHWC_ERR_WORKSPACE, "forward workspace must be 16-byte aligned and at least %zu bytes (got %p, %zu bytes)",
                 need, workspace, workspace_bytes);
-  const int vec = 16 / elem_size(dtype);
-  const bool vector_ok = C % vec == 0 && aligned16(x) && aligned16(y) && aligned16(add.residual) && aligned16(add.sum_out);
+  const int vec = lane_vector(C, dtype, (uintptr_t)x | (uintptr_t)y | (uintptr_t)add.residual | (uintptr_t)add.sum_out);
   FwdArgs a;
   a.streaming_only = streaming_only;
   a.add = add;
   a.x = x; a.w = weight; a.b = bias; a.y = y; a.mean = mean; a.rstd = rstd;
   a.eps = eps; a.act = act; a.pdtype = param_dtype; a.sdtype = stats_dtype; a.ydtype = y_dtype;
   a.ws = workspace; a.stream = (hipStream_t)stream;
-  a.plan = make_plan(N, R, C, G, vector_ok ? vec : 1, 1);
+  a.plan = make_plan(N, R, C, G, vec, elem_size(dtype), 1);
   if (a.plan.nchunk > 65535) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "too many channels for this build (C = %lld)", (long long)C);
   hipError_t e;
   switch (dtype) {
@@ -655,16 +660,15 @@ static int backward(const void *dy, const void *x, const void *weight, const voi
   if (!workspace || !aligned16(workspace) || workspace_bytes < need)
     return fail(GNNHWC_ERR_WORKSPACE, "backward workspace must be 16-byte aligned and at least %zu bytes (got %p, %zu bytes)",
                 need, workspace, workspace_bytes);
-  const int vec = 16 / elem_size(dtype);
   if (dy_dtype != dtype && dx == dy) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "dx of another type than dy cannot replace dy in place");
-  const bool vector_ok = C % vec == 0 && aligned16(x) && aligned16(dy) && aligned16(dx);
+  const int vec = lane_vector(C, dtype, (uintptr_t)x | (uintptr_t)dy | (uintptr_t)dx);
   BwdArgs a;
   a.dydtype = dy_dtype;
   a.dy = dy; a.x = x; a.w = weight; a.b = bias; a.mean = mean; a.rstd = rstd;
   a.dx = dx; a.dw = dweight; a.db = dbias;
   a.act = act; a.pdtype = param_dtype; a.sdtype = stats_dtype;
   a.ws = workspace; a.stream = (hipStream_t)stream;
-  a.plan = make_plan(N, R, C, G, vector_ok ? vec : 1, 2);
+  a.plan = make_plan(N, R, C, G, vec, elem_size(dtype), 2);
   if (a.plan.nchunk > 65535) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "too many channels for this build (C = %lld)", (long long)C);
   if (N * G > 0x7fffffffLL) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "N * G too large");
   hipError_t e;
@@ -880,7 +884,7 @@ int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int
   if (N == 0 || R == 0) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "empty problem: nothing is planned");
   const int vec = 16 / elem_size(dtype);
   if (vector && C % vec != 0) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "C = %lld is not a multiple of the vector width %d", (long long)C, vec);
-  const Plan p = make_plan(N, R, C, G, vector ? vec : 1, backward ? 2 : 1);
+  const Plan p = make_plan(N, R, C, G, vector ? vec : 1, elem_size(dtype), backward ? 2 : 1);
   const size_t elems = backward ? bwd_workspace(p).total : fwd_workspace(p).total;
   out[0] = p.vec; out[1] = p.cv; out[2] = p.lpr; out[3] = p.nchunk; out[4] = p.rpi; out[5] = p.tile_rows;
   out[6] = p.tiles; out[7] = p.gmax; out[8] = p.nblocks; out[9] = needs_compaction(p) ? 1 : 0;

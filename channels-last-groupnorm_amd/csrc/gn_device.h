@@ -26,6 +26,7 @@ template <typename T> struct vec_of { static constexpr int value = 16 / (int)siz
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -107,6 +108,59 @@ template <> struct LaneVec<bf16_t, 8> {
     return r;
   }
 };
+// narrower vectors, for channel counts and addresses that only halves or quarters of the full width divide
+template <> struct LaneVec<float, 2> {
+  typedef f32x2 raw_t;
+  static __device__ __forceinline__ raw_t load(const float *p) { return *(const raw_t *)p; }
+  static __device__ __forceinline__ void store(float *p, raw_t r) { *(raw_t *)p = r; }
+  static __device__ __forceinline__ void unpack(raw_t r, float (&v)[2]) { v[0] = r.x; v[1] = r.y; }
+  static __device__ __forceinline__ raw_t pack(const float (&v)[2]) { return raw_t{v[0], v[1]}; }
+};
+template <> struct LaneVec<f16_t, 4> {
+  typedef f16x4 raw_t;
+  static __device__ __forceinline__ raw_t load(const f16_t *p) { return *(const raw_t *)p; }
+  static __device__ __forceinline__ void store(f16_t *p, raw_t r) { *(raw_t *)p = r; }
+  static __device__ __forceinline__ void unpack(raw_t r, float (&v)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (float)r[j];
+  }
+  static __device__ __forceinline__ raw_t pack(const float (&v)[4]) {
+    raw_t r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = (_Float16)v[j];
+    return r;
+  }
+};
+template <> struct LaneVec<f16_t, 2> {
+  typedef f16x2 raw_t;
+  static __device__ __forceinline__ raw_t load(const f16_t *p) { return *(const raw_t *)p; }
+  static __device__ __forceinline__ void store(f16_t *p, raw_t r) { *(raw_t *)p = r; }
+  static __device__ __forceinline__ void unpack(raw_t r, float (&v)[2]) { v[0] = (float)r.x; v[1] = (float)r.y; }
+  static __device__ __forceinline__ raw_t pack(const float (&v)[2]) { return raw_t{(_Float16)v[0], (_Float16)v[1]}; }
+};
+template <> struct LaneVec<bf16_t, 4> {
+  typedef u32x2 raw_t;
+  static __device__ __forceinline__ raw_t load(const bf16_t *p) { return *(const raw_t *)p; }
+  static __device__ __forceinline__ void store(bf16_t *p, raw_t r) { *(raw_t *)p = r; }
+  static __device__ __forceinline__ void unpack(raw_t r, float (&v)[4]) {
+    const uint32_t lo = r.x, hi = r.y;
+    v[0] = bf16_bits_to_float(lo << 16);
+    v[1] = bf16_bits_to_float(lo & 0xffff0000u);
+    v[2] = bf16_bits_to_float(hi << 16);
+    v[3] = bf16_bits_to_float(hi & 0xffff0000u);
+  }
+  static __device__ __forceinline__ raw_t pack(const float (&v)[4]) { return raw_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])}; }
+};
+template <> struct LaneVec<bf16_t, 2> {
+  typedef uint32_t raw_t;
+  static __device__ __forceinline__ raw_t load(const bf16_t *p) { return *(const raw_t *)p; }
+  static __device__ __forceinline__ void store(bf16_t *p, raw_t r) { *(raw_t *)p = r; }
+  static __device__ __forceinline__ void unpack(raw_t r, float (&v)[2]) {
+    v[0] = bf16_bits_to_float(r << 16);
+    v[1] = bf16_bits_to_float(r & 0xffff0000u);
+  }
+  static __device__ __forceinline__ raw_t pack(const float (&v)[2]) { return pack_bf16x2(v[0], v[1]); }
+};
 // scalar fall-back: any C, any alignment
 template <> struct LaneVec<float, 1> {
   typedef float raw_t;
@@ -166,6 +220,9 @@ __device__ __forceinline__ void store_result(T *y, int64_t e, const A (&v)[VEC],
           r.y = __builtin_bit_cast(uint32_t, hi);
         }
         __builtin_nontemporal_store(r, (u32x2 *)yp);
+      } else if constexpr (VEC == 2) {
+        const f16x2 h = {(_Float16)v[0], (_Float16)v[1]};
+        __builtin_nontemporal_store(ydtype == GN_BF16 ? pack_bf16x2(v[0], v[1]) : __builtin_bit_cast(uint32_t, h), (uint32_t *)yp);
       } else {
         const _Float16 h = (_Float16)v[0];
         *yp = ydtype == GN_BF16 ? float_to_bf16_bits(v[0]) : __builtin_bit_cast(uint16_t, h);

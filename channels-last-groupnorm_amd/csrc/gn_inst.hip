@@ -355,7 +355,7 @@ bool try_resident(const FwdArgs &a) {
   else return a.has_add() ? GN_CAT(try_resident_fwd_added_, GN_SUFFIX)(a) : GN_CAT(try_resident_fwd_, GN_SUFFIX)(a);
 }
 template <int VEC> hipError_t fwd_impl(const FwdArgs &a) {
-  if (VEC != 1 && !a.streaming_only && try_resident(a)) return hipGetLastError();
+  if (VEC == kVec && !a.streaming_only && try_resident(a)) return hipGetLastError();
   note_streaming_call();
   if (a.has_add()) {
     // multi-launch form: materialise the sum (in sum_out, or in y when the caller does not want it), then
@@ -456,7 +456,7 @@ template <typename PT, int VEC> void bwd_act(const BwdArgs &a) {
   bwd_act_dy<PT, VEC, false>(a);
 }
 template <int VEC> hipError_t bwd_impl(const BwdArgs &a) {
-  if (VEC != 1 && try_resident(a)) return hipGetLastError();
+  if (VEC == kVec && try_resident(a)) return hipGetLastError();
   note_streaming_call();
   if (a.pdtype == GN_INST_DTYPE) bwd_act<elem_t, VEC>(a);
   else bwd_act<wide_param_t, VEC>(a);
@@ -468,11 +468,18 @@ template <int VEC> hipError_t bwd_impl(const BwdArgs &a) {
 }  // namespace
 
 #if GN_PART_STREAM
+// The widths below the full 16 bytes serve channel counts and addresses that only a half, a quarter or one element divides.
 hipError_t GN_CAT(launch_fwd_, GN_SUFFIX)(const FwdArgs &a) {
-  return a.plan.vec == 1 ? fwd_impl<1>(a) : fwd_impl<kVec>(a);
+  if (a.plan.vec == kVec) return fwd_impl<kVec>(a);
+  if constexpr (kVec >= 8) if (a.plan.vec == 4) return fwd_impl<4>(a);
+  if constexpr (kVec >= 4) if (a.plan.vec == 2) return fwd_impl<2>(a);
+  return fwd_impl<1>(a);
 }
 hipError_t GN_CAT(launch_bwd_, GN_SUFFIX)(const BwdArgs &a) {
-  return a.plan.vec == 1 ? bwd_impl<1>(a) : bwd_impl<kVec>(a);
+  if (a.plan.vec == kVec) return bwd_impl<kVec>(a);
+  if constexpr (kVec >= 8) if (a.plan.vec == 4) return bwd_impl<4>(a);
+  if constexpr (kVec >= 4) if (a.plan.vec == 2) return bwd_impl<2>(a);
+  return bwd_impl<1>(a);
 }
 #elif GN_PART_FWD
 bool GN_CAT(try_resident_fwd_, GN_SUFFIX)(const FwdArgs &a) { return try_resident_fwd(a); }

@@ -144,6 +144,8 @@ __device__ __forceinline__ typename LaneVec<T, VEC>::raw_t load_dy(const T *dy, 
       const u32x2 v = *(const u32x2 *)h;
       const uint32_t lo = v.x, hi = v.y;
       return f32x4{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi), 0.f, 0.f};
+    } else if constexpr (VEC == 2) {
+      return f32x2{__builtin_bit_cast(float, *(const uint32_t *)h), 0.f};
     } else {
       return __builtin_bit_cast(float, (uint32_t)*h);
     }
@@ -165,6 +167,11 @@ __device__ __forceinline__ void unpack_dy(typename LaneVec<T, VEC>::raw_t raw, a
     v[1] = widen_16(lo >> 16, dydtype);
     v[2] = widen_16(hi & 0xffffu, dydtype);
     v[3] = widen_16(hi >> 16, dydtype);
+  } else if constexpr (VEC == 2) {
+    const float r0 = raw.x;
+    const uint32_t both = __builtin_bit_cast(uint32_t, r0);
+    v[0] = widen_16(both & 0xffffu, dydtype);
+    v[1] = widen_16(both >> 16, dydtype);
   } else {
     v[0] = widen_16(__builtin_bit_cast(uint32_t, raw) & 0xffffu, dydtype);
   }

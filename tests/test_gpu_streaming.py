@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from gnnhwc import _cabi
-from tests.gpu_harness import cabi_bwd, cabi_fwd
+from tests.gpu_harness import cabi_bwd, cabi_fwd, err
 from tests.test_gpu_parity import _check_against_torch
 
 pytestmark = pytest.mark.gpu
@@ -28,6 +28,34 @@ def test_parameter_gradients_of_the_streaming_backward(N, R, C, G, dtype, device
     print("streaming", N, R, C, G, dtype, flush=True)
     _check_against_torch(N, R, C, G, "silu", dtype, device)
     assert _cabi.last_launch() == "multi-launch"
+
+
+# Lane vectors of 16, 8, 4 and 2 bytes (f32: 16, 8, 4): what the channel count divides, and what the addresses divide (the
+# tensors are cut out of larger buffers `shift` elements in).  Few and many channels, chunks of a whole row and of less.
+@pytest.mark.parametrize("C,G", [(4, 2), (12, 3), (36, 4), (140, 4), (1100, 4), (6, 1), (70, 2), (2050, 5), (35, 5), (64, 8)])
+@pytest.mark.parametrize("shift", [0, 1, 2, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_lane_vector_widths(C, G, shift, dtype, device):
+    N, R = 2, 67
+    gen = torch.Generator().manual_seed(C * 10 + shift)
+
+    def cut(t):
+        buf = torch.empty(t.numel() + 16, dtype=dtype, device=device)
+        out = buf[shift:shift + t.numel()].view(t.shape)
+        out.copy_(t)
+        return out
+
+    x, dy = (cut(torch.randn((N, R, C), generator=gen).to(dtype)) for _ in range(2))
+    w, b = torch.rand(C, generator=gen).to(dtype).to(device) + 0.5, torch.randn(C, generator=gen).to(dtype).to(device)
+    want = dtype if dtype == torch.float64 else torch.float32
+    eps = {torch.float32: 1e-5, torch.float64: 1e-12, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]  # two spacings
+    xt, wt, bt = x.to(want).permute(0, 2, 1).requires_grad_(), w.to(want).requires_grad_(), b.to(want).requires_grad_()
+    yt = torch.nn.functional.silu(torch.nn.functional.group_norm(xt.contiguous(), G, wt, bt, 1e-5))
+    gx, gw, gb = torch.autograd.grad(yt, (xt, wt, bt), dy.to(want).permute(0, 2, 1))
+    y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2, y=cut(torch.zeros(N, R, C)))
+    dx, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, G, 2, dx=cut(torch.zeros(N, R, C)))
+    for a, t in ((y, yt.permute(0, 2, 1)), (dx, gx.permute(0, 2, 1)), (dw, gw), (db, gb)):
+        assert err(a, t) <= eps, (err(a, t), eps)
 
 
 @pytest.mark.parametrize("want_dw,want_db", [(True, False), (False, True), (False, False)])
