@@ -887,7 +887,7 @@ int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int
   const Plan p = make_plan(N, R, C, G, vector ? vec : 1, elem_size(dtype), backward ? 2 : 1);
   const size_t elems = backward ? bwd_workspace(p).total : fwd_workspace(p).total;
   out[0] = p.vec; out[1] = p.cv; out[2] = p.lpr; out[3] = p.nchunk; out[4] = p.rpi; out[5] = p.tile_rows;
-  out[6] = p.tiles; out[7] = p.gmax; out[8] = p.nblocks; out[9] = needs_compaction(p) ? 1 : 0;
+  out[6] = p.tiles; out[7] = p.gmax; out[8] = p.nblocks; out[9] = needs_compaction(p, consumer_plan(p, p.vec * elem_size(dtype))) ? 1 : 0;
   out[10] = (int64_t)(kWorkspaceHeader + elems * acc_size(dtype));
   out[11] = p.D;
   return GNNHWC_OK;

@@ -216,11 +216,39 @@ int resident_min_rows();  // tuning knob (environment): smallest rows-per-lane v
 
 // Consumers merge the tile partials of their own groups in their prologue when every lane has at most kEarly
 // entries to fetch; otherwise a compaction kernel runs in between and leaves one entry per group.
-inline bool needs_compaction(const Plan &p) {
-  const int chunk_channels = p.lpr * p.vec;
-  const int64_t per_group = (int64_t)p.tiles * ((p.D - 1) / chunk_channels + 2);
-  const int lanes = merge_lanes_for(p.gmax);
+inline bool needs_compaction(const Plan &producer, const Plan &consumer) {
+  const int chunk_channels = producer.lpr * producer.vec;
+  const int64_t per_group = (int64_t)producer.tiles * ((producer.D - 1) / chunk_channels + 2);
+  const int lanes = merge_lanes_for(consumer.gmax);
   return lanes < 1 || per_group > (int64_t)kEarly * lanes;
+}
+// Tiling of a consumer (apply, dx) behind the producer's.  The producers want few, tall, narrow tiles, which leave few
+// partials; a consumer has none to leave, and many short tiles of whole rows, worked through in memory order, read and
+// write neighbouring lines at the same time: float16 (1, 256, 1024, 1024) apply 234 us with the producer's 764 tiles of
+// 128-byte rows, 206 with 8 rows per lane, 168 with 8 rows per lane of 512 bytes.  Rows widen to the widest power of two
+// of lane vectors that divides them, unless their groups would then need a compaction launch that the narrow chunk does not
+// (or no longer fit one merge round); rows whose width no larger power of two divides gained nothing (bf16 (16, 320, 128, 128):
+// 52.0 us in chunks of 128 bytes, 50.8 in rows of 640).
+constexpr int kConsumerBytes = 128;  // of a lane, i.e. 8 rows of 16 bytes (a tile of bf16 (8, 35, 200, 200), 2 bytes per lane and
+                                     // row, takes 22.8 us in tiles of 8 rows, 15.9 in the producer's of 63)
+inline Plan consumer_plan(const Plan &producer, int lane_bytes) {
+  Plan c = producer;
+  const int64_t most = kConsumerBytes / lane_bytes, own = producer.tile_rows / producer.rpi, steps = own < most ? own : most;
+  for (int lpr = kBlock; lpr > producer.lpr; lpr >>= 1) {
+    if (producer.cv % lpr != 0) continue;
+    c.lpr = lpr;
+    set_gmax(c);
+    if (c.gmax <= 64 && (!needs_compaction(producer, c) || needs_compaction(producer, producer))) break;
+    c = producer;
+  }
+  c.nchunk = (c.cv + c.lpr - 1) / c.lpr;
+  c.rpi = kBlock / c.lpr;
+  const int64_t lane_rows = (c.R + c.rpi - 1) / c.rpi;
+  c.tile_rows = (int)((steps < lane_rows ? steps : lane_rows) * c.rpi);
+  c.tiles = (int)((c.R + c.tile_rows - 1) / c.tile_rows);
+  c.nblocks = c.N * c.tiles * c.nchunk;
+  set_divisors(c);
+  return c;
 }
 // Whether a chunk's groups fit one merge round at all (more than kBlock groups per chunk do not; those plans
 // use the general looping merge).

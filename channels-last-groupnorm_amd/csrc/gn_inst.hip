@@ -61,18 +61,17 @@ dim3 tile_grid(const Plan &p, int extra_x) {
 [[maybe_unused]] constexpr bool kHasDy16 = GN_INST_DTYPE == 0;
 
 #if GN_PART_STREAM
-template <typename PT, int VEC, int ACT> void launch_apply(const FwdArgs &a, const A *part, const PartialGeo &q) {
-  const Plan &p = a.plan;
+template <typename PT, int VEC, int ACT> void launch_apply(const FwdArgs &a, const A *part, const PartialGeo &q, const Plan &p) {
   launch(kKindFwdApply, (apply_kernel<elem_t, PT, VEC, ACT>), tile_grid(p, 0), dim3(kBlock), a.stream, (const elem_t *)a.x,
          (elem_t *)a.y, part, q, a.w, a.b, a.mean, a.rstd, a.sdtype, a.ydtype, (A)a.eps, p);
 }
-template <typename PT, int VEC> void launch_apply_act(const FwdArgs &a, const A *part, const PartialGeo &q) {
+template <typename PT, int VEC> void launch_apply_act(const FwdArgs &a, const A *part, const PartialGeo &q, const Plan &p) {
   switch (a.act) {
-    case GN_ACT_IDENTITY: launch_apply<PT, VEC, GN_ACT_IDENTITY>(a, part, q); break;
-    case GN_ACT_RELU: launch_apply<PT, VEC, GN_ACT_RELU>(a, part, q); break;
-    case GN_ACT_SILU: launch_apply<PT, VEC, GN_ACT_SILU>(a, part, q); break;
-    case GN_ACT_GELU: launch_apply<PT, VEC, GN_ACT_GELU>(a, part, q); break;
-    default: launch_apply<PT, VEC, GN_ACT_GELU_TANH>(a, part, q); break;
+    case GN_ACT_IDENTITY: launch_apply<PT, VEC, GN_ACT_IDENTITY>(a, part, q, p); break;
+    case GN_ACT_RELU: launch_apply<PT, VEC, GN_ACT_RELU>(a, part, q, p); break;
+    case GN_ACT_SILU: launch_apply<PT, VEC, GN_ACT_SILU>(a, part, q, p); break;
+    case GN_ACT_GELU: launch_apply<PT, VEC, GN_ACT_GELU>(a, part, q, p); break;
+    default: launch_apply<PT, VEC, GN_ACT_GELU_TANH>(a, part, q, p); break;
   }
 }
 #else  // single-launch families
@@ -386,7 +385,8 @@ template <int VEC> hipError_t fwd_impl(const FwdArgs &a) {
     launch(kKindFwdStats, (stats_kernel<elem_t, VEC>), tile_grid(p, 0), dim3(kBlock), a.stream, (const elem_t *)a.x, part, p);
   }
   const A *src = part;
-  if (needs_compaction(p)) {
+  const Plan c = consumer_plan(p, VEC * (int)sizeof(elem_t));
+  if (needs_compaction(p, c)) {
     const int64_t items = p.N * p.G;
     const unsigned grid = (unsigned)((items + kBlock / 64 - 1) / (kBlock / 64));
     launch(kKindFwdStatsCompact, (stats_compact_kernel<A>), dim3(grid), dim3(kBlock), a.stream, (const A *)part, compact, q, p);
@@ -394,8 +394,8 @@ template <int VEC> hipError_t fwd_impl(const FwdArgs &a) {
     src = compact;
   }
   {
-    if (a.pdtype == GN_INST_DTYPE) launch_apply_act<elem_t, VEC>(a, src, q);
-    else launch_apply_act<wide_param_t, VEC>(a, src, q);
+    if (a.pdtype == GN_INST_DTYPE) launch_apply_act<elem_t, VEC>(a, src, q, c);
+    else launch_apply_act<wide_param_t, VEC>(a, src, q, c);
   }
   return hipGetLastError();
 }
@@ -419,7 +419,8 @@ template <typename PT, int VEC, int ACT, bool DY16> void launch_bwd_act(const Bw
                        (const elem_t *)a.x, (const elem_t *)a.dy, a.mean, a.rstd, a.sdtype, a.w, a.b, partC, partG, p, a.dydtype);
   }
   const A *srcC = partC, *srcG = partG;
-  if (needs_compaction(p)) {
+  const Plan c = consumer_plan(p, VEC * (int)sizeof(elem_t));
+  if (needs_compaction(p, c)) {
     const int nG = (int)((p.N * p.G + kBlock / 64 - 1) / (kBlock / 64));
     int cpb = 32;  // channels per workgroup: fewer when N C is small, so that about a CU's worth of workgroups exist
     while (cpb > 2 && p.N * p.C / cpb < kNumCU) cpb >>= 1;
@@ -432,12 +433,12 @@ template <typename PT, int VEC, int ACT, bool DY16> void launch_bwd_act(const Bw
   }
   {
     const int dcols = dwdb_columns(p.N * q.tiles);
-    const int pieces = (p.lpr * p.vec + dcols - 1) / dcols;  // per chunk, handed out over the samples of the grid
+    const int pieces = (c.lpr * c.vec + dcols - 1) / dcols;  // per chunk, handed out over the samples of the grid
     const int samples = (int)(p.N < 65535 ? p.N : 65535);
     const int extra = a.dw || a.db ? (pieces + samples - 1) / samples : 0;
-    launch(kKindBwdDx, (bwd_dx_kernel<elem_t, PT, VEC, ACT, DY16>), tile_grid(p, extra), dim3(kBlock), a.stream,
+    launch(kKindBwdDx, (bwd_dx_kernel<elem_t, PT, VEC, ACT, DY16>), tile_grid(c, extra), dim3(kBlock), a.stream,
                        (const elem_t *)a.x, (const elem_t *)a.dy, (elem_t *)a.dx, a.mean, a.rstd, a.sdtype, a.w, a.b, srcC,
-                       srcG, q, a.dw, a.db, p, a.dydtype, dcols);
+                       srcG, q, a.dw, a.db, c, a.dydtype, dcols);
   }
 }
 template <typename PT, int VEC, bool DY16> void bwd_act_dy(const BwdArgs &a) {

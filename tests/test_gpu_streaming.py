@@ -58,6 +58,17 @@ def test_lane_vector_widths(C, G, shift, dtype, device):
         assert err(a, t) <= eps, (err(a, t), eps)
 
 
+# The consumers' own tiling: rows that widen to 16, 32, 64 and 128 lane vectors or stay, with and without the compaction launch,
+# more groups than a widened row may have, a row count of one tile, one row more, and one row less than whole tiles.
+@pytest.mark.parametrize("N,R,C,G", [(1, 8192, 128, 32), (2, 8193, 256, 8), (1, 65535, 512, 64), (1, 4097, 1024, 128),
+                                     (1, 4096, 1024, 512), (3, 2047, 320, 32), (1, 70001, 64, 1), (2, 513, 2048, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_consumer_tiling(N, R, C, G, dtype, device):
+    print("consumer tiling", N, R, C, G, dtype, flush=True)
+    _check_against_torch(N, R, C, G, "gelu_tanh", dtype, device)
+    assert _cabi.last_launch() == "multi-launch"
+
+
 @pytest.mark.parametrize("want_dw,want_db", [(True, False), (False, True), (False, False)])
 def test_parameter_gradients_not_asked_for(want_dw, want_db, device):
     x, dy = torch.randn(3, 500, 35, device=device), torch.randn(3, 500, 35, device=device)
