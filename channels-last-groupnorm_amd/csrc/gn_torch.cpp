@@ -95,6 +95,27 @@ Tensor workspace(size_t bytes, const Tensor &x, const char *what) {
 void *ptr(const optional<Tensor> &t) { return t.has_value() && t->defined() ? t->data_ptr() : nullptr; }
 void check(int rc, const char *what) { TORCH_CHECK(rc == 0, what, " failed (code ", rc, "): ", abi.last_error()); }
 
+// A tensor the kernels may read: memory of x's device.
+void require_device(const Tensor &t, const Tensor &x, const char *name) {
+  TORCH_CHECK(t.defined() && t.is_cuda() && t.layout() == at::kStrided, name, " must be a CUDA tensor");
+  TORCH_CHECK(t.device() == x.device(), name, " is on ", t.device(), ", the other tensors on ", x.device());
+}
+// t in the layout of the kernels -- `first`: contiguous, else channels-last -- and without a lazy negation; t itself where
+// it already is.
+Tensor in_layout(const Tensor &t, bool first) {
+  const Tensor r = t.is_neg() ? t.resolve_neg() : t;
+  if (first) return r.contiguous();
+  const int64_t nd = r.dim();
+  if (nd < 3 || channels_last(r)) return r;
+  c10::SmallVector<int64_t, 6> last(nd), back(nd);
+  last[0] = back[0] = 0;
+  for (int64_t d = 2; d < nd; ++d) last[d - 1] = d;
+  last[nd - 1] = 1;
+  back[1] = nd - 1;
+  for (int64_t d = 2; d < nd; ++d) back[d] = d - 1;
+  return r.permute(last).contiguous().permute(back);
+}
+
 struct Added {  // pre-additions of the forward (group_norm_nhwc)
   optional<Tensor> residual, channel_bias;
   Tensor sum;  // where x + residual + channel_bias goes (undefined: nowhere)
@@ -143,30 +164,33 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const auto call = ctx->saved_data["call"].toIntVector();
-    const Tensor &x = saved[0], &weight = saved[1], &bias = saved[2], &stats = saved[3];
     const int64_t G = call[0], act = call[1];
     const bool first = call[2] != 0;
     const char *what = first ? "gnop::bwd_nchw" : "gnop::bwd";
-    const c10::DeviceGuard guard(x.device());
     const at::AutoGradMode no_graph(false);
-    Tensor dy = grads[0];
-    TORCH_CHECK(dy.is_cuda(), "dy must be a CUDA tensor");
-    TORCH_CHECK(dy.sizes() == x.sizes(), what, " expects dy and X of the same shape, got ", dy.sizes(), " and ", x.sizes());
+    // The saved tensors are what the caller's saved-tensor hooks return, which need not be what the forward saved: offloading
+    // hooks give back contiguous copies, others may leave a tensor on the host.
+    require_device(grads[0], grads[0], "dy");
+    require_device(saved[0], grads[0], "X");
+    require_device(saved[3], grads[0], "means");
+    const c10::DeviceGuard guard(saved[0].device());
+    const Tensor dy = in_layout(grads[0], first), x = in_layout(saved[0], first), stats = saved[3].contiguous();
+    TORCH_CHECK(x.dim() >= 3 && dy.sizes() == x.sizes(), what, " expects dy and X of the same shape, got ", dy.sizes(), " and ",
+                x.sizes());
     const bool dy16 = !first && x.scalar_type() == at::kFloat && is_half(dy.scalar_type());
     TORCH_CHECK(dy.scalar_type() == x.scalar_type() || dy16,
                 "dy and X must have the same dtype, or dy float16 / bfloat16 with float32 X (", dy.scalar_type(), " vs ",
                 x.scalar_type(), ")");
-    if (first) {
-      dy = dy.contiguous();
-    } else if (dy.is_conj() || dy.is_neg() || !channels_last(dy)) {  // dy in x's own layout, whatever its rank
-      const int64_t nd = dy.dim();
-      c10::SmallVector<int64_t, 6> last(nd), back(nd);
-      last[0] = back[0] = 0;
-      for (int64_t d = 2; d < nd; ++d) last[d - 1] = d;
-      last[nd - 1] = 1;
-      back[1] = nd - 1;
-      for (int64_t d = 2; d < nd; ++d) back[d] = d - 1;
-      dy = dy.permute(last).contiguous().permute(back);
+    TORCH_CHECK(stats.numel() == 2 * x.size(0) * G, "means and rstds must have N*G = ", x.size(0) * G, " elements");
+    Tensor weight, bias;
+    if (saved[1].defined()) {
+      require_device(saved[1], x, "weight");
+      require_device(saved[2], x, "bias");
+      weight = saved[1].contiguous();
+      bias = saved[2].contiguous();
+      TORCH_CHECK(bias.scalar_type() == weight.scalar_type(), "weight and bias must have the same dtype (", weight.scalar_type(),
+                  " vs ", bias.scalar_type(), ")");
+      TORCH_CHECK(weight.numel() == x.size(1) && bias.numel() == x.size(1), "weight and bias must have ", x.size(1), " elements");
     }
     const at::AutoDispatchBelowADInplaceOrView below;
     const Shape s = shape_of(x);

@@ -233,3 +233,65 @@ def test_host_tensors_are_declined():
     assert _native.group_norm(None, w, b, 2, 1e-5, 0, None, None, None, False) is NotImplemented
     with pytest.raises(RuntimeError):
         _native.group_norm(x)
+
+
+# What unpacking hooks may hand to the backward in place of the saved tensors, each with equal values: other strides (what
+# offloading hooks that pack into empty(size) return), a view into a larger buffer, a broadcastable stride pattern undone.
+def _contiguous(t):
+    return t.contiguous(memory_format=torch.contiguous_format).clone(memory_format=torch.contiguous_format)
+
+
+def _cut(t):
+    buf = t.new_empty((2, *t.shape))
+    buf[1] = t
+    return buf[1]
+
+
+def _reversed_dims(t):
+    return t.permute(*reversed(range(t.dim()))).contiguous().permute(*reversed(range(t.dim())))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unpack", [_contiguous, _cut, _reversed_dims])
+@pytest.mark.parametrize("functional", [False, True])
+@pytest.mark.parametrize("shape,first", [((2, 32, 6, 5), False), ((2, 32, 6, 5), True), ((3, 8, 3, 4, 5), False), ((2, 12, 7), False)])
+def test_saved_tensors_may_come_back_in_any_layout(unpack, functional, shape, first, device):
+    if functional and first:
+        pytest.skip("group_norm_nhwc takes channels-last input only")
+    m = GN_NHWC(4, shape[1], activation="silu").to(device)
+    x = torch.randn(shape, device=device)
+    x = (x if first else _channels_last(x)).requires_grad_()
+    dy = torch.randn(shape, device=device)
+    call = (lambda: group_norm_nhwc(x, m.weight, m.bias, 4, m.eps, "silu")) if functional else (lambda: m(x))
+    want = torch.autograd.grad(call(), (x, m.weight, m.bias), dy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = call()
+    for s, t in zip(torch.autograd.grad(y, (x, m.weight, m.bias), dy), want):
+        assert torch.equal(s, t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pin", [False, True])
+def test_save_on_cpu(pin, device):
+    m = GN_NHWC(4, 32, activation="gelu").to(device)
+    x, dy = (_channels_last(torch.randn(2, 32, 6, 5, device=device)) for _ in range(2))
+    x.requires_grad_()
+    want = torch.autograd.grad(m(x), (x, m.weight, m.bias), dy)
+    with torch.autograd.graph.save_on_cpu(pin_memory=pin):
+        y = m(x)
+    for s, t in zip(torch.autograd.grad(y, (x, m.weight, m.bias), dy), want):
+        assert torch.equal(s, t)
+
+
+@pytest.mark.gpu
+def test_saved_tensors_of_another_device_type_or_size_are_refused(device):
+    m = GN_NHWC(4, 32).to(device)
+    x = _channels_last(torch.randn(2, 32, 6, 5, device=device)).requires_grad_()
+    for pick, change, message in [(4, lambda t: t.cpu(), "must be a CUDA tensor"), (1, lambda t: t.cpu(), "must be a CUDA tensor"),
+                                  (3, lambda t: t.cpu(), "must be a CUDA tensor"), (4, lambda t: t.half(), "same dtype"),
+                                  (1, lambda t: t[:16], "32 elements"), (4, lambda t: t[:1], "same shape"), (3, lambda t: t[:1], "N\\*G")]:
+        # pick: the parameters (1 dimension), the statistics (3) or x (4)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: change(t) if t.dim() == pick else t):
+            y = m(x)
+        with pytest.raises(RuntimeError, match=message):
+            y.sum().backward()
