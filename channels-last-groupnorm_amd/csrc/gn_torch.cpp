@@ -10,6 +10,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -100,20 +101,26 @@ void require_device(const Tensor &t, const Tensor &x, const char *name) {
   TORCH_CHECK(t.defined() && t.is_cuda() && t.layout() == at::kStrided, name, " must be a CUDA tensor");
   TORCH_CHECK(t.device() == x.device(), name, " is on ", t.device(), ", the other tensors on ", x.device());
 }
-// t in the layout of the kernels -- `first`: contiguous, else channels-last -- and without a lazy negation; t itself where
-// it already is.
+// Dimension orders that take the channels of an nd-dimensional tensor behind the spatial dimensions, and back.
+struct Orders {
+  c10::SmallVector<int64_t, 6> last, back;
+};
+Orders orders_of(int64_t nd) {
+  Orders o = {c10::SmallVector<int64_t, 6>(nd), c10::SmallVector<int64_t, 6>(nd)};
+  o.last[0] = o.back[0] = 0;
+  for (int64_t d = 2; d < nd; ++d) o.last[d - 1] = d;
+  o.last[nd - 1] = 1;
+  o.back[1] = nd - 1;
+  for (int64_t d = 2; d < nd; ++d) o.back[d] = d - 1;
+  return o;
+}
+Tensor resolved(const Tensor &t) { return t.is_neg() ? t.resolve_neg() : t; }
+// t in the layout of the kernels -- `first`: contiguous, else channels-last --; t itself where it already is.
 Tensor in_layout(const Tensor &t, bool first) {
-  const Tensor r = t.is_neg() ? t.resolve_neg() : t;
-  if (first) return r.contiguous();
-  const int64_t nd = r.dim();
-  if (nd < 3 || channels_last(r)) return r;
-  c10::SmallVector<int64_t, 6> last(nd), back(nd);
-  last[0] = back[0] = 0;
-  for (int64_t d = 2; d < nd; ++d) last[d - 1] = d;
-  last[nd - 1] = 1;
-  back[1] = nd - 1;
-  for (int64_t d = 2; d < nd; ++d) back[d] = d - 1;
-  return r.permute(last).contiguous().permute(back);
+  if (first) return t.contiguous();
+  if (t.dim() < 3 || channels_last(t)) return t;
+  const Orders o = orders_of(t.dim());
+  return t.permute(o.last).contiguous().permute(o.back);
 }
 
 struct Added {  // pre-additions of the forward (group_norm_nhwc)
@@ -150,14 +157,64 @@ Tensor run_forward(const Tensor &x, const optional<Tensor> &weight, const option
   return y;
 }
 
+// Dispatch keys of a plain device tensor; any other key (a subclass, a transform's wrapper, a lazy conjugate ...) declines.
+const c10::DispatchKeySet &plain_keys() {
+  static const c10::DispatchKeySet keys = c10::DispatchKeySet(c10::DispatchKey::CUDA) |
+                                          c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) |
+                                          c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) |
+                                          c10::DispatchKeySet(c10::DispatchKey::AutocastCUDA);
+  return keys;
+}
+// Keys that are switched on for every thread, or by autocast (which has no rule for this operation).
+const c10::DispatchKeySet &plain_tls() {
+  static const c10::DispatchKeySet keys =
+      c10::default_included_set | c10::autocast_dispatch_keyset | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
+  return keys;
+}
+// (by the bits: the sets' difference keeps the bits of the backends)
+bool only(c10::DispatchKeySet keys, c10::DispatchKeySet allowed) { return (keys.raw_repr() & ~allowed.raw_repr()) == 0; }
+bool ordinary_dispatch() {
+  return !c10::impl::TorchDispatchModeTLS::any_modes_set() && only(c10::impl::tls_local_dispatch_key_set().included_, plain_tls());
+}
+bool ordinary_thread() { return at::impl::PythonTorchFunctionTLS::stack_len() == 0 && ordinary_dispatch(); }
+bool plain(const Tensor &t, const c10::Device &device) {
+  return t.defined() && t.is_cuda() && t.device() == device && t.layout() == at::kStrided && only(t.key_set(), plain_keys()) &&
+         !t._fw_grad(0).defined();
+}
+
+// The backward through the dispatcher, as the operators' registered formula calls it: for gradients and saved tensors that are
+// no plain device tensors (batched gradients, subclasses), and where something on this thread is to see the operator.
+torch::autograd::variable_list backward_operator(const Tensor &dy, const Tensor &x, const Tensor &weight, const Tensor &bias,
+                                                 const Tensor &stats, int64_t G, int64_t act, bool first) {
+  const char *what = first ? "gnop::bwd_nchw" : "gnop::bwd";
+  TORCH_CHECK(weight.defined(), what, " of a normalisation without parameters takes plain device tensors only");
+  TORCH_CHECK(x.dim() >= 3 && dy.sizes() == x.sizes(), what, " expects dy and X of the same shape, got ", dy.sizes(), " and ", x.sizes());
+  using Signature = std::tuple<Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
+                                                       const Tensor &, const Tensor &, int64_t, int64_t);
+  const auto op = c10::Dispatcher::singleton().findSchemaOrThrow(what, "").typed<Signature>();
+  const Orders o = orders_of(x.dim());
+  const Shape s = shape_of(x);
+  const auto flat = [&](const Tensor &t) {  // (N, C, R), channels-last unless `first`
+    if (first) return t.contiguous().view({s.N, s.C, s.R});
+    return t.permute(o.last).contiguous().view({s.N, s.R, s.C}).permute({0, 2, 1});
+  };
+  const Tensor mean = stats.select(0, 0), rstd = stats.select(0, 1);
+  const auto [dx, dw, db] = op.call(flat(dy), flat(x), weight, bias, mean, rstd, G, act);
+  if (first) return {dx.reshape(x.sizes()), dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  c10::SmallVector<int64_t, 6> sizes(x.dim());
+  for (int64_t d = 0; d < x.dim(); ++d) sizes[d] = x.size(o.last[d]);
+  return {dx.permute({0, 2, 1}).reshape(sizes).permute(o.back), dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+}
+
 // The derivative of the normalisation (no pre-additions), either layout.
 struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
   static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const optional<Tensor> &weight,
-                        const optional<Tensor> &bias, int64_t G, double eps, int64_t act, bool first, int64_t out) {
+                        const optional<Tensor> &bias, int64_t G, double eps, int64_t act, bool first, int64_t out,
+                        bool functional) {
     Tensor stats;
     Tensor y = run_forward(x, weight, bias, G, eps, (int)act, first, (at::ScalarType)out, Added{}, stats);
     ctx->save_for_backward({x, weight.value_or(Tensor()), bias.value_or(Tensor()), stats});
-    ctx->saved_data["call"] = std::vector<int64_t>{G, act, first ? 1 : 0};
+    ctx->saved_data["call"] = std::vector<int64_t>{G, act, first ? 1 : 0, functional ? 1 : 0};
     // a view, as the Python function returns: an in-place change of y is refused the same way
     return y.view(y.sizes());
   }
@@ -165,16 +222,30 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
     const auto saved = ctx->get_saved_variables();
     const auto call = ctx->saved_data["call"].toIntVector();
     const int64_t G = call[0], act = call[1];
-    const bool first = call[2] != 0;
+    const bool first = call[2] != 0, functional = call[3] != 0;
     const char *what = first ? "gnop::bwd_nchw" : "gnop::bwd";
-    const at::AutoGradMode no_graph(false);
     // The saved tensors are what the caller's saved-tensor hooks return, which need not be what the forward saved: offloading
     // hooks give back contiguous copies, others may leave a tensor on the host.
     require_device(grads[0], grads[0], "dy");
     require_device(saved[0], grads[0], "X");
     require_device(saved[3], grads[0], "means");
-    const c10::DeviceGuard guard(saved[0].device());
-    const Tensor dy = in_layout(grads[0], first), x = in_layout(saved[0], first), stats = saved[3].contiguous();
+    if (saved[1].defined()) {
+      require_device(saved[1], grads[0], "weight");
+      require_device(saved[2], grads[0], "bias");
+    }
+    const c10::Device device = grads[0].device();
+    const c10::DeviceGuard guard(device);
+    // (the module's own autograd function never recorded a graph of its backward; the functional form went through the operator)
+    const at::AutoGradMode graph(functional && at::GradMode::is_enabled());
+    Tensor dy = resolved(grads[0]), x = resolved(saved[0]);
+    const bool all_plain = plain(dy, device) && plain(x, device) && plain(saved[3], device) &&
+                           (!saved[1].defined() || (plain(saved[1], device) && plain(saved[2], device)));
+    if (!all_plain || (functional && saved[1].defined() && (at::GradMode::is_enabled() || !ordinary_dispatch())))
+      return backward_operator(dy, x, saved[1], saved[2], saved[3], G, act, first);
+    const at::AutoGradMode no_graph(false);
+    dy = in_layout(dy, first);
+    x = in_layout(x, first);
+    const Tensor stats = saved[3].contiguous();
     TORCH_CHECK(x.dim() >= 3 && dy.sizes() == x.sizes(), what, " expects dy and X of the same shape, got ", dy.sizes(), " and ",
                 x.sizes());
     const bool dy16 = !first && x.scalar_type() == at::kFloat && is_half(dy.scalar_type());
@@ -184,8 +255,6 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
     TORCH_CHECK(stats.numel() == 2 * x.size(0) * G, "means and rstds must have N*G = ", x.size(0) * G, " elements");
     Tensor weight, bias;
     if (saved[1].defined()) {
-      require_device(saved[1], x, "weight");
-      require_device(saved[2], x, "bias");
       weight = saved[1].contiguous();
       bias = saved[2].contiguous();
       TORCH_CHECK(bias.scalar_type() == weight.scalar_type(), "weight and bias must have the same dtype (", weight.scalar_type(),
@@ -213,35 +282,11 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
                          : abi.bwd_cast(dy.data_ptr(), x.data_ptr(), wp, bp, mean, rstd, dx.data_ptr(), dwp, dbp, s.N, s.R, s.C, G,
                                         (int)act, dt, pdt, sdt, code_of(dy.scalar_type()), ws.data_ptr(), bytes, stream_of(x));
     check(rc, what);
-    return {dx, dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dx, dw, db, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
 // ---- what group_norm() takes -----------------------------------------------------------------------------------------
-// Dispatch keys of a plain device tensor; any other key (a subclass, a transform's wrapper, a lazy conjugate ...) declines.
-const c10::DispatchKeySet &plain_keys() {
-  static const c10::DispatchKeySet keys = c10::DispatchKeySet(c10::DispatchKey::CUDA) |
-                                          c10::DispatchKeySet(c10::DispatchKey::AutogradCUDA) |
-                                          c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView) |
-                                          c10::DispatchKeySet(c10::DispatchKey::AutocastCUDA);
-  return keys;
-}
-// Keys that are switched on for every thread, or by autocast (which has no rule for this operation).
-const c10::DispatchKeySet &plain_tls() {
-  static const c10::DispatchKeySet keys =
-      c10::default_included_set | c10::autocast_dispatch_keyset | c10::DispatchKeySet(c10::DispatchKey::ADInplaceOrView);
-  return keys;
-}
-// (by the bits: the sets' difference keeps the bits of the backends)
-bool only(c10::DispatchKeySet keys, c10::DispatchKeySet allowed) { return (keys.raw_repr() & ~allowed.raw_repr()) == 0; }
-bool ordinary_thread() {
-  if (at::impl::PythonTorchFunctionTLS::stack_len() != 0 || c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
-  return only(c10::impl::tls_local_dispatch_key_set().included_, plain_tls());
-}
-bool plain(const Tensor &t, const c10::Device &device) {
-  return t.defined() && t.is_cuda() && t.device() == device && t.layout() == at::kStrided && only(t.key_set(), plain_keys()) &&
-         !t._fw_grad(0).defined();
-}
 bool needs_grad(const optional<Tensor> &t) { return t.has_value() && t->requires_grad(); }
 
 // None -> no value; an exact torch.Tensor / Parameter -> its tensor; anything else -> false.
@@ -252,12 +297,12 @@ bool tensor_or_none(PyObject *o, optional<Tensor> &t) {
   return true;
 }
 
-// group_norm(x, weight, bias, num_groups, eps, act_code, out_dtype, residual, channel_bias, return_sum)
-//   -> y, (y, sum), or NotImplemented.
+// group_norm(x, weight, bias, num_groups, eps, act_code, out_dtype, residual, channel_bias, return_sum[, functional])
+//   -> y, (y, sum), or NotImplemented.  functional: on behalf of group_norm_nhwc, whose derivative is the operators' own.
 PyObject *group_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK(nargs == 10, "group_norm takes 10 arguments");
-  constexpr int kX = 0, kW = 1, kB = 2, kG = 3, kEps = 4, kAct = 5, kOut = 6, kRes = 7, kCb = 8, kSum = 9;
+  TORCH_CHECK(nargs == 10 || nargs == 11, "group_norm takes 10 or 11 arguments");
+  constexpr int kX = 0, kW = 1, kB = 2, kG = 3, kEps = 4, kAct = 5, kOut = 6, kRes = 7, kCb = 8, kSum = 9, kFunctional = 10;
   auto decline = []() { Py_RETURN_NOTIMPLEMENTED; };
   if (!THPVariable_CheckExact(args[kX]) || !ordinary_thread()) return decline();
   const Tensor &x = THPVariable_Unpack(args[kX]);
@@ -313,7 +358,9 @@ PyObject *group_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     }
   }
   if (grad) {
-    return THPVariable_Wrap(GroupNormNode::apply(x, weight, bias, G, eps, act, first, (int64_t)out));
+    // (the module goes through the functional form where the result leaves in another type)
+    const bool functional = (nargs == 11 && args[kFunctional] == Py_True) || out != x.scalar_type();
+    return THPVariable_Wrap(GroupNormNode::apply(x, weight, bias, G, eps, act, first, (int64_t)out, functional));
   }
   Tensor stats;
   if (add.any && want_sum) {
@@ -352,7 +399,7 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 
 PyMethodDef methods[] = {
     {"group_norm", (PyCFunction)(void (*)(void))group_norm, METH_FASTCALL,
-     "group_norm(x, weight, bias, num_groups, eps, act_code, out_dtype, residual, channel_bias, return_sum) -> y, (y, sum) "
+     "group_norm(x, weight, bias, num_groups, eps, act_code, out_dtype, residual, channel_bias, return_sum[, functional]) -> y, (y, sum) "
      "or NotImplemented"},
     {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, "bind(*addresses): the C ABI's entry points"},
     {nullptr, nullptr, 0, nullptr}};

@@ -532,7 +532,7 @@ def group_norm_nhwc(x, weight, bias, num_groups, eps=1e-5, activation="identity"
         raise RuntimeError("group_norm_nhwc expects channels-last input (stride 1 along dim 1)")
     if weight is not None and not torch.compiler.is_compiling():
         out = _native.group_norm(x, weight, bias, num_groups, eps, ACTIVATION_CODES[activation], out_dtype, residual, channel_bias,
-                                 return_sum)
+                                 return_sum, True)
         if out is not NotImplemented:
             return out
     nd = x.dim()

@@ -295,3 +295,74 @@ def test_saved_tensors_of_another_device_type_or_size_are_refused(device):
             y = m(x)
         with pytest.raises(RuntimeError, match=message):
             y.sum().backward()
+
+
+# Backwards that are no ordinary call go through the operators, whose formula group_norm_nhwc's derivative is.
+@pytest.mark.gpu
+@pytest.mark.filterwarnings("ignore:There is a performance drop")
+@pytest.mark.parametrize("out", [None, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(2, 32, 6, 5), (2, 12, 7), (1, 8, 3, 4, 5)])
+def test_batched_gradients_of_the_functional_form(shape, out, device):
+    m = GN_NHWC(4, shape[1]).to(device)
+    x = _channels_last(torch.randn(shape, device=device)).requires_grad_()
+    y = group_norm_nhwc(x, m.weight, m.bias, 4, m.eps, "silu", out_dtype=out)
+    dys = torch.randn((3, *shape), device=device).to(y.dtype)
+    got = torch.autograd.grad(y, (x, m.weight, m.bias), dys, retain_graph=True, is_grads_batched=True)
+    for i in range(3):
+        want = torch.autograd.grad(y, (x, m.weight, m.bias), dys[i], retain_graph=True)
+        for s, t in zip(got, want):
+            assert torch.equal(s[i], t)
+    small = _channels_last(torch.randn(1, 4, 2, device=device))
+    jac = torch.autograd.functional.jacobian(lambda t: group_norm_nhwc(t, m.weight[:4].detach(), m.bias[:4].detach(), 2), small, vectorize=True)
+    want = torch.autograd.functional.jacobian(lambda t: torch.nn.functional.group_norm(t, 2, m.weight[:4], m.bias[:4]), small)
+    assert (jac - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.gpu
+def test_the_functional_forms_backward_is_seen_by_modes_and_graphs(device):
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    m = GN_NHWC(4, 32, activation="silu").to(device)
+    x = _channels_last(torch.randn(2, 32, 6, 5, device=device)).requires_grad_()
+    y = group_norm_nhwc(x, m.weight, m.bias, 4, m.eps, "silu")
+    want = torch.autograd.grad(y, (x, m.weight, m.bias), x.detach(), retain_graph=True)
+    with Mode():
+        got = torch.autograd.grad(y, (x, m.weight, m.bias), x.detach(), retain_graph=True)
+    assert "gnop.bwd.default" in seen
+    again = torch.autograd.grad(y, (x, m.weight, m.bias), x.detach(), create_graph=True)
+    for s, t, u in zip(got, want, again):
+        assert torch.equal(s, t) and torch.equal(u, t)
+        assert u.requires_grad  # the operator has no second derivative: autograd's fallback notes it and warns when it is asked for
+    # the module's own function never recorded its backward
+    assert not any(g.requires_grad for g in torch.autograd.grad(m(x), (x, m.weight, m.bias), x.detach(), create_graph=True))
+
+
+@pytest.mark.gpu
+def test_gradients_of_another_kind_through_the_module(device):
+    class Sub(torch.Tensor):
+        pass
+
+    for first in (False, True):
+        m = GN_NHWC(4, 32, activation="silu").to(device)
+        x = torch.randn(2, 32, 6, 5, device=device)
+        x = (x if first else _channels_last(x)).requires_grad_()
+        dys = torch.randn(3, 2, 32, 6, 5, device=device)
+        y = m(x)
+        want = [torch.autograd.grad(y, (x, m.weight, m.bias), d, retain_graph=True) for d in dys]
+        got = torch.autograd.grad(y, (x, m.weight, m.bias), dys, retain_graph=True, is_grads_batched=True)
+        for i in range(3):
+            for s, t in zip(got, want[i]):
+                assert torch.equal(s[i], t)
+        for s, t in zip(torch.autograd.grad(y, (x, m.weight, m.bias), dys[0].as_subclass(Sub)), want[0]):
+            assert torch.equal(s, t)
+    bare = GN_NHWC(4, 32, affine=False).to(device)
+    y = bare(x)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(y, x, dys, is_grads_batched=True)
