@@ -287,6 +287,18 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
 };
 
 // ---- what group_norm() takes -----------------------------------------------------------------------------------------
+// While it lives, other Python threads run: allocations may have to wait for the device, launches for a full queue or for
+// another thread's.  (Saved-tensor hooks and operators implemented in Python take the lock again by themselves.)
+class WithoutGil {
+ public:
+  WithoutGil() : state_(PyEval_SaveThread()) {}
+  ~WithoutGil() { PyEval_RestoreThread(state_); }
+  WithoutGil(const WithoutGil &) = delete;
+  WithoutGil &operator=(const WithoutGil &) = delete;
+
+ private:
+  PyThreadState *state_;
+};
 bool needs_grad(const optional<Tensor> &t) { return t.has_value() && t->requires_grad(); }
 
 // None -> no value; an exact torch.Tensor / Parameter -> its tensor; anything else -> false.
@@ -305,7 +317,7 @@ PyObject *group_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
   constexpr int kX = 0, kW = 1, kB = 2, kG = 3, kEps = 4, kAct = 5, kOut = 6, kRes = 7, kCb = 8, kSum = 9, kFunctional = 10;
   auto decline = []() { Py_RETURN_NOTIMPLEMENTED; };
   if (!THPVariable_CheckExact(args[kX]) || !ordinary_thread()) return decline();
-  const Tensor &x = THPVariable_Unpack(args[kX]);
+  const Tensor x = THPVariable_Unpack(args[kX]);
   optional<Tensor> weight, bias;
   Added add;
   if (!tensor_or_none(args[kW], weight) || !tensor_or_none(args[kB], bias) || !tensor_or_none(args[kRes], add.residual) ||
@@ -357,18 +369,23 @@ PyObject *group_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         return decline();
     }
   }
-  if (grad) {
-    // (the module goes through the functional form where the result leaves in another type)
-    const bool functional = (nargs == 11 && args[kFunctional] == Py_True) || out != x.scalar_type();
-    return THPVariable_Wrap(GroupNormNode::apply(x, weight, bias, G, eps, act, first, (int64_t)out, functional));
+  Tensor y;
+  {
+    const WithoutGil released;
+    if (grad) {
+      // (the module goes through the functional form where the result leaves in another type)
+      const bool functional = (nargs == 11 && args[kFunctional] == Py_True) || out != x.scalar_type();
+      y = GroupNormNode::apply(x, weight, bias, G, eps, act, first, (int64_t)out, functional);
+    } else {
+      if (want_sum) {
+        const c10::DeviceGuard guard(device);
+        const at::AutoDispatchBelowADInplaceOrView below;
+        add.sum = empty_channels_last(x, x.scalar_type());
+      }
+      Tensor stats;
+      y = run_forward(x, weight, bias, G, eps, (int)act, first, out, add, stats);
+    }
   }
-  Tensor stats;
-  if (add.any && want_sum) {
-    const c10::DeviceGuard guard(device);
-    const at::AutoDispatchBelowADInplaceOrView below;
-    add.sum = empty_channels_last(x, x.scalar_type());
-  }
-  Tensor y = run_forward(x, weight, bias, G, eps, (int)act, first, out, add, stats);
   if (!want_sum) return THPVariable_Wrap(y);
   PyObject *yo = THPVariable_Wrap(y);
   PyObject *so = yo ? THPVariable_Wrap(add.sum) : nullptr;

@@ -112,9 +112,10 @@ try:
     from . import _native  # csrc/gn_torch.cpp: the eager calls of GN_NHWC and group_norm_nhwc
 except ImportError as exc:
     raise ImportError("gnnhwc: the _native extension is not built or does not load (make -C %s): %s" % (_CSRC, exc)) from exc
-_native.bind(*[ctypes.cast(getattr(lib, "gnnhwc_" + name), ctypes.c_void_p).value
-               for name in ("last_error", "fwd_workspace_bytes", "bwd_workspace_bytes", "nchw_workspace_bytes", "fwd_cast",
-                            "bwd_cast", "fwd_add", "fwd_nchw", "bwd_nchw")])
+# the entry points the extension calls, in the order it binds them
+NATIVE_ENTRY_POINTS = ("last_error", "fwd_workspace_bytes", "bwd_workspace_bytes", "nchw_workspace_bytes", "fwd_cast", "bwd_cast",
+                       "fwd_add", "fwd_nchw", "bwd_nchw")
+_native.bind(*[ctypes.cast(getattr(lib, "gnnhwc_" + name), ctypes.c_void_p).value for name in NATIVE_ENTRY_POINTS])
 
 
 def last_error():

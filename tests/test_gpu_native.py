@@ -366,3 +366,32 @@ def test_gradients_of_another_kind_through_the_module(device):
     y = bare(x)
     with pytest.raises(RuntimeError):
         torch.autograd.grad(y, x, dys, is_grads_batched=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first", [False, True])
+def test_the_interpreter_lock_is_released_around_the_kernels(first, device):
+    """The extension's launches are replaced by CPython's own question whether the calling thread holds the lock: an answer
+    other than 0 is an error code of the launch."""
+    import ctypes
+
+    from gnnhwc import _cabi
+
+    asked = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    real = [ctypes.cast(getattr(_cabi.lib, "gnnhwc_" + name), ctypes.c_void_p).value for name in _cabi.NATIVE_ENTRY_POINTS]
+    launches = ("fwd_cast", "bwd_cast", "fwd_add", "fwd_nchw", "bwd_nchw")
+    m = GN_NHWC(4, 32).to(device)
+    x = torch.randn(2, 32, 6, 5, device=device)
+    x = x if first else _channels_last(x)
+    dy = torch.zeros_like(x)
+    _native.bind(*[asked if name in launches else address for name, address in zip(_cabi.NATIVE_ENTRY_POINTS, real)])
+    try:
+        with torch.no_grad():
+            m(x)
+            if not first:
+                group_norm_nhwc(x, m.weight, m.bias, 4, residual=x, return_sum=True)
+        x.requires_grad_()
+        torch.autograd.grad(m(x), x, dy)
+    finally:
+        _native.bind(*real)
+    torch.cuda.synchronize()
