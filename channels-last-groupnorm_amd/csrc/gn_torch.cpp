@@ -11,6 +11,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/dispatch/Dispatcher.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -123,6 +124,17 @@ Tensor in_layout(const Tensor &t, bool first) {
   return t.permute(o.last).contiguous().permute(o.back);
 }
 
+// The operator's name in torch's profiler, around one call.
+class OperatorRange {
+ public:
+  explicit OperatorRange(const char *what) : range_(at::RecordScope::FUNCTION) {
+    if (range_.isActive()) range_.before(what);
+  }
+
+ private:
+  at::RecordFunction range_;
+};
+
 struct Added {  // pre-additions of the forward (group_norm_nhwc)
   optional<Tensor> residual, channel_bias;
   Tensor sum;  // where x + residual + channel_bias goes (undefined: nowhere)
@@ -141,6 +153,7 @@ Tensor run_forward(const Tensor &x, const optional<Tensor> &weight, const option
   char *mean = (char *)stats.data_ptr(), *rstd = mean + s.N * G * stats.element_size();
   const size_t bytes = first ? abi.nchw_workspace_bytes(s.N, s.C, s.R, G, dt, 0) : abi.fwd_workspace_bytes(s.N, s.R, s.C, G, dt);
   const char *what = first ? "gnop::fwd_nchw" : add.any ? "gnop::fwd_add" : out != x.scalar_type() ? "gnop::fwd_cast" : "gnop::fwd";
+  const OperatorRange range(what);
   const Tensor ws = workspace(bytes, x, what);
   int rc;
   if (first)
@@ -274,6 +287,7 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
     }
     const char *mean = (const char *)stats.data_ptr(), *rstd = mean + s.N * G * stats.element_size();
     const size_t bytes = first ? abi.nchw_workspace_bytes(s.N, s.C, s.R, G, dt, 1) : abi.bwd_workspace_bytes(s.N, s.R, s.C, G, dt);
+    const OperatorRange range(what);
     const Tensor ws = workspace(bytes, x, what);
     void *const wp = weight.defined() ? weight.data_ptr() : nullptr, *const bp = bias.defined() ? bias.data_ptr() : nullptr;
     void *const dwp = dw.defined() ? dw.data_ptr() : nullptr, *const dbp = db.defined() ? db.data_ptr() : nullptr;

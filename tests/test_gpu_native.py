@@ -395,3 +395,22 @@ def test_the_interpreter_lock_is_released_around_the_kernels(first, device):
     finally:
         _native.bind(*real)
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_calls_appear_under_their_operators_names_in_the_profiler(device):
+    from torch.profiler import ProfilerActivity, profile
+
+    m = GN_NHWC(4, 32, activation="silu").to(device)
+    x = torch.randn(2, 32, 6, 5, device=device)
+    last = _channels_last(x).requires_grad_()
+    first = x.clone().requires_grad_()
+    with profile(activities=[ProfilerActivity.CPU]) as p:
+        m(last).sum().backward()
+        m(first).sum().backward()
+        with torch.no_grad():
+            group_norm_nhwc(last, m.weight, m.bias, 4, residual=last)
+            GN_NHWC(4, 32, out_dtype=torch.bfloat16).to(device)(last)
+    names = [e.key for e in p.key_averages()]
+    for name in ("gnop::fwd", "gnop::bwd", "gnop::fwd_nchw", "gnop::bwd_nchw", "gnop::fwd_add", "gnop::fwd_cast"):
+        assert name in names, (name, names)
