@@ -95,11 +95,18 @@ template <typename K> int resident_slots(K kernel) {
 
 // Row tiling of a resident launch with a register capacity of nv rows per lane: tiles of exactly nv rows per
 // lane (all loads useful; only the last tile of a sample may be short), every workgroup resident.
-// Returns false if it does not fit.  `rolling`: only the workgroups that exchange records have to be resident together.
+// Returns false if it does not fit.  `rolling`: only the workgroups that exchange records (a set) have to be resident
+// together, and they may take half of the device at most.  A set that fills the device waits for whatever else holds a
+// single slot of it, and while an expired set recovers (milliseconds) the set behind it could not become resident either,
+// so that its waits would expire as well, and so on through the launch.  With two sets' room the next one completes beside
+// it, a tenant may hold the other half, and two rolling launches (replayed graphs) do not starve each other.
+// What the other half gave: float16 (1, R, 256, 32), R = 320 / 384 / 448 / 512 Ki rows, 87 / 97 / 120 / 129 us against the
+// streaming pair's 91 / 114 / 118 / 134 us; at half, R = 256 Ki, 56 against 73.
 bool resident_tiling(const Plan &base, int64_t samples, int nv, int slots, Plan &out, bool rolling = false) {
   const int64_t columns = samples * base.nchunk;
   if (slots <= 0 || samples > 65535) return false;
   const int64_t together = rolling ? exchange_chunks(base) : columns;
+  if (rolling) slots /= 2;
   if (together > slots) return false;
   if (base.G > 8192 || base.C >= (1 << 23)) return false;  // the kernels index their records with 24-bit multiplies
   if ((base.lpr & (base.lpr - 1)) != 0) return false;  // ... and find a lane's row and column by shifts
@@ -160,10 +167,11 @@ ResidentWorkspace resident_bwd_ws(void *ws, const Plan &p) {
   return r;
 }
 
-// How many consecutive single-launch kernels over groups of samples still beat the streaming pair in the backward.  Each
-// launch pays a fixed latency of roughly 9 microseconds but moves 3 S bytes instead of the pair's 5 S (about 5.4 bytes
-// per nanosecond either way, and about 14 us fixed for the pair); measured on (N, 320, 128, 128) bf16: two launches
-// equal the pair at N = 4 and beat it by 14 % at N = 6, three launches by 6 % at N = 8.
+// How many consecutive single-launch kernels over groups of samples still beat the streaming kernels in the backward.  Each
+// launch pays a fixed latency of roughly 9 microseconds but moves 3 S bytes instead of 5 S (about 5.4 bytes per nanosecond
+// either way, and about 14 us fixed for the streaming kernels).  Measured on (N, 320, 128, 128) bf16, cold tensors: one
+// launch 27.0 against 44.4 us at N = 4 and 35.9 against 67.4 at N = 6, two 52.5 against 87.6 at N = 8 and 71.0 against 121.0
+// at N = 12, three 103.4 against 162.2 at N = 16.
 int worthwhile_batches(const Plan &p) {
   const double s_mb = (double)p.N * p.R * p.C * sizeof(elem_t) / 1e6;
   const double k = (14.0 + 0.405 * s_mb) / 9.0;
@@ -174,11 +182,11 @@ size_t stat_size(int sdtype) { return sdtype == GN_F32 ? 4 : sdtype == GN_F64 ? 
 
 #if GN_PART_FWD || GN_PART_ADD
 // One NV variant: the tensor resident as a whole, or (rolling) set by set.  A rolling launch reads x once where the streaming
-// pair reads it twice, and its sets overlap each other's loads, exchanges and stores: bf16 (8 / 12 / 16, 320, 128, 128)
-// 47.7 / 72.1 / 100.2 -> 35.8 / 48.6 / 78.7 us (cold tensors), float32 (2, 256, 256, 256) 67.6 -> 49.4 = 5.4 TB/s, float16
-// (1, 256, 512, 1024) 143.6 -> 133.9; with a residual and the sum written, (16, 320, 128, 128) 185 -> 146.  One sample of a
-// chunk has to fit the device: 524288 rows of 128 bytes (chunks of half the width, which would fit twice the rows, are
-// slower than the streaming pair: 371 against 343 us for (1, 256, 1024, 1024) float16).
+// pair reads it twice, and its sets overlap each other's loads, exchanges and stores; on cold tensors, rolling against the
+// streaming pair: bf16 (8 / 12 / 16, 320, 128, 128) 39.1 / 58.3 / 76.7 against 48.1 / 70.7 / 99.0 us, float32
+// (2, 256, 256, 256) 58.8 against 70.3, float16 (1, 256, 512, 512) 55.7 against 73.4; with a residual and the sum written,
+// bf16 (16, 320, 128, 128) 145 against 193.  One set has to fit half of the device (resident_tiling): with groups inside a
+// chunk, samples of 262144 rows of 128 bytes.
 template <typename PT, int ACT, int NV, int ADD>
 bool try_resident_fwd_nv(const FwdArgs &a, const FwdRecords &records, bool rolling) {
   if (NV < resident_min_rows()) return false;

@@ -9,10 +9,10 @@ from tests.gpu_harness import cabi_fwd, cabi_fwd_add
 
 pytestmark = pytest.mark.gpu
 
-# N, R, C, G: sets of one chunk (groups inside a chunk; several in flight, and one that fills the device), of two and three
+# N, R, C, G: sets of one chunk (groups inside a chunk; several in flight, and one that takes half the device), of two and three
 # chunks (groups across chunk borders), of a whole sample (one group), a last tile of one row, of all but one, chunks of 32 bytes
-SHAPES = [(7, 16384, 320, 32), (1, 524288, 192, 12), (2, 65537, 256, 32), (3, 40000, 640, 8), (70, 513, 1280, 32), (2, 32767, 1088, 4),
-          (3, 65536, 256, 1), (9, 16384, 272, 17)]
+SHAPES = [(7, 16384, 320, 32), (1, 262144, 192, 12), (2, 65537, 256, 32), (3, 40000, 640, 8), (70, 513, 1280, 32), (2, 24575, 1088, 4),
+          (6, 32768, 256, 1), (9, 16384, 272, 17)]
 
 
 def _inputs(N, R, C, dtype, device):
@@ -99,3 +99,55 @@ def test_replayed_graph(device):
         want = cabi_fwd(x, w, b, 32, 1e-5, 2)[0]
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+# One row more than half the device holds, and sets of two and of four chunks beyond it: such a launch would have to have the
+# device to itself, so the streaming kernels take these calls.
+@pytest.mark.parametrize("N,R,C,G", [(1, 262145, 192, 12), (1, 524288, 192, 12), (1, 131073, 320, 32), (2, 65537, 256, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_sets_beyond_half_the_device_are_streamed(N, R, C, G, dtype, device):
+    C = C // 2 if dtype == torch.float32 and C != 320 else C  # chunks are 128 bytes wide
+    x, w, b = _inputs(N, R, C, dtype, device)
+    cabi_fwd(x, w, b, G, 1e-5, 2)
+    assert _cabi.last_launch() == "multi-launch"
+    cabi_fwd_add(x, None, torch.zeros(N, C, device=device, dtype=dtype), w, b, G, 1e-5, 2)
+    assert _cabi.last_launch() == "multi-launch"
+
+
+def _beside(tenant, x, w, b, x2, w2, b2):
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    want = [cabi_fwd(x, w, b, 32, 1e-5, 2), cabi_fwd(x2, w2, b2, 32, 1e-5, 2)]
+    torch.cuda.synchronize()
+    _cabi.lib.gnnhwc_resident_status()
+    for stream in streams:
+        with torch.cuda.stream(stream):
+            tenant()
+    got = [cabi_fwd(x, w, b, 32, 1e-5, 2), cabi_fwd(x2, w2, b2, 32, 1e-5, 2)]
+    torch.cuda.current_stream().synchronize()
+    print("tenants still there at the end:", [not stream.query() for stream in streams], flush=True)
+    torch.cuda.synchronize()
+    return want, got, _cabi.lib.gnnhwc_resident_status()
+
+
+def test_beside_kernels_that_hold_a_few_places(device):
+    """Kernels of other streams hold a place of the device each for as long as the launches below take many times over: the
+    largest set there is becomes resident beside them, no wait expires, and the results are those of a quiet device."""
+    a, c = _inputs(1, 262144, 256, torch.float16, device), _inputs(9, 16384, 320, torch.bfloat16, device)
+    want, got, expired = _beside(lambda: torch.cuda._sleep(50_000_000), *a, *c)
+    assert expired == 0
+    for s, t in zip(got, want):
+        for u, v in zip(s, t):
+            assert torch.equal(u, v)
+
+
+def test_beside_kernels_that_fill_the_device(device):
+    """The same beside matrix products of another stream, whose workgroups take whole CUs: whether waits expire is then a
+    matter of timing, the results are not (statistics that were recomputed are rounded once, from double precision)."""
+    a, c = _inputs(1, 262144, 256, torch.float16, device), _inputs(9, 16384, 320, torch.bfloat16, device)
+    m = torch.randn(8192, 8192, device=device).bfloat16()
+    out = torch.empty_like(m)
+    torch.mm(m, m, out=out)
+    want, got, expired = _beside(lambda: [torch.mm(m, m, out=out) for _ in range(4)], *a, *c)
+    print("expired", expired, flush=True)
+    for (y, mean, rstd), (y0, mean0, rstd0) in zip(got, want):
+        _close(y, y0, mean, mean0, rstd, rstd0)
