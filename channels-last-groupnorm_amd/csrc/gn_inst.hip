@@ -194,6 +194,7 @@ bool try_resident_fwd_nv(const FwdArgs &a, const FwdRecords &records, bool rolli
   auto kernel_two = fused_fwd_kernel<elem_t, PT, kVec, ACT, NV, ADD, true>;   // two-level exchange (many tiles)
   static const int slots = std::min(resident_slots(kernel_all), resident_slots(kernel_two));
   Plan p;
+  if (rolling && cooperative_launches()) return false;  // the runtime refuses a cooperative grid larger than the device
   if (!resident_tiling(a.plan, a.plan.N, NV, slots, p, rolling)) return false;
   // A rolling launch works with 16 rows per lane while a set is at most an eighth of what is resident -- several sets are
   // then in every phase at any time -- and with 32 beyond that, where a set's exchange weighs more: bf16 (8, 320, 128, 128)

@@ -151,3 +151,28 @@ def test_beside_kernels_that_fill_the_device(device):
     print("expired", expired, flush=True)
     for (y, mean, rstd), (y0, mean0, rstd0) in zip(got, want):
         _close(y, y0, mean, mean0, rstd, rstd0)
+
+
+def test_cooperative_switch_keeps_to_grids_the_runtime_admits(device):
+    """GNNHWC_COOPERATIVE=1 sends single-launch kernels through the runtime's cooperative launch, which refuses a grid larger
+    than the device: calls too large to be resident as a whole run on the streaming kernels then, the others as before."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import sys, torch
+from gnnhwc import _cabi
+from tests.gpu_harness import cabi_fwd
+for N in (2, 9):
+    x = torch.randn(N, 16384, 320, device="cuda", dtype=torch.bfloat16)
+    w = torch.ones(320, device="cuda", dtype=torch.bfloat16)
+    cabi_fwd(x, w, w, 32, 1e-5, 2)
+    torch.cuda.synchronize()
+    print(_cabi.last_launch().split()[0])
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = dict(os.environ, GNNHWC_COOPERATIVE="1", PYTHONPATH=os.pathsep.join((root, os.path.join(root, "channels-last-groupnorm_amd"))))
+    run = subprocess.run([sys.executable, "-c", code], env=env, cwd=root, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stderr
+    assert run.stdout.split() == ["fused_fwd", "multi-launch"]
