@@ -1,7 +1,7 @@
 """ctypes binding of libgnnhwc_hip.so (C ABI declared in include/gnnhwc.h).
 
-The library is built ahead of time, in-tree, by ``make -C channels-last-groupnorm_amd/csrc`` (or
-``__graft_entry__.build()``).  There is no fallback: if the shared object is missing or does not
+The library is built ahead of time, in-tree, by ``make -C channels-last-groupnorm_amd/csrc all native`` (or
+``__graft_entry__.build()``); `native` is the extension of the eager calls.  There is no fallback: if the shared object is missing or does not
 export the expected symbols, importing this module raises.
 """
 import ctypes
@@ -111,7 +111,7 @@ lib = _load()
 try:
     from . import _native  # csrc/gn_torch.cpp: the eager calls of GN_NHWC and group_norm_nhwc
 except ImportError as exc:
-    raise ImportError("gnnhwc: the _native extension is not built or does not load (make -C %s): %s" % (_CSRC, exc)) from exc
+    raise ImportError("gnnhwc: the _native extension is not built or does not load (make -C %s native): %s" % (_CSRC, exc)) from exc
 # the entry points the extension calls, in the order it binds them
 NATIVE_ENTRY_POINTS = ("last_error", "fwd_workspace_bytes", "bwd_workspace_bytes", "nchw_workspace_bytes", "fwd_cast", "bwd_cast",
                        "fwd_add", "fwd_nchw", "bwd_nchw")

@@ -272,3 +272,13 @@ def test_channels_first_argument_checks_need_no_gpu():
     rc = lib.gnnhwc_fwd_nchw(one, None, None, one, None, None, 1, 2, 2 ** 31, 1, 1e-5, 0, 0, 0, 0, one, 1 << 40, None)
     assert rc == -1 and "beyond the supported range" in _cabi.last_error()
 
+
+
+def test_the_libraries_build_without_torch():
+    """The default target is the C ABI alone; only `native` asks for torch and Python headers."""
+    import subprocess
+
+    csrc = os.path.join(ROOT, "channels-last-groupnorm_amd", "csrc")
+    plan = lambda *goals: subprocess.run(["make", "-n", "-B", "-C", csrc, *goals], check=True, capture_output=True, text=True).stdout  # noqa: E731
+    assert "libgnnhwc_hip.so" in plan() and "torch" not in plan()
+    assert "_native.so" in plan("native") and "torch" in plan("native")
