@@ -4,11 +4,11 @@
 //   forward : load tile -> per-tile group moments -> publish -> wait for the tiles that share my
 //             groups -> merge -> y = act(x a + b) from registers
 //   backward: load tile (x, dy) -> per-tile channel / group sums -> publish -> wait -> merge ->
-//             dx from registers; the workgroups of row tile 0 of sample 0 also finish dgamma / dbeta
+//             dx from registers; workgroups of the first sample also finish dgamma / dbeta (tail_blocks)
 //
-// The launch must be small enough for every workgroup to be resident at once (the host checks this
-// against the occupancy the runtime reports and otherwise uses the streaming kernels): a workgroup
-// spins on data written by other workgroups of the same launch.
+// A workgroup spins on data written by other workgroups of the same launch, so those must be resident together: the
+// whole launch, or in a forward larger than that each set of workgroups that exchange with each other (the host checks
+// this against the occupancy the runtime reports and otherwise uses the streaming kernels).
 //
 // Exchange protocol.  The XCDs' L2 caches are not coherent with each other, and the fences that would
 // make ordinary stores visible across them (L2 write-back / invalidate) cost tens of microseconds when
@@ -151,8 +151,9 @@ __device__ __forceinline__ float record_count(const Plan &p, int t, int k, int g
   const int rows = rem < p.tile_rows ? (int)rem : p.tile_rows;
   return (float)(c_hi - c_lo) * (float)rows;
 }
-// Slot of a record, in 32 bits with 24-bit multiplies: a single-launch kernel has at most kMaxResidentBlocksDev
-// workgroups, so (n nchunk + k) and tiles are small, and the host only sizes the record area for G below 2^20.
+// Slot of a record, in 32 bits with 24-bit multiplies.  A launch that is resident as a whole has at most
+// kMaxResidentBlocksDev workgroups and G is at most 8192, so (n nchunk + k) G + g and tiles are below 2^23; for a forward
+// run set by set the host checks both (resident_fwd_records, which also bounds all records by 32 MB).
 __device__ __forceinline__ int record_slot(const PartialGeo &q, int G, int n, int t, int k, int g) {
   const int col = __mul24(n, q.nchunk) + k;
   return __mul24(__mul24(col, G) + g, q.tiles) + t;

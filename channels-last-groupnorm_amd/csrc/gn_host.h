@@ -110,7 +110,8 @@ constexpr size_t kWorkspaceHeader = 256;
 constexpr int kMaxResidentBlocks = 4 * kNumCU;
 constexpr size_t kRollingRecordBytes = (size_t)32 << 20;
 inline size_t resident_rec_bytes(int64_t G) { return (size_t)16 * G * kMaxResidentBlocks; }
-// Final records of the two-level exchange, one per (sample, group) of a launch: a launch has at most kMaxResidentBlocks samples.
+// Final records of the two-level exchange, one per (sample, group) of a launch: a launch that is resident as a whole has at
+// most kMaxResidentBlocks samples (resident_fwd_records makes room for more where it runs set by set).
 inline size_t resident_frec_bytes(int64_t G) { return (size_t)16 * G * kMaxResidentBlocks; }
 // A forward too large to be resident as a whole still runs as ONE launch ("rolling") if every set of workgroups that
 // exchange records with each other is: workgroups are dispatched in linear order (row tiles, then chunks, then samples),
@@ -181,7 +182,8 @@ struct CapturedEpoch {
   unsigned long long next_sequence() const;  // differs between the captured launches of one graph
 };
 bool captured_epoch(hipStream_t stream, CapturedEpoch &out);
-// Two single-launch kernels must not share the device: each needs all of its workgroups resident at once.  Kernels
+// Two single-launch kernels must not share the device: each needs its workgroups resident at once, all of them or (a
+// forward run set by set) up to half of the device's worth.  Kernels
 // of one stream follow each other anyway; when a call arrives on another stream than the previous single-launch
 // call of the device, this makes the new stream wait for everything submitted so far on the previous one (an
 // event recorded there, no host synchronisation).  The object also serialises the host-side bookkeeping and the
@@ -223,8 +225,8 @@ inline bool needs_compaction(const Plan &producer, const Plan &consumer) {
   return lanes < 1 || per_group > (int64_t)kEarly * lanes;
 }
 // Tiling of a consumer (apply, dx) behind the producer's.  The producers want few, tall, narrow tiles, which leave few
-// partials; a consumer has none to leave, and many short tiles of whole rows, worked through in memory order, read and
-// write neighbouring lines at the same time: float16 (1, 256, 1024, 1024) apply 234 us with the producer's 764 tiles of
+// partials; a consumer has none to leave, and many short tiles of whole rows, of which those in flight are neighbours (from
+// the far end in blocks of eight, lane_pos), read and write neighbouring lines at the same time: float16 (1, 256, 1024, 1024) apply 234 us with the producer's 764 tiles of
 // 128-byte rows, 206 with 8 rows per lane, 168 with 8 rows per lane of 512 bytes.  Rows widen to the widest power of two
 // of lane vectors that divides them, unless their groups would then need a compaction launch that the narrow chunk does not
 // (or no longer fit one merge round); rows whose width no larger power of two divides gained nothing (bf16 (16, 320, 128, 128):

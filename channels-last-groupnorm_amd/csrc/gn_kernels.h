@@ -5,7 +5,7 @@
 //
 // Every large kernel walks the same Plan: a workgroup owns a tile of consecutive rows of one sample and
 // a chunk of whole 128-byte lines of each row; each lane owns VEC fixed channels and moves them with
-// one 128-bit access per row, two batches of rows in flight at a time.  The producers (stats,
+// one access per row (128 bits where channel count and addresses allow), two batches of rows in flight at a time.  The producers (stats,
 // bwd_reduce) leave one partial result per tile; the consumers (apply, bwd_dx) merge the partials of
 // the groups they touch in their own prologue, while their first loads are already in flight, so there
 // is no separate finalize launch unless a sample has so many tiles that the merge is first compacted

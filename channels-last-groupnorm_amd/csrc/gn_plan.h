@@ -63,7 +63,7 @@ __host__ __device__ __forceinline__ int div_by(int n, const Divisor &v) {
 struct Plan {
   int64_t N, R, C;
   int G, D;         // groups, channels per group
-  int vec;          // elements per lane vector (16 bytes / sizeof(T), or 1 for the scalar path)
+  int vec;          // elements per lane vector (16 bytes / sizeof(T), or a smaller power of two that divides C and the addresses)
   int cv;           // lane vectors per row = C / vec
   int lpr;          // lane vectors of a row handled by one workgroup (<= kBlock)
   int nchunk;       // workgroups side by side along C = ceil(cv / lpr)
