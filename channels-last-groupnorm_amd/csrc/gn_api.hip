@@ -877,19 +877,38 @@ int gnnhwc_bwd_nchw(const void *dy, const void *x, const void *weight, const voi
   return nchw_call(a, dtype, workspace, workspace_bytes, "channels-first backward");
 }
 
-int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward, int64_t *out) {
+static int debug_producer_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward, int64_t *out, Plan &p) {
   if (!out) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "null output array");
   const int rc = check_shape(N, R, C, G, dtype);
   if (rc != GNNHWC_OK) return rc;
   if (N == 0 || R == 0) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "empty problem: nothing is planned");
-  const int vec = 16 / elem_size(dtype);
-  if (vector && C % vec != 0) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "C = %lld is not a multiple of the vector width %d", (long long)C, vec);
-  const Plan p = make_plan(N, R, C, G, vector ? vec : 1, elem_size(dtype), backward ? 2 : 1);
+  const int full = 16 / elem_size(dtype), vec = vector == 0 ? 1 : vector == 1 ? full : vector;
+  if (vec != 1 && vec != 2 && vec != 4 && vec != full) return fail(GNNHWC_ERR_INVALID_ARGUMENT, "no kernels of vector width %d", vec);
+  if (vec > full || C % vec != 0)
+    return fail(GNNHWC_ERR_INVALID_ARGUMENT, "C = %lld is not a multiple of the vector width %d", (long long)C, vec);
+  p = make_plan(N, R, C, G, vec, elem_size(dtype), backward ? 2 : 1);
+  return GNNHWC_OK;
+}
+int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward, int64_t *out) {
+  Plan p;
+  const int rc = debug_producer_plan(N, R, C, G, dtype, vector, backward, out, p);
+  if (rc != GNNHWC_OK) return rc;
   const size_t elems = backward ? bwd_workspace(p).total : fwd_workspace(p).total;
   out[0] = p.vec; out[1] = p.cv; out[2] = p.lpr; out[3] = p.nchunk; out[4] = p.rpi; out[5] = p.tile_rows;
   out[6] = p.tiles; out[7] = p.gmax; out[8] = p.nblocks; out[9] = needs_compaction(p, consumer_plan(p, p.vec * elem_size(dtype))) ? 1 : 0;
   out[10] = (int64_t)(kWorkspaceHeader + elems * acc_size(dtype));
   out[11] = p.D;
+  return GNNHWC_OK;
+}
+int gnnhwc_debug_consumer_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward, int64_t *out) {
+  Plan p;
+  const int rc = debug_producer_plan(N, R, C, G, dtype, vector, backward, out, p);
+  if (rc != GNNHWC_OK) return rc;
+  const Plan c = consumer_plan(p, p.vec * elem_size(dtype));
+  out[0] = c.lpr; out[1] = c.nchunk; out[2] = c.rpi; out[3] = c.tile_rows; out[4] = c.tiles; out[5] = c.gmax; out[6] = c.nblocks;
+  const bool sets = !backward && dtype != GN_F64 && p.vec == 16 / elem_size(dtype);
+  const FwdRecords r = sets ? resident_fwd_records(p) : FwdRecords{0, 0, false};
+  out[7] = r.rolling ? 1 : 0; out[8] = (int64_t)r.rec; out[9] = (int64_t)r.frec; out[10] = sets ? exchange_chunks(p) : 0;
   return GNNHWC_OK;
 }
 

@@ -40,6 +40,7 @@ SYMBOLS = (
     "gnnhwc_resident_status",
     "gnnhwc_debug_read_trace",
     "gnnhwc_debug_plan",
+    "gnnhwc_debug_consumer_plan",
     "gnnhwc_debug_last_launch",
     "gnnhwc_debug_load_tile",
 )
@@ -100,6 +101,8 @@ def _load():
     lib.gnnhwc_debug_copy.restype = ci
     lib.gnnhwc_debug_plan.argtypes = [i64, i64, i64, i64, ci, ci, ci, ctypes.POINTER(i64)]
     lib.gnnhwc_debug_plan.restype = ci
+    lib.gnnhwc_debug_consumer_plan.argtypes = list(lib.gnnhwc_debug_plan.argtypes)
+    lib.gnnhwc_debug_consumer_plan.restype = ci
     lib.gnnhwc_debug_last_launch.argtypes = [ctypes.POINTER(i64)]
     lib.gnnhwc_debug_last_launch.restype = ci
     lib.gnnhwc_kernel_kind_name.argtypes = [ci]

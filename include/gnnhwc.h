@@ -314,13 +314,22 @@ int gnnhwc_debug_load_tile(const void *x, const void *dy, void *sink, int64_t N,
  * The tiling the multi-launch kernels would use for a problem (no counterpart in the reference, whose
  * calc_block_params, gn_kernel.cu:37-60, is internal too); nothing is launched, no GPU is needed.  For tests of the
  * host-side planning.  vector: 1 = 16-byte lane vectors (C must be a multiple of 16 / sizeof(dtype)), 0 = scalar
- * kernels; backward: 0 / 1.  out[12] receives: elements per lane vector, lane vectors per row, lane vectors of a
+ * kernels, 2 or 4 = lane vectors of that many elements; backward: 0 / 1.  out[12] receives: elements per lane vector, lane vectors per row, lane vectors of a
  * row per workgroup, chunks along C, rows per step, rows per tile, tiles per sample, most groups a chunk
  * intersects, workgroups per launch, 1 if a compaction launch runs between producer and consumer, bytes of
  * workspace this tiling needs, channels per group.
  */
 int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward,
                       int64_t *out /* [12] */);
+/*
+ * The tiling of the consumer (apply, dx) behind that plan, and what a forward run set by set would need.  out[11]
+ * receives: lane vectors of a row per workgroup, chunks along C, rows per step, rows per tile, tiles per sample, most
+ * groups a chunk intersects, workgroups per launch; then, forward with 16-byte lane vectors only (else 0): 1 if the
+ * record indices and the record memory allow such a launch, bytes of its tile records and of its final records
+ * (whether or not it is allowed), chunks of a set.
+ */
+int gnnhwc_debug_consumer_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward,
+                               int64_t *out /* [11] */);
 
 /*
  * In-kernel timeline of the single-launch kernels, for tuning (no counterpart in the reference; its

@@ -282,3 +282,89 @@ def test_the_libraries_build_without_torch():
     plan = lambda *goals: subprocess.run(["make", "-n", "-B", "-C", csrc, *goals], check=True, capture_output=True, text=True).stdout  # noqa: E731
     assert "libgnnhwc_hip.so" in plan() and "torch" not in plan()
     assert "_native.so" in plan("native") and "torch" in plan("native")
+
+
+def _sample_shapes(seed, count):
+    import random
+
+    rng = random.Random(seed)
+    for _ in range(count):
+        G = rng.choice([1, 2, 3, 4, 7, 8, 16, 24, 32, 64, 512])
+        D = rng.choice([1, 2, 3, 4, 5, 8, 10, 12, 20, 33, 40, 60, 128])
+        N = rng.choice([1, 1, 2, 3, 9, 70, 3000, 70000])
+        yield N, rng.choice([1, 2, 7, 64, 289, 1000, 1961, 4096, 16384, 100003, 1 << 20] if N < 100 else [1, 7, 64, 513]), G * D, G
+
+
+_ELEM = {0: 4, 1: 8, 2: 2, 3: 2}
+
+
+def test_narrow_lane_vectors_and_consumer_tilings_over_many_shapes():
+    """The plans of every lane vector width there are kernels for, and the consumer's own tiling behind them: rows and
+    channels are covered exactly once, a workgroup's lanes fit, no chunk meets more groups than the consumer's shared arrays
+    were sized for, and without a compaction launch the lanes of a group fetch all of its partials in one round."""
+    for (N, R, C, G) in _sample_shapes(6, 250):
+        for dtype in (0, 1, 2, 3):
+            full = 16 // _ELEM[dtype]
+            for vec in [v for v in (1, 2, 4, 8) if v <= full and C % v == 0]:
+                for backward in (0, 1):
+                    vector = 0 if vec == 1 else 1 if vec == full else vec
+                    p = _plan(N, R, C, G, dtype, vector, backward)
+                    out = (ctypes.c_int64 * 11)()
+                    assert _cabi.lib.gnnhwc_debug_consumer_plan(N, R, C, G, dtype, vector, backward, out) == 0
+                    lpr, nchunk, rpi, tile_rows, tiles, gmax, nblocks = (int(v) for v in out[:7])
+                    ctx = (N, R, C, G, dtype, vec, backward, p, list(out))
+                    assert p["vec"] == vec and p["cv"] * vec == C and p["nchunk"] <= 65535, ctx
+                    assert (p["nchunk"] - 1) * p["lpr"] < p["cv"] <= p["nchunk"] * p["lpr"], ctx
+                    assert (p["tiles"] - 1) * p["tile_rows"] < R <= p["tiles"] * p["tile_rows"], ctx
+                    query = (_cabi.lib.gnnhwc_bwd_workspace_bytes if backward else _cabi.lib.gnnhwc_fwd_workspace_bytes)(N, R, C, G, dtype)
+                    assert p["bytes"] <= query, ctx
+                    assert p["lpr"] <= lpr <= 256 and rpi == 256 // lpr and tile_rows % rpi == 0 and tile_rows >= rpi, ctx
+                    assert (nchunk - 1) * lpr < p["cv"] <= nchunk * lpr, ctx
+                    assert (tiles - 1) * tile_rows < R <= tiles * tile_rows and nblocks == N * tiles * nchunk, ctx
+                    assert tile_rows // rpi * vec * _ELEM[dtype] <= max(128, vec * _ELEM[dtype]), ctx
+                    D = C // G
+                    width = lpr * vec
+                    for k in {0, 1, nchunk // 2, nchunk - 2, nchunk - 1}:
+                        if 0 <= k < nchunk:
+                            assert (min(C, (k + 1) * width) - 1) // D - k * width // D + 1 <= gmax, (k, ctx)
+                    lanes = min(64, 256 // (1 << (gmax - 1).bit_length()))
+                    partials = p["tiles"] * ((D - 1) // (p["lpr"] * vec) + 2)  # of a group, over the producer's chunks
+                    assert p["compaction"] == (1 if lanes < 1 or partials > 4 * lanes else 0), ctx
+    out = (ctypes.c_int64 * 12)()
+    assert _cabi.lib.gnnhwc_debug_plan(1, 16, 12, 4, 3, 8, 0, out) == -1 and "vector width" in _cabi.last_error()
+    assert _cabi.lib.gnnhwc_debug_plan(1, 16, 12, 4, 0, 8, 0, out) == -1
+    assert _cabi.lib.gnnhwc_debug_plan(1, 16, 12, 4, 3, 3, 0, out) == -1
+
+
+def test_records_of_forwards_run_set_by_set():
+    """Where such a launch is allowed, its record indices stay below the kernels' 24-bit multiplies, the record memory holds
+    every (sample, chunk, group, tile) and (sample, group) it can address, and the workspace query covers it; the chunks of a
+    set are those that the groups of a chunk reach into."""
+    allowed = 0
+    shapes = [(16, 16384, 320, 32), (1, 262144, 256, 32), (70, 513, 1280, 32), (2, 24575, 1088, 4), (65535, 512, 64, 8), (65536, 512, 64, 8),
+              (3000, 513, 512, 512), (1, 511, 64, 8)]
+    for (N, R, C, G) in shapes + list(_sample_shapes(7, 400)):
+        for dtype in (0, 2, 3):
+            full = 16 // _ELEM[dtype]
+            if C % full:
+                continue
+            p = _plan(N, R, C, G, dtype, 1, 0)
+            out = (ctypes.c_int64 * 11)()
+            assert _cabi.lib.gnnhwc_debug_consumer_plan(N, R, C, G, dtype, 1, 0, out) == 0
+            rolling, rec, frec, chunks = (int(v) for v in out[7:])
+            ctx = (N, R, C, G, dtype, p, list(out))
+            assert rec >= 16 * G * 1024 and frec >= 16 * G * 1024, ctx  # launches that are resident as a whole
+            assert 256 + rec + frec <= _cabi.lib.gnnhwc_fwd_workspace_bytes(N, R, C, G, dtype), ctx
+            D, width = C // G, p["lpr"] * full
+            reach = max((((min(C, (k + 1) * width) - 1) // D + 1) * D - 1) // width - k for k in range(p["nchunk"])) + 1
+            assert reach <= chunks <= p["nchunk"], ctx
+            if not rolling:
+                continue
+            allowed += 1
+            columns = N * p["nchunk"]
+            for rows in (16, 32):  # rows per lane
+                tiles = -(-R // (rows * p["rpi"]))
+                assert columns * G < 1 << 23 and tiles < 1 << 23 and N <= 65535, ctx
+                assert 16 * columns * G * tiles <= rec and 16 * N * G <= frec, ctx
+            assert rec <= max(32 << 20, 16 * G * 1024 + 255), ctx
+    assert allowed > 100, allowed
