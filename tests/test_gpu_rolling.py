@@ -1,11 +1,13 @@
 """GPU tests of forward launches with more workgroups than fit the device at once: sets of workgroups that exchange records
-follow each other through it.  Against the streaming kernels on the same inputs (which tests/test_gpu_parity.py holds to
-the float64 oracle): statistics agree to float32 rounding, y to that or to one spacing of its 16-bit type."""
+follow each other through it.  Against torch in float64 and against the streaming kernels on the same inputs: statistics
+agree to float32 rounding, y to that or to one spacing of its 16-bit type."""
+import ctypes
+
 import pytest
 import torch
 
 from gnnhwc import _cabi
-from tests.gpu_harness import cabi_fwd, cabi_fwd_add
+from tests.gpu_harness import cabi_fwd, cabi_fwd_add, err
 
 pytestmark = pytest.mark.gpu
 
@@ -34,6 +36,31 @@ def _close(y, y0, mean, mean0, rstd, rstd0):
         assert ((a - t).abs() <= (eps if y.dtype != torch.float32 else 0) * t.abs() + 1e-5).all()
 
 
+def _assert_set_by_set(x, kernel="fused_fwd"):
+    """The last call was one launch of a single-launch kernel on more than the 64 MiB that such a launch can hold in
+    registers (512 workgroups of 32 rows per lane, or 1024 of 16): its workgroups were not all resident at once."""
+    out = (ctypes.c_int64 * 7)()
+    _cabi.check(_cabi.lib.gnnhwc_debug_last_launch(out), "gnnhwc_debug_last_launch")
+    assert out[0] >= 0 and _cabi.kernel_kind_names()[out[0]] == kernel, _cabi.last_launch()
+    rows, workgroups = int(out[1]), int(out[5])
+    assert out[4] == 1 and x.numel() * x.element_size() > 64 << 20
+    assert workgroups > (512 if rows == 32 else 1024), (rows, workgroups)
+
+
+def _against_float64(x, w, b, G, y, mean, rstd, eps=1e-5):
+    """y = silu(normalised x): within one rounding to its type of a value that meets the float32 bar (1e-5)."""
+    N, R, C = x.shape
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[x.dtype]
+    for n in range(N):
+        t = x[n].double().view(R, G, C // G)
+        mu = t.mean((0, 2), keepdim=True)
+        var = (t - mu).square().mean((0, 2), keepdim=True)
+        rs = (var + eps).rsqrt()
+        assert err(mean[n], mu) <= 1e-5 and err(rstd[n], rs) <= 1e-5
+        z = torch.nn.functional.silu(((t - mu) * rs).view(R, C) * w.double() + b.double())
+        assert bool(((y[n].double() - z).abs() <= half * z.abs() * 1.001 + 1e-5 * (z.abs() + 1.0)).all())
+
+
 def _streaming(fn):
     before = _cabi.set_resident(False)
     try:
@@ -44,11 +71,12 @@ def _streaming(fn):
 
 @pytest.mark.parametrize("N,R,C,G", SHAPES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-def test_against_the_streaming_kernels(N, R, C, G, dtype, device):
+def test_against_float64_and_the_streaming_kernels(N, R, C, G, dtype, device):
     print("rolling", N, R, C, G, dtype, flush=True)
     x, w, b = _inputs(N, R, C, dtype, device)
     y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
-    assert _cabi.last_launch().startswith("fused_fwd"), _cabi.last_launch()
+    _assert_set_by_set(x)
+    _against_float64(x, w, b, G, y, mean, rstd)
     again = cabi_fwd(x, w, b, G, 1e-5, 2)
     for s, t in zip((y, mean, rstd), again):
         assert torch.equal(s, t)
@@ -63,23 +91,62 @@ def test_with_fused_additions(device):
     x, w, b = _inputs(9, 16384, 320, torch.bfloat16, device)
     r, cb = torch.randn_like(x), torch.randn(9, 320, device=device).bfloat16()
     y, s, mean, rstd = cabi_fwd_add(x, r, cb, w, b, 32, 1e-5, 2)
-    assert _cabi.last_launch().startswith("fused_fwd_add"), _cabi.last_launch()
+    _assert_set_by_set(x, "fused_fwd_add")
+    _against_float64(s, w, b, 32, y, mean, rstd)
     y0, s0, mean0, rstd0 = _streaming(lambda: cabi_fwd_add(x, r, cb, w, b, 32, 1e-5, 2))
     assert torch.equal(s, s0)
     _close(y, y0, mean, mean0, rstd, rstd0)
 
 
+# The all-to-all exchange, and the two-level one (one row of the last tile; groups in the middle of chunks and across them).
+@pytest.mark.parametrize("N,R,C,G", [(14, 16384, 160, 16), (2, 65537, 256, 32)])
 @pytest.mark.parametrize("spins", [-2, 0, 2])
-def test_expired_waits_are_recovered(spins, device):
-    x, w, b = _inputs(14, 16384, 160, torch.bfloat16, device)
-    y0, mean0, rstd0 = _streaming(lambda: cabi_fwd(x, w, b, 16, 1e-5, 2))
+def test_expired_waits_are_recovered(spins, N, R, C, G, device):
+    x, w, b = _inputs(N, R, C, torch.bfloat16, device)
+    y0, mean0, rstd0 = _streaming(lambda: cabi_fwd(x, w, b, G, 1e-5, 2))
+    _cabi.lib.gnnhwc_resident_status()
     before = _cabi.lib.gnnhwc_debug_set_spin_limit(spins)
     try:
-        y, mean, rstd = cabi_fwd(x, w, b, 16, 1e-5, 2)
+        y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
+        torch.cuda.synchronize()
+    finally:
+        _cabi.lib.gnnhwc_debug_set_spin_limit(before)
+    _assert_set_by_set(x)
+    assert ("two_level=1" in _cabi.last_launch()) == (G == 32)
+    expired = _cabi.lib.gnnhwc_resident_status()
+    assert expired == 1 or spins != -2
+    _close(y, y0, mean, mean0, rstd, rstd0)
+    _against_float64(x, w, b, G, y, mean, rstd)
+    if spins == -2:
+        return  # (recomputes records whose workgroups may have stored already: out of place only)
+    before = _cabi.lib.gnnhwc_debug_set_spin_limit(spins)
+    try:
+        y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2, y=x)
         torch.cuda.synchronize()
     finally:
         _cabi.lib.gnnhwc_debug_set_spin_limit(before)
     _cabi.lib.gnnhwc_resident_status()
+    _close(y, y0, mean, mean0, rstd, rstd0)
+
+
+@pytest.mark.parametrize("R,G", [(16384, 32), (65537, 32)])
+@pytest.mark.parametrize("spins", [-2, 2])
+def test_expired_waits_with_fused_additions(spins, R, G, device):
+    N, C = (9, 320) if R == 16384 else (2, 256)
+    x, w, b = _inputs(N, R, C, torch.bfloat16, device)
+    r, cb = torch.randn_like(x), torch.randn(N, C, device=device).bfloat16()
+    y0, s0, mean0, rstd0 = _streaming(lambda: cabi_fwd_add(x, r, cb, w, b, G, 1e-5, 2))
+    _cabi.lib.gnnhwc_resident_status()
+    before = _cabi.lib.gnnhwc_debug_set_spin_limit(spins)
+    try:
+        y, s, mean, rstd = cabi_fwd_add(x, r, cb, w, b, G, 1e-5, 2)
+        torch.cuda.synchronize()
+    finally:
+        _cabi.lib.gnnhwc_debug_set_spin_limit(before)
+    _assert_set_by_set(x, "fused_fwd_add")
+    expired = _cabi.lib.gnnhwc_resident_status()
+    assert expired == 1 or spins != -2
+    assert torch.equal(s, s0)
     _close(y, y0, mean, mean0, rstd, rstd0)
 
 
@@ -92,6 +159,7 @@ def test_replayed_graph(device):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         cabi_fwd(x, w, b, 32, 1e-5, 2, y=y, ws=ws)
+        _assert_set_by_set(x)
     for i in range(3):
         x.add_(i)
         graph.replay()
