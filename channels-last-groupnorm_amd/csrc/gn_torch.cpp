@@ -195,6 +195,9 @@ bool plain(const Tensor &t, const c10::Device &device) {
          !t._fw_grad(0).defined();
 }
 
+// Memory the kernels can be given, whatever else the tensor carries.
+bool readable(const Tensor &t) { return t.has_storage() && !t.key_set().has(c10::DispatchKey::Python); }
+
 // The backward through the dispatcher, as the operators' registered formula calls it: for gradients and saved tensors that are
 // no plain device tensors (batched gradients, subclasses), and where something on this thread is to see the operator.
 torch::autograd::variable_list backward_operator(const Tensor &dy, const Tensor &x, const Tensor &weight, const Tensor &bias,
@@ -251,9 +254,10 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
     // (the module's own autograd function never recorded a graph of its backward; the functional form went through the operator)
     const at::AutoGradMode graph(functional && at::GradMode::is_enabled());
     Tensor dy = resolved(grads[0]), x = resolved(saved[0]);
-    const bool all_plain = plain(dy, device) && plain(x, device) && plain(saved[3], device) &&
-                           (!saved[1].defined() || (plain(saved[1], device) && plain(saved[2], device)));
-    if (!all_plain || (functional && saved[1].defined() && (at::GradMode::is_enabled() || !ordinary_dispatch())))
+    const bool formula = functional && saved[1].defined();  // (without parameters there is no operator to go through)
+    const auto kernels_take = [&](const Tensor &t) { return !t.defined() || (formula ? plain(t, device) : readable(t)); };
+    if ((formula && (at::GradMode::is_enabled() || !ordinary_dispatch())) || !kernels_take(dy) || !kernels_take(x) ||
+        !kernels_take(saved[1]) || !kernels_take(saved[2]) || !kernels_take(saved[3]))
       return backward_operator(dy, x, saved[1], saved[2], saved[3], G, act, first);
     const at::AutoGradMode no_graph(false);
     dy = in_layout(dy, first);

@@ -414,3 +414,23 @@ def test_calls_appear_under_their_operators_names_in_the_profiler(device):
     names = [e.key for e in p.key_averages()]
     for name in ("gnop::fwd", "gnop::bwd", "gnop::fwd_nchw", "gnop::bwd_nchw", "gnop::fwd_add", "gnop::fwd_cast"):
         assert name in names, (name, names)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("affine", [True, False])
+@pytest.mark.parametrize("out", [None, torch.bfloat16])
+def test_gradients_with_a_tangent(affine, out, device):
+    """The operators have no forward-mode derivative: a tangent of the gradient is dropped, the gradients are the same."""
+    import torch.autograd.forward_ad as fwAD
+
+    m = GN_NHWC(4, 32, activation="silu", affine=affine, out_dtype=out).to(device)
+    x = _channels_last(torch.randn(2, 32, 6, 5, device=device)).requires_grad_()
+    dy = torch.randn(2, 32, 6, 5, device=device).to(out or torch.float32)
+    inputs = (x, *m.parameters())
+    y = m(x)
+    want = torch.autograd.grad(y, inputs, dy, retain_graph=True)
+    with fwAD.dual_level():
+        got = torch.autograd.grad(y, inputs, fwAD.make_dual(dy, torch.ones_like(dy)))
+        got = [fwAD.unpack_dual(t).primal.clone() for t in got]
+    for s, t in zip(got, want):
+        assert torch.equal(s, t)
