@@ -224,6 +224,10 @@ inline bool needs_compaction(const Plan &producer, const Plan &consumer) {
   const int lanes = merge_lanes_for(consumer.gmax);
   return lanes < 1 || per_group > (int64_t)kEarly * lanes;
 }
+// What the 256 MB memory-side cache is counted on to hold from a producer's reads to its consumer's (the consumer of float16
+// (1, 256, 1024, 1024), 537 MB: 171 us with 96 MB kept, 169 with 160, 167 with 192 or 224, 165 with 256, where the producer
+// in turn takes 4 us more).
+constexpr size_t kCacheBytes = (size_t)224 << 20;
 // Tiling of a consumer (apply, dx) behind the producer's.  The producers want few, tall, narrow tiles, which leave few
 // partials; a consumer has none to leave, and many short tiles of whole rows, of which those in flight are neighbours (from
 // the far end in blocks of eight, lane_pos), read and write neighbouring lines at the same time: float16 (1, 256, 1024, 1024) apply 234 us with the producer's 764 tiles of

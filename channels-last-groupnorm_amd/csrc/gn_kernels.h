@@ -288,80 +288,123 @@ __device__ __forceinline__ void group_span(const Plan &p, const LanePos &l, int 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Running per-channel statistics of one lane over its rows of the tile.  Each batch of rows is folded
-// with an exact two-pass mean / sum of squares on the values held in registers and merged into the
-// running moments with Chan's update: one reciprocal per batch instead of the per-element division of
-// WelfordOps::reduce (src/gnnhwc/csrc/Welford.h:30-42).
+// Running per-channel statistics of one lane over the rows it sweeps (sweep_rows).  A batch of rows is folded as sums of
+// deviations, and of their squares, from a pivot K: the lane's running mean (its first row to begin with: a value of the
+// data), so that nothing cancels.  With n elements behind K and m more, S1 = sum (v - K), S2 = sum (v - K)^2,
+//   mean = K + S1 / (n + m),   M2 += S2 - S1^2 / (n + m)
+// (Chan's update in pivot form; WelfordOps::reduce, src/gnnhwc/csrc/Welford.h:30-42, divides once per element): three
+// operations per element and four per channel and batch.
 // ---------------------------------------------------------------------------------------------
 template <typename T, int VEC, int U>
 __device__ __forceinline__ void fold_batch(const typename LaneVec<T, VEC>::raw_t (&raw)[U], int m, acc_t<T> &cnt,
                                            acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
   using A = acc_t<T>;
-  A s[VEC], qq[VEC];
+  A s1[VEC], s2[VEC];
+  if (cnt == (A)0) LaneVec<T, VEC>::unpack(raw[0], mean);
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) { s[j] = (A)0; qq[j] = (A)0; }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const A keep = u < m ? (A)1 : (A)0;
-    A v[VEC];
-    LaneVec<T, VEC>::unpack(raw[u], v);
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) s[j] += keep * v[j];
-  }
-  const A mf = (A)m;
-  const A inv_m = fast_rcp(mf);
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) s[j] *= inv_m;  // batch mean
+  for (int j = 0; j < VEC; ++j) { s1[j] = (A)0; s2[j] = (A)0; }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const A keep = u < m ? (A)1 : (A)0;
-    A v[VEC];
-    LaneVec<T, VEC>::unpack(raw[u], v);
+    if (u < m) {  // (m is U except in a lane's last batch)
+      A v[VEC];
+      LaneVec<T, VEC>::unpack(raw[u], v);
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) { const A d = v[j] - s[j]; qq[j] += keep * d * d; }
+      for (int j = 0; j < VEC; ++j) {
+        const A d = v[j] - mean[j];
+        s1[j] += d;
+        s2[j] += d * d;
+      }
+    }
   }
-  const A nn = cnt + mf;
-  const A f = mf * fast_rcp(nn);
+  cnt += (A)m;
+  const A inv = fast_rcp(cnt);
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
-    const A d = s[j] - mean[j];
-    mean[j] += d * f;
-    m2[j] += qq[j] + d * d * cnt * f;
+    const A t = s1[j] * inv;
+    mean[j] += t;
+    m2[j] += s2[j] - s1[j] * t;
   }
-  cnt = nn;
 }
 
+// The rows of a statistics workgroup: not a run of neighbours but every p.tiles-th batch of the sample (Sweep), beginning
+// with batch number `tile`.  The workgroups in flight then sweep the
+// sample from its first row to its last together, and the rows read last are the sample's last rows -- where the consumer,
+// which walks from the far end, begins.
+struct SweptRows {
+  int nb;     // batches of this workgroup, the last one of a sample possibly short
+  bool last;  // it owns that one
+};
+__device__ __forceinline__ SweptRows sweep_rows(const Plan &p, const Sweep &sw, LanePos &l) {
+  SweptRows s;
+  const int behind = sw.batches - 1 - l.tile;  // (a plan has no more tiles than batches)
+  const int more = div_by(behind, p.by_tiles);
+  s.nb = more + 1;
+  s.last = behind == more * p.tiles;
+  const int batch_rows = sw.steps * p.rpi;
+  const int rem = s.last ? sw.last_rows : batch_rows;  // rows of the workgroup's last batch
+  l.row0 = (int64_t)l.tile * batch_rows;
+  l.len = more * batch_rows + rem;
+  l.rows_base = div_by(rem, p.by_rpi);
+  l.rows_rem = rem - l.rows_base * p.rpi;
+  l.rows_base += more * sw.steps;
+  l.rows = l.active ? l.rows_base + (l.ty < l.rows_rem ? 1 : 0) : 0;
+  return s;
+}
+
+// Batches below sw.keep_from are read with the non-temporal hint, which leaves no copy behind in the memory-side cache.
+// Bound: memory.  A tensor that exceeds that cache arrives at 6.0 TB/s by plain loads and at 6.9 by non-temporal ones, and
+// what non-temporal loads have read is not found there by a later pass (measured on a 537 MB read alone: 88 against 78 us; a
+// copy behind it, from the far end: 160 against 167).  float16 (1, 256, 1024, 1024): 103 us with tiles of neighbouring rows, plain
+// loads and the statistics in two passes over each batch (7.5 vector operations per element); 90 in this form.
 template <typename T, int VEC, int U>
-__device__ __forceinline__ void lane_stats(const T *__restrict__ x, const Plan &p, const LanePos &l,
-                                           acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
+__device__ __forceinline__ void lane_stats(const T *__restrict__ x, const Plan &p, const LanePos &l, const Sweep &sw,
+                                           const SweptRows &s, acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
   using A = acc_t<T>;
   using LV = LaneVec<T, VEC>;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) { mean[j] = (A)0; m2[j] = (A)0; }
   A cnt = (A)0;
   const int rows = l.rows;
-  const int nb = block_batches<U>(p, l);
   if (rows == 0) return;
   const T *base = x + ((l.n * p.R + l.row0 + l.ty) * p.C + (int64_t)l.cvi * VEC);
-  const int64_t step = (int64_t)p.rpi * p.C;
-  typename LV::raw_t buf0[U], buf1[U];
-  auto issue = [&](auto sel, int b) {
+  const int64_t step = (int64_t)p.rpi * p.C, sweep = (int64_t)p.tiles * sw.steps * step;
+  // batches with all U rows for every lane: [0, keep) non-temporal, [keep, full) plain; no choice is left to the inside of
+  // either loop, where a branch around the loads would make the waits behind it drain the queue
+  const int full = sw.steps == U ? (s.last ? s.nb - 1 : s.nb) : 0;
+  // (narrow lane vectors do without the first loop: tensors of that size and such a channel count are not worth its code)
+  constexpr bool kSweepCold = VEC == vec_of<T>::value;
+  const int keep = sw.keep_from < full ? sw.keep_from : full;
+  auto sweep_batches = [&](auto streaming, int first, int end) {
+    if (first >= end) return;
+    typename LV::raw_t buf0[U], buf1[U];
+    auto issue = [&](auto sel, int b) {
+      const T *src = base + (first + b) * sweep;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const T *src = base + (int64_t)clamp_row(b * U + u, rows) * step;
-      if constexpr (decltype(sel)::value == 0) buf0[u] = LV::load(src);
-      else buf1[u] = LV::load(src);
-    }
+      for (int u = 0; u < U; ++u) {
+        typename LV::raw_t &r = decltype(sel)::value == 0 ? buf0[u] : buf1[u];
+        if constexpr (decltype(streaming)::value) r = load_streaming<LV>(src + u * step);
+        else r = LV::load(src + u * step);
+      }
+      issue_order_fence();  // ahead of the rows consumed meanwhile
+    };
+    auto consume = [&](auto sel, int) {
+      if constexpr (decltype(sel)::value == 0) fold_batch<T, VEC, U>(buf0, U, cnt, mean, m2);
+      else fold_batch<T, VEC, U>(buf1, U, cnt, mean, m2);
+    };
+    issue(std::integral_constant<int, 0>{}, 0);
+    double_buffered(end - first, issue, consume);
   };
-  auto consume = [&](auto sel, int b) {
-    int m = rows - b * U;
-    m = m < 0 ? 0 : (m > U ? U : m);
-    if (m == 0) return;  // only in the last batch of a lane row that is one row short
-    if constexpr (decltype(sel)::value == 0) fold_batch<T, VEC, U>(buf0, m, cnt, mean, m2);
-    else fold_batch<T, VEC, U>(buf1, m, cnt, mean, m2);
-  };
-  issue(std::integral_constant<int, 0>{}, 0);
-  double_buffered(nb, issue, consume);
+  if constexpr (kSweepCold) sweep_batches(std::true_type{}, 0, keep);
+  sweep_batches(std::false_type{}, kSweepCold ? keep : 0, full);
+  // the rows of the one batch left: the sample's last, or that of a tile shorter than U rows per lane
+  constexpr int V = U < kUnrollFwd ? U : kUnrollFwd;
+  const T *src = base + full * sweep;
+  for (int m = rows - full * sw.steps; m > 0; m -= V, src += V * step) {
+    typename LV::raw_t buf[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) buf[u] = LV::load(src + clamp_row(u, m) * step);
+    fold_batch<T, VEC, V>(buf, m < V ? m : V, cnt, mean, m2);
+  }
 }
 
 // Sum of col[0], col[stride], ... (n entries) with eight reads in flight: the loop is latency bound otherwise.
@@ -552,16 +595,17 @@ __global__ __launch_bounds__(kBlock) void add_flat_kernel(const T *__restrict__ 
 // ---------------------------------------------------------------------------------------------
 template <typename T, int VEC>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void stats_kernel(
-    const T *__restrict__ x, acc_t<T> *__restrict__ part, Plan p) {
+    const T *__restrict__ x, acc_t<T> *__restrict__ part, Plan p, Sweep sw) {
   using A = acc_t<T>;
   __shared__ A sm_mean[kBlock * VEC];
   __shared__ A sm_m2[kBlock * VEC];
   const PartialGeo q = producer_geo(p);
   const int64_t plane = group_plane(q, p.G, p.N);
   for (int64_t n = blockIdx.z; n < p.N; n += gridDim.z) {
-    const LanePos l = lane_pos(p, n, false);
+    LanePos l = lane_pos(p, n, false);
+    const SweptRows sweep = sweep_rows(p, sw, l);
     A mean[VEC], m2[VEC];
-    lane_stats<T, VEC, kUnrollFwd>(x, p, l, mean, m2);
+    lane_stats<T, VEC, kUnrollStats>(x, p, l, sw, sweep, mean, m2);
     block_group_moments<A, VEC>(p, l, mean, m2, sm_mean, sm_m2, [&](int g, A cnt, A mu, A s2) {
       const int64_t slot = group_slot(q, p.G, n, l.tile, l.chunk, g);
       part[slot] = cnt;
@@ -778,7 +822,7 @@ __device__ __forceinline__ void lane_coeffs(const Plan &p, const LanePos &l, con
 // shape with one code path (no R % 8 fast / slow split).  y is computed from the unrounded mean / rstd
 // whatever type the reported statistics have (cf. gn_kernel.cu:290-291).
 // ---------------------------------------------------------------------------------------------
-template <typename T, typename PT, int VEC, int ACT>
+template <typename T, typename PT, int VEC, int ACT, bool LAST_USE>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void apply_kernel(
     const T *__restrict__ x, T *__restrict__ y, const acc_t<T> *__restrict__ part, PartialGeo q, const void *w,
     const void *b, void *mean_out, void *rstd_out, int sdtype, int ydtype, acc_t<T> eps, Plan p) {
@@ -788,7 +832,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   __shared__ A sm_mu[kBlock * VEC];
   __shared__ A sm_rs[kBlock * VEC];
   const bool one_round = pow2_at_least(p.gmax) <= kBlock;
-  for (int64_t n = blockIdx.z; n < p.N; n += gridDim.z) {
+  for (int64_t z = blockIdx.z; z < p.N; z += gridDim.z) {
+    const int64_t n = p.N - 1 - z;  // from the far end, as the tiles
     const LanePos l = lane_pos(p, n, true);
     const int rows = l.rows;
     const int nb = block_batches<U>(p, l);
@@ -801,8 +846,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const T *src = x + off + (int64_t)clamp_row(bi * U + u, sfl.rows) * step;
-        if constexpr (decltype(sel)::value == 0) buf0[u] = LV::load(src);
-        else buf1[u] = LV::load(src);
+        typename LV::raw_t &r = decltype(sel)::value == 0 ? buf0[u] : buf1[u];
+        if constexpr (LAST_USE) r = load_streaming<LV>(src);
+        else r = LV::load(src);
       }
     };
     auto consume = [&](auto sel, int bi) {

@@ -18,6 +18,7 @@ enum { GN_ACT_IDENTITY = 0, GN_ACT_RELU = 1, GN_ACT_SILU = 2, GN_ACT_GELU = 3, G
 
 constexpr int kBlock = 256;         // threads per workgroup (4 wavefronts)
 constexpr int kUnrollFwd = 4;       // independent row loads in flight per lane, one-input kernels
+constexpr int kUnrollStats = 8;     // ... the forward's statistics pass (4: 96 us where 8 take 90, 16: 143, see lane_stats)
 constexpr int kUnrollBwd = 2;       // ... two-input kernels (x and dy)
 constexpr int kNumCU = 256;         // MI355X
 constexpr int kTargetBlocks = 768;  // ~3 workgroups per CU, what the streaming kernels' registers allow: one resident wave
@@ -87,6 +88,26 @@ inline void set_divisors(Plan &p) {
 inline void set_gmax(Plan &p) {
   const int64_t g = ((int64_t)p.lpr * p.vec + p.D - 2) / p.D + 1;  // groups a window of lpr * vec channels can touch
   p.gmax = (int)(g < p.G ? g : p.G);
+}
+
+// How the workgroups of the forward's statistics pass share a sample's rows: in batches of `steps` rows per lane (kUnrollStats, or
+// fewer where the plan's tiles are shorter), workgroup t of p.tiles taking the batches t, t + tiles, ...
+struct Sweep {
+  int steps;
+  int batches;    // of a sample
+  int last_rows;  // rows of the sample's last batch
+  int keep_from;  // first batch of a workgroup that is to stay in the memory-side cache
+};
+// kept: the share of the tensor's bytes that cache is counted on to hold until the consumer reads them again.
+inline Sweep make_sweep(const Plan &p, double kept) {
+  Sweep s;
+  const int k = p.tile_rows / p.rpi;
+  s.steps = k < kUnrollStats ? k : kUnrollStats;
+  const int64_t rows = (int64_t)s.steps * p.rpi, batches = (p.R + rows - 1) / rows;  // (a batch is 128 elements or more, or the
+  s.batches = (int)batches;                                                          // tensor small: the count fits)
+  s.last_rows = (int)(p.R - (batches - 1) * rows);
+  s.keep_from = kept >= 1.0 ? 0 : (int)((double)((batches + p.tiles - 1) / p.tiles) * (1.0 - kept));
+  return s;
 }
 
 // Pre-additions of the forward (fused-addition variant): the tensor that is normalised is s = x + residual + channel_bias[n][c],
