@@ -727,11 +727,13 @@ __device__ __forceinline__ void recover_bwd_tail(const T *x, const T *dy, int dy
 // sums about the lane's own first row.
 //   records : {mean, M2, epoch} per (n, chunk, group, tile)
 // ---------------------------------------------------------------------------------------------
-// Occupancy the register budget is sized for.
+// Occupancy the register budget is sized for.  16 rows fit four workgroups per CU for every type because gamma / beta are
+// requested behind the statistics (with them in front, float data and float parameters took 131 - 135 registers, three workgroups):
+// bf16 (16, 320, 128, 128), float parameters, 76.5 -> 74.5 us; float32 (2, 256, 256, 256) 59.3 -> 56.9.
 // (with a residual: the tile plus a window of residual_window(nv) rows of the residual)
 constexpr int residual_window(int nv) { return nv <= 8 ? nv : 8; }
 constexpr int fused_fwd_waves(int nv, int add) {
-  return add == kAddResidual ? (nv <= 4 ? 4 : nv <= 16 ? 3 : 2) : (nv <= 8 ? 4 : nv <= 16 ? 3 : 2);
+  return add == kAddResidual ? (nv <= 4 ? 4 : nv <= 16 ? 3 : 2) : (nv <= 16 ? 4 : 2);
 }
 // TWO_LEVEL: the exchange of a launch with many row tiles per sample (two_level_exchange on the host).  A template
 // parameter, not a run-time switch: the code of the form a launch does not use would sit in the middle of the path every
@@ -786,15 +788,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
   const int64_t step = (int64_t)p.rpi * p.C;
   typename LV::raw_t buf[NV];
   trace_point(sync, 0);
-  // gamma / beta are needed only after the exchange, but they are requested first and without any branch: a load
-  // under a branch makes the compiler drain every outstanding load where the branch joins, and then the statistics
-  // below could not start on the first rows while the later ones are still arriving
-  A sa[VEC], sb[VEC];
-  {
-    const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
-    lane_params_flat<A, PT, VEC>(cvi * VEC, w, b, sync.area, sa, sb);
-  }
-  // ADD: the per-(sample, channel) addend of the lane's channels, requested with the parameters and without branches
+  // ADD: the per-(sample, channel) addend of the lane's channels, requested ahead of the rows and without branches: a load under a
+  // branch makes the compiler drain every outstanding load where the branch joins
   A tb[VEC];
   if constexpr (ADD != kAddNone) {
     const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
@@ -906,6 +901,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
     record_store(rb, record_slot(q, p.G, (int)n, l.tile, l.chunk, g), mu, s2, sync.epoch);
   });
   trace_point(sync, 2);
+  // gamma / beta are needed only after the exchange: requested here, when the moments have left their registers, their
+  // latency passes behind the exchange (no branch around the loads, see above)
+  A sa[VEC], sb[VEC];
+  {
+    const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
+    lane_params_flat<A, PT, VEC>(cvi * VEC, w, b, sync.area, sa, sb);
+  }
+  issue_order_fence();
   // Each of the two phases that follow works on its own copy of the kernel's arguments, read again where the phase
   // begins: what the phases before it loaded need not stay in scalar registers (or be spilled and restored) all the way.
   const unsigned long long epoch = sync.epoch;
