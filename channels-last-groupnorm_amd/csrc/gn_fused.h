@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
     for (int u = 0; u < NB; ++u) {
       const int64_t o = row_offset(u);
       bx[u] = LV::load(x + o);
-      bd[u] = load_dy<T, VEC, DY16>(dy, o);
+      bd[u] = load_dy<T, VEC, DY16, true>(dy, o);
     }
   } else {
     // the window of x first (row 0's arithmetic needs it), then all of dy; the rest of x follows row by row below
@@ -1180,7 +1180,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
 #pragma unroll
     for (int u = 0; u < NBX; ++u) bx[u] = LV::load(tile_row(x, t0, u));
 #pragma unroll
-    for (int u = 0; u < NBW; ++u) bd[u] = load_dy<T, VEC, DY16>(dy_row(t0, u), 0);
+    for (int u = 0; u < NBW; ++u) bd[u] = load_dy<T, VEC, DY16, true>(dy_row(t0, u), 0);
   }
   commit_chunk_stats<A>(st, l, sm_mu, sm_rs);
   __builtin_amdgcn_s_setprio(2);  // towards the exchange: ahead of wavefronts that are already past theirs
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
             issue_order_fence();  // in program order behind the row just consumed
             const int64_t o = row_offset(u + NB);
             bx[u + NB] = LV::load(x + o);
-            bd[u + NB] = load_dy<T, VEC, DY16>(dy, o);
+            bd[u + NB] = load_dy<T, VEC, DY16, true>(dy, o);
           }
         }
         if constexpr (XW > 0) {
@@ -1253,7 +1253,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
             bx[(u + NBX) % NX] = LV::load(tile_row(x, t1, u + NBX));  // (its slot held row u + NBX - NX, consumed long ago)
           }
           if constexpr (NBW < NV) {
-            if (u + NBW < NV) bd[u + NBW] = load_dy<T, VEC, DY16>(dy_row(t1, u + NBW), 0);
+            if (u + NBW < NV) bd[u + NBW] = load_dy<T, VEC, DY16, true>(dy_row(t1, u + NBW), 0);
           }
         }
       }
