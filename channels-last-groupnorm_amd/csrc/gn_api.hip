@@ -181,7 +181,7 @@ size_t bwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype) {
   for (int vec = 1; vec <= full && C % vec == 0; vec *= 2) {
     const Plan pv = make_plan(N, R, C, G, vec, esize, 2);
     need = max_size(need, bwd_workspace(pv).total);
-    if (vec == full && dtype != GN_F64) resident = resident_bwd_bytes((int64_t)pv.lpr * vec, G);
+    if (vec == full && dtype != GN_F64) resident = resident_bwd_bytes(pv);
   }
   return max_size(kWorkspaceHeader + need * acc_size(dtype), resident);
 }

@@ -4,10 +4,10 @@
 //   forward : load tile -> per-tile group moments -> publish -> wait for the tiles that share my
 //             groups -> merge -> y = act(x a + b) from registers
 //   backward: load tile (x, dy) -> per-tile channel / group sums -> publish -> wait -> merge ->
-//             dx from registers; workgroups of the first sample also finish dgamma / dbeta (tail_blocks)
+//             dx from registers; workgroups of the first sample (or the last: tail_blocks) also finish dgamma / dbeta
 //
 // A workgroup spins on data written by other workgroups of the same launch, so those must be resident together: the
-// whole launch, or in a forward larger than that each set of workgroups that exchange with each other (the host checks
+// whole launch, or in a call larger than that each set of workgroups that exchange with each other (the host checks
 // this against the occupancy the runtime reports and otherwise uses the streaming kernels).
 //
 // Exchange protocol.  The XCDs' L2 caches are not coherent with each other, and the fences that would
@@ -152,8 +152,8 @@ __device__ __forceinline__ float record_count(const Plan &p, int t, int k, int g
   return (float)(c_hi - c_lo) * (float)rows;
 }
 // Slot of a record, in 32 bits with 24-bit multiplies.  A launch that is resident as a whole has at most
-// kMaxResidentBlocksDev workgroups and G is at most 8192, so (n nchunk + k) G + g and tiles are below 2^23; for a forward
-// run set by set the host checks both (resident_fwd_records, which also bounds all records by 32 MB).
+// kMaxResidentBlocksDev workgroups and G is at most 8192, so (n nchunk + k) G + g and tiles are below 2^23; for a call
+// run set by set the host checks both (resident_fwd_records, resident_bwd_records, which also bound all records by 32 MB).
 __device__ __forceinline__ int record_slot(const PartialGeo &q, int G, int n, int t, int k, int g) {
   const int col = __mul24(n, q.nchunk) + k;
   return __mul24(__mul24(col, G) + g, q.tiles) + t;
@@ -634,18 +634,21 @@ __device__ __forceinline__ void recover_bwd_dx(const T *x, const T *dy, T *dx, i
   }
 }
 
-// Which channels a workgroup of the launch's first sample finishes dgamma / dbeta for.  The C channels are cut into
+// Which channels a workgroup of the launch's first (tail_last: last) sample finishes dgamma / dbeta for.  The C channels are cut into
 // blocks of cpp channels (cpp lanes segments of a workgroup work side by side, each with as many lanes as there are
 // (sample, tile) pairs, 64 at most); block s lies in chunk s / bpc.  Workgroup (tile, chunk) takes the blocks
 // chunk * tiles + tile, that + tiles * nchunk, ...: the blocks go to the workgroups with the LOWEST linear index, the
 // first to be dispatched and the first to be done with their own rows, whatever chunk the block belongs to -- a
 // workgroup dispatched last (on a CU that serves two others first) then has nothing left to do after its dx.
+// A launch that runs set by set (tail_last) hands them to the workgroups with the HIGHEST index instead, one block each, in
+// order: a waiting workgroup holds its place on the device, so it may only wait for workgroups that were dispatched before
+// it or share its set.  With bpc <= tiles (the host checks) workgroup W - total + s lies in chunk s / bpc or behind it.
 struct TailBlocks {
   int first, stride, total;  // this workgroup's blocks: first, first + stride, ... below total
   int bpc_log2;              // log2 of the blocks per chunk
   int chunk_channels;        // channels of a full chunk
 };
-__device__ __forceinline__ TailBlocks tail_blocks(const Plan &p, const LanePos &l, int cpp) {
+__device__ __forceinline__ TailBlocks tail_blocks(const Plan &p, const LanePos &l, int cpp, int tail_last) {
   TailBlocks t;
   t.chunk_channels = p.lpr * p.vec;  // a power of two (the host admits no other chunk width), as is cpp
   const int bpc = t.chunk_channels > cpp ? t.chunk_channels >> __builtin_ctz(cpp) : 1;
@@ -653,6 +656,10 @@ __device__ __forceinline__ TailBlocks tail_blocks(const Plan &p, const LanePos &
   t.first = l.chunk * p.tiles + l.tile;
   t.stride = p.tiles * p.nchunk;
   t.total = p.nchunk << t.bpc_log2;
+  if (tail_last) {
+    t.first -= t.stride - t.total;
+    if (t.first < 0) t.first = t.total;  // none
+  }
   return t;
 }
 // Block s: its first channel and how many of its cpp channels exist (the last chunk of a row may be narrower).
@@ -670,14 +677,14 @@ __device__ __forceinline__ void tail_block_channels(const Plan &p, const TailBlo
 template <typename T, typename PT, int ACT, bool DY16>
 __device__ __forceinline__ void recover_bwd_tail(const T *x, const T *dy, int dydtype, const void *w, const void *b, const void *mean_all,
                                                  const void *rstd_all, int sdtype, const SyncArea &sync, const Plan &p,
-                                                 RecoveryLds &r, int64_t n0, int64_t n_all, void *dw, void *db) {
+                                                 RecoveryLds &r, int64_t n0, int64_t n_all, int tail_last, void *dw, void *db) {
   const int salt = opaque_zero();
   const LanePos l = lane_pos<true>(p, blockIdx.z + salt, false, salt);
   const int cpp = kBlock / pow2_ceil_clamped((int)n_all * p.tiles, 64);  // channels per pass of the workgroup, as on the fast path
   const RecordArray rbc = channel_record_buffer(sync);
   if (threadIdx.x == 0) *sync.status = sync.epoch;
   const int pairs = (int)n_all * p.tiles;
-  const TailBlocks tb = tail_blocks(p, l, cpp);
+  const TailBlocks tb = tail_blocks(p, l, cpp, tail_last);
 #pragma nounroll
   for (int s = tb.first; s < tb.total; s += tb.stride) {
     int c0, count;
@@ -1080,6 +1087,8 @@ struct FusedBwdParams {
   int64_t n0, n_all;
   int sdtype;
   int dydtype;  // type dy is stored in: the data type, or for float data GN_F16 / GN_BF16 (kernels instantiated with DY16)
+  int tail_last;  // the last sample's workgroups finish dgamma / dbeta, not the first's (tail_blocks)
+  int pad_;
   Plan p;
 };
 // Statistics slots in LDS of a backward kernel: one per group of the chunk.  The kernels with parked rows need their LDS
@@ -1377,7 +1386,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
   // samples are complete because those launches have ended.  The first kTailFast records of a lane are requested
   // here, so that their latency passes behind the dx phase below, and checked after it.
   __builtin_amdgcn_s_setprio(0);
-  const bool tail = n == 0 && (dw || db);
+  const int tail_last = args.tail_last;
+  const bool tail = (int)blockIdx.z == (tail_last ? (int)gridDim.z - 1 : 0) && (dw || db);
   const int pairs = (int)n_all * p.tiles;
   const int TL = pow2_ceil_clamped(pairs, 64);
   const int tlg = __builtin_ctz(TL);
@@ -1390,13 +1400,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
     ks.epoch = epoch;
     recover_bwd_dx<T, PT, VEC, ACT, TWO_LEVEL, DY16>((const T *)ka.x, (const T *)ka.dy, (T *)ka.dx, ka.dydtype, ka.mean, ka.rstd,
                                                      ka.sdtype, ka.w, ka.b, ks, ka.p, recovery, sm_mu, sm_rs, sm1, sm2);
-    if (blockIdx.z == 0 && (ka.dw || ka.db))
+    if ((int)blockIdx.z == (ka.tail_last ? (int)gridDim.z - 1 : 0) && (ka.dw || ka.db))
       recover_bwd_tail<T, PT, ACT, DY16>((const T *)ka.x, (const T *)ka.dy, ka.dydtype, ka.w, ka.b, ka.mean_all, ka.rstd_all, ka.sdtype,
-                                         ks, ka.p, recovery, ka.n0, ka.n_all, ka.dw, ka.db);
+                                         ks, ka.p, recovery, ka.n0, ka.n_all, ka.tail_last, ka.dw, ka.db);
     return;
   }
   const int tslot = threadIdx.x >> tlg, tsl = threadIdx.x & (TL - 1);
-  const TailBlocks tb = tail_blocks(p, l, cpp);
+  const TailBlocks tb = tail_blocks(p, l, cpp, tail_last);
   int tail_c0 = 0, tail_count = 0;
   if (tail && tb.first < tb.total) tail_block_channels(p, tb, tb.first, cpp, tail_c0, tail_count);
   const bool tail_lane = tslot < tail_count;
@@ -1518,7 +1528,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
       SyncArea ks = ka.sync;
       ks.epoch = epoch;
       recover_bwd_tail<T, PT, ACT, DY16>((const T *)ka.x, (const T *)ka.dy, ka.dydtype, ka.w, ka.b, ka.mean_all, ka.rstd_all, ka.sdtype,
-                                         ks, ka.p, recovery, ka.n0, ka.n_all, ka.dw, ka.db);
+                                         ks, ka.p, recovery, ka.n0, ka.n_all, ka.tail_last, ka.dw, ka.db);
     }
   }
   }

@@ -166,9 +166,37 @@ inline size_t resident_crec_bytes(int64_t chunk_channels) {
   const size_t many = one * kMaxBatches < ((size_t)16 << 20) ? one * kMaxBatches : ((size_t)16 << 20);
   return align_up(one > many ? one : many, 256);
 }
-inline size_t resident_bwd_bytes(int64_t chunk_channels, int64_t G) {
-  return kWorkspaceHeader + resident_crec_bytes(chunk_channels) + align_up(resident_rec_bytes(G), 256) +
-         align_up(resident_frec_bytes(G), 256);
+// Record areas of the backward.  A backward too large to be resident as a whole runs as one launch, set by set, like the
+// forward (resident_fwd_records): the records of all sets then exist at once.
+struct BwdRecords {
+  size_t crec, rec, frec;  // bytes of the channel records, of the tile records and of the final records
+  bool rolling;            // a rolling launch is allowed
+};
+inline BwdRecords resident_bwd_records(const Plan &p) {
+  const int64_t cc = (int64_t)p.lpr * p.vec;
+  BwdRecords r = {resident_crec_bytes(cc), align_up(resident_rec_bytes(p.G), 256), align_up(resident_frec_bytes(p.G), 256), false};
+  const int64_t rows = (int64_t)kRollingRows * p.rpi;
+  const int64_t columns = p.N * p.nchunk, tiles = (p.R + rows - 1) / rows;
+  // full tiles only, and record indices within the kernels' 24-bit multiplies
+  if (p.N > 65535 || p.R < rows || columns * p.G >= (1 << 23) || p.N * tiles >= (1 << 23) || p.C >= (1 << 23)) return r;
+  const size_t rec = (size_t)16 * p.G * columns * tiles, crec = (size_t)16 * p.N * tiles * p.C;
+  if (rec > kRollingRecordBytes || crec > kRollingRecordBytes) return r;
+  r.rolling = true;
+  if (crec > r.crec) r.crec = align_up(crec, 256);
+  if (rec > r.rec) r.rec = align_up(rec, 256);
+  const size_t frec = (size_t)16 * p.G * p.N;
+  if (frec > r.frec) r.frec = align_up(frec, 256);
+  return r;
+}
+inline size_t resident_bwd_bytes(const Plan &p) {
+  const BwdRecords r = resident_bwd_records(p);
+  return kWorkspaceHeader + r.crec + r.rec + r.frec;
+}
+// Blocks of channels that the dgamma / dbeta stage of the single-launch backward cuts a chunk into (tail_blocks).
+inline int tail_blocks_per_chunk(const Plan &p, int64_t samples) {
+  const int64_t pairs = samples * p.tiles;
+  const int cpp = kBlock / pow2_at_least(pairs < 64 ? (int)pairs : 64), cc = p.lpr * p.vec;
+  return cc > cpp ? cc / cpp : 1;
 }
 // A fresh nonzero 64-bit value per call (gn_api.hip).
 unsigned long long next_epoch();
@@ -183,7 +211,7 @@ struct CapturedEpoch {
 };
 bool captured_epoch(hipStream_t stream, CapturedEpoch &out);
 // Two single-launch kernels must not share the device: each needs its workgroups resident at once, all of them or (a
-// forward run set by set) up to half of the device's worth.  Kernels
+// call run set by set) up to half of the device's worth.  Kernels
 // of one stream follow each other anyway; when a call arrives on another stream than the previous single-launch
 // call of the device, this makes the new stream wait for everything submitted so far on the previous one (an
 // event recorded there, no host synchronisation).  The object also serialises the host-side bookkeeping and the

@@ -156,15 +156,14 @@ ResidentWorkspace resident_fwd_ws(void *ws, const Plan &p, const FwdRecords &rec
   r.sync.trace_wait = trace_waits() ? 1 : 0;
   return r;
 }
-ResidentWorkspace resident_bwd_ws(void *ws, const Plan &p) {
+ResidentWorkspace resident_bwd_ws(void *ws, const Plan &p, const BwdRecords &records) {
   ResidentWorkspace r;
   char *base = (char *)ws + kWorkspaceHeader;
-  const size_t cc = (size_t)p.lpr * p.vec;
   r.sync.area = base;
-  r.sync.area_bytes = (unsigned)(resident_bwd_bytes(cc, p.G) - kWorkspaceHeader);
+  r.sync.area_bytes = (unsigned)(records.crec + records.rec + records.frec);
   r.sync.crec_first = 0;  // channel records of the whole tensor, [N][tiles][C]
-  r.sync.rec_first = (unsigned)(resident_crec_bytes(cc) / 16);
-  r.sync.frec_first = (unsigned)((resident_crec_bytes(cc) + align_up(resident_rec_bytes(p.G), 256)) / 16);
+  r.sync.rec_first = (unsigned)(records.crec / 16);
+  r.sync.frec_first = (unsigned)((records.crec + records.rec) / 16);
   r.sync.two_level = two_level_exchange(p) ? 1 : 0;
   r.sync.status = resident_status();
   r.sync.generation = nullptr;
@@ -266,29 +265,46 @@ bool try_resident_fwd(const FwdArgs &a) {
 #endif  // GN_PART_FWD || GN_PART_ADD
 
 #if GN_PART_BWD
-template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, int batches);
-template <typename PT, int ACT, int NV, int XW = 0, int XL = 0> bool try_resident_bwd_nv(const BwdArgs &a, int batches) {
+// A backward that no one launch can hold runs as a few launches over groups of samples where these fill the device well
+// (80 % of the workgroups that can be resident), else as one launch set by set, as the forward does (try_resident_fwd_nv), in the form
+// that holds the most rows per workgroup.  Full launches load, exchange and store in step and reach 5.6 TB/s; set by set, no
+// launch is left half empty and no gap lies between two.  Launches against set by set: bf16 (16, 320, 128, 128), 83 % full,
+// 89.5 / 96 us; (12, 320, 128, 128), 94 %, 80.5 / 89; float32 (2, 256, 256, 256), full, 73 / 76; but (3, 640, 200, 200), 78 %,
+// 97 / 88; (3, 640, 150, 160), 70 %, 50.9 / 49.7.  Where only the streaming kernels were left: float32 (1, 128, 512, 512) 107.9 / 73.7;
+// float16 (1, 256, 400, 500) 87 / 66; bf16 (32, 320, 128, 128) 320 / 190.
+// (set by set with 16 or 22 rows of both tensors in registers: bf16 (16, 320, 128, 128) 128 and 101 us.)
+constexpr int kRolling = 0;  // in the place of a number of launches: one launch, set by set
+template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled);
+template <typename PT, int ACT, int NV, int XW = 0, int XL = 0> bool try_resident_bwd_nv(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
   if (a.dydtype != GN_INST_DTYPE) {
-    if constexpr (kHasDy16) return try_resident_bwd_one<PT, ACT, NV, XW, XL, true>(a, batches);
+    if constexpr (kHasDy16) return try_resident_bwd_one<PT, ACT, NV, XW, XL, true>(a, records, batches, underfilled);
     else return false;
   }
-  return try_resident_bwd_one<PT, ACT, NV, XW, XL, false>(a, batches);
+  return try_resident_bwd_one<PT, ACT, NV, XW, XL, false>(a, records, batches, underfilled);
 }
-template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, int batches) {
+template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
   if (NV < resident_min_rows()) return false;
   // (kernels that park rows of x in LDS have statistics slots for chunks of at most kBlock channels)
   if (XL > 0 && a.plan.lpr * a.plan.vec > kBlock) return false;
   auto kernel_all = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, false, XW, XL, DY16>;
   auto kernel_two = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, true, XW, XL, DY16>;
   static const int slots = std::min(resident_slots(kernel_all), resident_slots(kernel_two));
-  const int64_t per = (a.plan.N + batches - 1) / batches;
+  const int64_t per = batches == kRolling ? a.plan.N : (a.plan.N + batches - 1) / batches;
   Plan p;
-  if (!resident_tiling(a.plan, per, NV, slots, p)) return false;
+  const bool rolling = batches == kRolling;
+  if (rolling && cooperative_launches()) return false;  // the runtime refuses a cooperative grid larger than the device
+  if (!resident_tiling(a.plan, per, NV, slots, p, rolling)) return false;
+  if (rolling && tail_blocks_per_chunk(p, a.plan.N) > p.tiles) return false;  // (tail_blocks relies on it)
+  const int64_t count = rolling ? 1 : (a.plan.N + per - 1) / per;  // launches
+  if (underfilled && a.plan.N * p.nchunk * p.tiles * 10 < count * slots * 8) {
+    *underfilled = true;
+    return false;
+  }
   // (the windowed form addresses the rows of a tile by 32-bit byte offsets from the tile's first row)
   if (XW > 0 && (int64_t)p.tile_rows * p.C * (int64_t)sizeof(elem_t) >= ((int64_t)1 << 31)) return false;
   // the channel records of every sample stay in the workspace until the last launch has summed them
   const size_t crec_need = (size_t)a.plan.N * p.tiles * a.plan.C * 16;
-  if (crec_need > resident_crec_bytes((int64_t)p.lpr * p.vec)) return false;
+  if (crec_need > records.crec) return false;
   if (!resident_status()) return false;
   CapturedEpoch cap;
   if (!captured_epoch(a.stream, cap)) return false;
@@ -300,7 +316,7 @@ template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resi
     Plan pb = p;
     if (a.plan.N - n0 < per) resident_tiling(a.plan, a.plan.N - n0, NV, slots, pb);  // the last, shorter group
     pb.tiles = p.tiles;  // same row tiling in every group (it depends on R and NV only)
-    ResidentWorkspace r = resident_bwd_ws(a.ws, pb);
+    ResidentWorkspace r = resident_bwd_ws(a.ws, pb, records);
     arm_generation(r, cap);
     const bool last = n0 + per >= a.plan.N;
     FusedBwdParams k = {};
@@ -320,26 +336,38 @@ template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resi
     k.n0 = n0;
     k.n_all = a.plan.N;
     k.sdtype = a.sdtype;
+    k.tail_last = rolling ? 1 : 0;
     k.p = pb;
     launch(kKindFusedBwd, r.sync.two_level ? kernel_two : kernel_all, tile_grid(pb, 0), dim3(kBlock), a.stream, k);
-    note_resident_launch(kKindFusedBwd, NV, XW, XL, r.sync.two_level, batches, pb.nblocks);
+    note_resident_launch(kKindFusedBwd, NV, XW, XL, r.sync.two_level, rolling ? 1 : batches, pb.nblocks);
   }
   return true;
 }
 template <typename PT, int ACT> bool try_resident_bwd_act(const BwdArgs &a) {
+  // the form that keeps g' and reads most of x twice
+  // (window: what the registers leave beside 32 rows of g', 16 rows for 16-bit data; parked: the rows of x that two
+  // workgroups per CU can keep in LDS beside their reduction arrays, 14 x 4 KB for 16-bit data, 16 x 4 KB for float)
+  constexpr int window = sizeof(elem_t) == 2 ? 16 : 12;
+  constexpr int parked = sizeof(elem_t) == 2 ? 14 : 16;
+  const BwdRecords records = resident_bwd_records(a.plan);
   const int most = a.plan.N < worthwhile_batches(a.plan) ? (int)a.plan.N : worthwhile_batches(a.plan);
-  for (int b = 1; b <= most; ++b) {
-    if (try_resident_bwd_nv<PT, ACT, 4>(a, b) || try_resident_bwd_nv<PT, ACT, 8>(a, b) ||
-        try_resident_bwd_nv<PT, ACT, 16>(a, b) || try_resident_bwd_nv<PT, ACT, 22>(a, b) ||
-        try_resident_bwd_nv<PT, ACT, 32>(a, b))
+  const auto launches = [&](int b, bool *underfilled) {
+    if (try_resident_bwd_nv<PT, ACT, 4>(a, records, b, underfilled) || try_resident_bwd_nv<PT, ACT, 8>(a, records, b, underfilled) ||
+        try_resident_bwd_nv<PT, ACT, 16>(a, records, b, underfilled) || try_resident_bwd_nv<PT, ACT, 22>(a, records, b, underfilled) ||
+        try_resident_bwd_nv<PT, ACT, 32>(a, records, b, underfilled))
       return true;
-    // too large for two tiles in registers: the form that keeps g' and reads most of x twice, before the tensor is cut
-    // into more launches (measured on bf16 (N, 320, 128, 128): 32.6 against 39.3 us at N = 5, 37.2 against 43.4 at N = 6)
-    // (window: what the registers leave beside 32 rows of g', 16 rows for 16-bit data; parked: the rows of x that two
-    // workgroups per CU can keep in LDS beside their reduction arrays, 14 x 4 KB for 16-bit data, 16 x 4 KB for float)
-    constexpr int window = sizeof(elem_t) == 2 ? 16 : 12;
-    constexpr int parked = sizeof(elem_t) == 2 ? 14 : 16;
-    if (try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, b) || try_resident_bwd_nv<PT, ACT, 36, 8, parked>(a, b)) return true;
+    // too large for two tiles in registers: that form, before the tensor is cut into more launches (measured on bf16
+    // (N, 320, 128, 128): 32.6 against 39.3 us at N = 5, 37.2 against 43.4 at N = 6)
+    return try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, records, b, underfilled) ||
+           try_resident_bwd_nv<PT, ACT, 36, 8, parked>(a, records, b, underfilled);
+  };
+  bool underfilled = false;
+  for (int b = 1; b <= most && !underfilled; ++b) {  // as few launches as it takes, each well filled ...
+    if (launches(b, b > 1 ? &underfilled : nullptr)) return true;
+  }
+  if (records.rolling && try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, records, kRolling, nullptr)) return true;
+  for (int b = 2; b <= most && underfilled; ++b) {  // ... or filled as they may be
+    if (launches(b, nullptr)) return true;
   }
   return false;
 }

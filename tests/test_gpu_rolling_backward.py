@@ -1,0 +1,114 @@
+"""GPU tests of backward launches with more workgroups than fit the device at once (set by set, like the forwards of
+test_gpu_rolling.py) against torch in float64: float32 parameters and float32 statistics, so that what the sums lose shows in
+dgamma / dbeta and not in how they are stored."""
+import ctypes
+
+import pytest
+import torch
+
+from gnnhwc import _cabi
+from tests.gpu_harness import cabi_bwd, cabi_fwd, err
+
+pytestmark = pytest.mark.gpu
+
+# N, R, C, G for 16-bit data (float32 takes half the channels: chunks are 128 bytes wide): one sample in sets of one chunk that
+# take half the device (two-level exchange); sets of two and of three chunks, the last tile of one row or nearly full; groups of
+# several chunks; a last chunk of 32 bytes; one group, i.e. a sample per set
+SHAPES = [(1, 262144, 256, 32), (7, 16385, 640, 32), (3, 40000, 640, 8), (2, 24575, 1088, 4), (33, 16384, 272, 17), (6, 32768, 256, 1)]
+DTYPES = [torch.bfloat16, torch.float16, torch.float32]
+
+
+def _case(N, R, C, G, dtype, device):
+    C = C // 2 if dtype == torch.float32 else C
+    gen = torch.Generator(device=device).manual_seed(N + R + C)
+    x = torch.empty((N, R, C), device=device, dtype=dtype).normal_(generator=gen).mul_(1.5).add_(
+        torch.randn((C,), device=device, generator=gen).to(dtype))
+    dy = torch.empty((N, R, C), device=device, dtype=dtype).normal_(generator=gen)
+    w, b = torch.rand((C,), device=device, generator=gen) + 0.5, 0.1 * torch.randn((C,), device=device, generator=gen)
+    _, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
+    return x, dy, w, b, mean, rstd
+
+
+def _assert_set_by_set():
+    out = (ctypes.c_int64 * 7)()
+    _cabi.check(_cabi.lib.gnnhwc_debug_last_launch(out), "gnnhwc_debug_last_launch")
+    assert out[0] >= 0 and _cabi.kernel_kind_names()[out[0]] == "fused_bwd", _cabi.last_launch()
+    # one launch of more workgroups than two of these fit a CU
+    assert out[4] == 1 and out[2] > 0 and out[5] > 512, _cabi.last_launch()
+
+
+def _against_float64(x, dy, w, b, G, dx, dw, db, eps=1e-5):
+    """dx passes through two roundings to the data type, of g' and of itself, each of half a spacing at most: relative 2-norm
+    below one spacing of 1 (float32: the sums' own rounding, 1e-6).  dgamma, dbeta: the float32 bar, 1e-5 of the largest."""
+    N, R, C = x.shape
+    W, B = w.double(), b.double()
+    DW, DB, off, size = torch.zeros_like(W), torch.zeros_like(W), 0.0, 0.0
+    for n in range(N):
+        t = x[n].double().view(R, G, C // G)
+        mu = t.mean((0, 2), keepdim=True)
+        rs = ((t - mu).square().mean((0, 2), keepdim=True) + eps).rsqrt()
+        xh = ((t - mu) * rs).view(R, C)
+        z = xh * W + B
+        s = torch.sigmoid(z)
+        g = dy[n].double() * s * (1 + z * (1 - s))
+        DW += (g * xh).sum(0)
+        DB += g.sum(0)
+        gw, xg = (g * W).view(R, G, -1), xh.view(R, G, -1)
+        want = (rs * (gw - gw.mean((0, 2), keepdim=True) - xg * (gw * xg).mean((0, 2), keepdim=True))).reshape(R, C)
+        off += (dx[n].double() - want).square().sum().item()
+        size += want.square().sum().item()
+    bar = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 1e-6}[x.dtype]
+    assert (off / size) ** 0.5 <= bar
+    assert err(dw, DW) <= 1e-5 and err(db, DB) <= 1e-5
+
+
+@pytest.mark.parametrize("N,R,C,G", SHAPES)
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_against_float64(N, R, C, G, dtype, device):
+    print("rolling backward", N, R, C, G, dtype, flush=True)
+    x, dy, w, b, mean, rstd = _case(N, R, C, G, dtype, device)
+    dx, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, G, 2)
+    _assert_set_by_set()
+    _against_float64(x, dy, w, b, G, dx, dw, db)
+    again = cabi_bwd(dy, x, w, b, mean, rstd, G, 2)
+    for s, t in zip((dx, dw, db), again):
+        assert torch.equal(s, t)
+    inplace = cabi_bwd(dy, x, w, b, mean, rstd, G, 2, dx=dy)
+    for s, t in zip((dx, dw, db), inplace):
+        assert torch.equal(s, t)
+
+
+@pytest.mark.parametrize("N,R,C,G", [(7, 16385, 640, 32), (1, 262144, 256, 32)])
+@pytest.mark.parametrize("spins", [-2, 0, 2])
+def test_expired_waits_are_recovered(spins, N, R, C, G, device):
+    x, dy, w, b, mean, rstd = _case(N, R, C, G, torch.bfloat16, device)
+    _cabi.lib.gnnhwc_resident_status()
+    before = _cabi.lib.gnnhwc_debug_set_spin_limit(spins)
+    try:
+        dx, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, G, 2)
+        torch.cuda.synchronize()
+    finally:
+        _cabi.lib.gnnhwc_debug_set_spin_limit(before)
+    _assert_set_by_set()
+    assert _cabi.lib.gnnhwc_resident_status() == 1 or spins != -2
+    _against_float64(x, dy, w, b, G, dx, dw, db)
+
+
+def test_replayed_graph(device):
+    x, dy, w, b, mean, rstd = _case(7, 16385, 640, 32, torch.bfloat16, device)
+    ws = torch.empty((_cabi.lib.gnnhwc_bwd_workspace_bytes(7, 16385, 640, 32, 3),), dtype=torch.uint8, device=device)
+    dx = torch.empty_like(x)
+    cabi_bwd(dy, x, w, b, mean, rstd, 32, 2, dx=dx, ws=ws)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, 32, 2, dx=dx, ws=ws)
+        _assert_set_by_set()
+    for i in range(3):
+        dy.add_(i)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = cabi_bwd(dy, x, w, b, mean, rstd, 32, 2)
+        torch.cuda.synchronize()
+        for s, t in zip((dx, dw, db), want):
+            assert torch.equal(s, t)
