@@ -138,8 +138,8 @@ template <typename PT, typename A> __device__ __forceinline__ void store_param(v
 // (16, 320, 128, 128) forward + backward 169 -> 163 us, float32 (4, 256, 128, 128) 76 -> 66.  x itself is read plainly: with the
 // hint in the forward, the backward lost more than the forward gained (float32 (2, 256, 256, 256) 57.6 + 75.0 -> 54.2 + 89.3).
 template <bool LAST_USE, typename V> __device__ __forceinline__ V load_hinted(const V *p) {
-  if constexpr (LAST_USE) return __builtin_nontemporal_load(p);
-  else return *p;
+  if constexpr (LAST_USE) return __builtin_nontemporal_load((const global_mem<V> *)p);
+  else return load_global<V>(p);
 }
 template <typename T, int VEC, bool DY16, bool LAST_USE = false>
 __device__ __forceinline__ typename LaneVec<T, VEC>::raw_t load_dy(const T *dy, int64_t e) {
