@@ -1240,6 +1240,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
           vd[j] = g;
         }
         bd[u] = LV::pack(vd);
+        if constexpr (XW == 0 && NV > 16 && std::is_same<T, f16_t>::value) {
+          // row by row here too (see the windowed form below): without it the conversions of float16, which the scheduler
+          // takes further ahead than bfloat16's shifts, spilled up to 66 registers to memory.  float16 (2, 128, 400, 400)
+          // gelu_tanh, two launches of 22 rows: 87 -> 59 us.  (bfloat16 and float do not spill, and lose 6 - 10 % by it.)
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) { pin(s1[j]); pin(s2[j]); }
+          pin(bd[u]);
+        }
         if constexpr (XW == 0 && NB < NV) {
           if (u + NB < NV) {
             issue_order_fence();  // in program order behind the row just consumed
