@@ -55,7 +55,9 @@ const char *dtype_name(int dtype) {
 // whole 128-byte lines, divides the row evenly and leaves no lane idle is preferred.
 // Rows per tile: chosen so that a large tensor yields about `target` workgroups and a small one still
 // yields as many workgroups as it has lane rows, down to one row per lane.
-Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int esize, int streams) {
+//
+// cut_plan: without the divisors (set_divisors), which only kernels and their launches need; for sizing a workspace.
+Plan cut_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int esize, int streams) {
   static const int forced_lpr = env_int("GNNHWC_LPR", 0);
   static const int forced_fwd_steps = env_int("GNNHWC_FWD_STEPS", 0);
   static const int forced_bwd_steps = env_int("GNNHWC_BWD_STEPS", 0);
@@ -115,8 +117,12 @@ Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int esize, i
   p.tile_rows = (int)(k * p.rpi);
   p.tiles = (int)((R + p.tile_rows - 1) / p.tile_rows);
   p.nblocks = N * p.tiles * p.nchunk;
-  set_divisors(p);
   set_gmax(p);
+  return p;
+}
+Plan make_plan(int64_t N, int64_t R, int64_t C, int64_t G, int vec, int esize, int streams) {
+  Plan p = cut_plan(N, R, C, G, vec, esize, streams);
+  set_divisors(p);
   static const int debug = env_int("GNNHWC_DEBUG_PLAN", 0);
   if (debug)
     fprintf(stderr, "[gnnhwc] plan(%s) N=%lld R=%lld C=%lld G=%d D=%d vec=%d cv=%d lpr=%d nchunk=%d rpi=%d tile_rows=%d tiles=%d nblocks=%lld\n",
@@ -169,7 +175,7 @@ size_t fwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, bool 
   const int esize = elem_size(dtype), full = 16 / esize;
   size_t need = 0, resident = 0;
   for (int vec = 1; vec <= full && C % vec == 0; vec *= 2) {
-    const Plan pv = make_plan(N, R, C, G, vec, esize, 1);
+    const Plan pv = cut_plan(N, R, C, G, vec, esize, 1);
     need = max_size(need, fwd_workspace(pv).total);
     if (vec == full && dtype != GN_F64 && !streaming_only) resident = resident_fwd_bytes(pv);
   }
@@ -179,7 +185,7 @@ size_t bwd_ws_bytes(int64_t N, int64_t R, int64_t C, int64_t G, int dtype) {
   const int esize = elem_size(dtype), full = 16 / esize;
   size_t need = 0, resident = 0;
   for (int vec = 1; vec <= full && C % vec == 0; vec *= 2) {
-    const Plan pv = make_plan(N, R, C, G, vec, esize, 2);
+    const Plan pv = cut_plan(N, R, C, G, vec, esize, 2);
     need = max_size(need, bwd_workspace(pv).total);
     if (vec == full && dtype != GN_F64) resident = resident_bwd_bytes(pv);
   }

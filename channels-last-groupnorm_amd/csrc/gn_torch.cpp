@@ -140,17 +140,21 @@ struct Added {  // pre-additions of the forward (group_norm_nhwc)
   Tensor sum;  // where x + residual + channel_bias goes (undefined: nowhere)
   bool any = false;
 };
-// One forward call on checked arguments; stats comes back as (2, N, G): mean, 1 / sqrt(var + eps).
+// One forward call on checked arguments; stats (null: nobody will ask for them) comes back as (2, N, G): mean, 1 / sqrt(var + eps).
 Tensor run_forward(const Tensor &x, const optional<Tensor> &weight, const optional<Tensor> &bias, int64_t G, double eps, int act,
-                   bool first, at::ScalarType out, const Added &add, Tensor &stats) {
+                   bool first, at::ScalarType out, const Added &add, Tensor *stats) {
   const c10::DeviceGuard guard(x.device());
   const at::AutoDispatchBelowADInplaceOrView below;
   const Shape s = shape_of(x);
   const int dt = code_of(x.scalar_type()), pdt = ptr(weight) ? code_of(weight->scalar_type()) : dt;
   const at::ScalarType st = stats_type(x.scalar_type());
   Tensor y = first ? at::empty(x.sizes(), x.options()) : empty_channels_last(x, out);
-  stats = at::empty({2, s.N, G}, x.options().dtype(st));
-  char *mean = (char *)stats.data_ptr(), *rstd = mean + s.N * G * stats.element_size();
+  char *mean = nullptr, *rstd = nullptr;
+  if (stats) {
+    *stats = at::empty({2, s.N, G}, x.options().dtype(st));
+    mean = (char *)stats->data_ptr();
+    rstd = mean + s.N * G * stats->element_size();
+  }
   const size_t bytes = first ? abi.nchw_workspace_bytes(s.N, s.C, s.R, G, dt, 0) : abi.fwd_workspace_bytes(s.N, s.R, s.C, G, dt);
   const char *what = first ? "gnop::fwd_nchw" : add.any ? "gnop::fwd_add" : out != x.scalar_type() ? "gnop::fwd_cast" : "gnop::fwd";
   const OperatorRange range(what);
@@ -228,7 +232,7 @@ struct GroupNormNode : public torch::autograd::Function<GroupNormNode> {
                         const optional<Tensor> &bias, int64_t G, double eps, int64_t act, bool first, int64_t out,
                         bool functional) {
     Tensor stats;
-    Tensor y = run_forward(x, weight, bias, G, eps, (int)act, first, (at::ScalarType)out, Added{}, stats);
+    Tensor y = run_forward(x, weight, bias, G, eps, (int)act, first, (at::ScalarType)out, Added{}, &stats);
     ctx->save_for_backward({x, weight.value_or(Tensor()), bias.value_or(Tensor()), stats});
     ctx->saved_data["call"] = std::vector<int64_t>{G, act, first ? 1 : 0, functional ? 1 : 0};
     // a view, as the Python function returns: an in-place change of y is refused the same way
@@ -400,8 +404,7 @@ PyObject *group_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         const at::AutoDispatchBelowADInplaceOrView below;
         add.sum = empty_channels_last(x, x.scalar_type());
       }
-      Tensor stats;
-      y = run_forward(x, weight, bias, G, eps, (int)act, first, out, add, stats);
+      y = run_forward(x, weight, bias, G, eps, (int)act, first, out, add, nullptr);
     }
   }
   if (!want_sum) return THPVariable_Wrap(y);

@@ -434,3 +434,20 @@ def test_gradients_with_a_tangent(affine, out, device):
         got = [fwAD.unpack_dual(t).primal.clone() for t in got]
     for s, t in zip(got, want):
         assert torch.equal(s, t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first,dtype,out", [(False, torch.bfloat16, None), (False, torch.float32, torch.float16),
+                                             (False, torch.float64, None), (True, torch.float16, None), (True, torch.float32, None)])
+@pytest.mark.parametrize("shape,G", [((2, 64, 8, 8), 8), ((3, 35, 9, 13), 5), ((1, 128, 600, 500), 32)])
+def test_result_without_a_graph_equals_the_one_with(first, dtype, out, shape, G, device):
+    """Without a graph the kernels are given nowhere to leave the statistics."""
+    torch.manual_seed(2)
+    x = torch.randn(shape, device=device).to(dtype)
+    x = x if first else _channels_last(x)
+    m = GN_NHWC(G, shape[1], activation="gelu", out_dtype=out).to(device).to(dtype)
+    with torch.no_grad():
+        y = m(x)
+    want = m(x.clone().requires_grad_())
+    assert want.grad_fn is not None and y.grad_fn is None
+    _same((y,), (want.detach(),))
