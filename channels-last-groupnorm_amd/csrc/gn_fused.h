@@ -734,14 +734,15 @@ __device__ __forceinline__ void recover_bwd_tail(const T *x, const T *dy, int dy
 // sums about the lane's own first row.
 //   records : {mean, M2, epoch} per (n, chunk, group, tile)
 // ---------------------------------------------------------------------------------------------
-// Occupancy the register budget is sized for.  16 rows fit four workgroups per CU for every type because gamma / beta are
-// requested behind the statistics (with them in front, float data and float parameters took 131 - 135 registers, three workgroups):
+// Occupancy the register budget is sized for.  16 rows fit four workgroups per CU for every type because float gamma / beta are
+// requested behind the statistics (late_params; with them in front, those kernels took 131 - 135 registers, three workgroups):
 // bf16 (16, 320, 128, 128), float parameters, 76.5 -> 74.5 us; float32 (2, 256, 256, 256) 59.3 -> 56.9.
 // (with a residual: the tile plus a window of residual_window(nv) rows of the residual)
 constexpr int residual_window(int nv) { return nv <= 8 ? nv : 8; }
 constexpr int fused_fwd_waves(int nv, int add) {
   return add == kAddResidual ? (nv <= 4 ? 4 : nv <= 16 ? 3 : 2) : (nv <= 16 ? 4 : 2);
 }
+constexpr bool late_params(int nv, int param_bytes) { return nv >= 16 && param_bytes == 4; }
 // TWO_LEVEL: the exchange of a launch with many row tiles per sample (two_level_exchange on the host).  A template
 // parameter, not a run-time switch: the code of the form a launch does not use would sit in the middle of the path every
 // workgroup executes once, and these kernels are sensitive to their own size.
@@ -795,8 +796,19 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
   const int64_t step = (int64_t)p.rpi * p.C;
   typename LV::raw_t buf[NV];
   trace_point(sync, 0);
-  // ADD: the per-(sample, channel) addend of the lane's channels, requested ahead of the rows and without branches: a load under a
-  // branch makes the compiler drain every outstanding load where the branch joins
+  // gamma / beta are needed only after the exchange, but they are requested first and without any branch: a load
+  // under a branch makes the compiler drain every outstanding load where the branch joins, and then the statistics
+  // below could not start on the first rows while the later ones are still arriving.  Where they would cost a fourth
+  // workgroup per CU (see fused_fwd_waves) they are requested behind the publication of the tile's moments instead, which
+  // takes a kernel that is not short of registers 0.2 - 0.6 us longer.
+  constexpr bool kLateParams = late_params(NV, (int)sizeof(PT));
+  A sa[VEC], sb[VEC];
+  auto request_params = [&]() {
+    const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
+    lane_params_flat<A, PT, VEC>(cvi * VEC, w, b, sync.area, sa, sb);
+  };
+  if constexpr (!kLateParams) request_params();
+  // ADD: the per-(sample, channel) addend of the lane's channels, requested with the parameters and without branches
   A tb[VEC];
   if constexpr (ADD != kAddNone) {
     const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
@@ -908,14 +920,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
     record_store(rb, record_slot(q, p.G, (int)n, l.tile, l.chunk, g), mu, s2, sync.epoch);
   });
   trace_point(sync, 2);
-  // gamma / beta are needed only after the exchange: requested here, when the moments have left their registers, their
-  // latency passes behind the exchange (no branch around the loads, see above)
-  A sa[VEC], sb[VEC];
-  {
-    const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
-    lane_params_flat<A, PT, VEC>(cvi * VEC, w, b, sync.area, sa, sb);
+  if constexpr (kLateParams) {
+    request_params();
+    issue_order_fence();
   }
-  issue_order_fence();
   // Each of the two phases that follow works on its own copy of the kernel's arguments, read again where the phase
   // begins: what the phases before it loaded need not stay in scalar registers (or be spilled and restored) all the way.
   const unsigned long long epoch = sync.epoch;
@@ -1091,6 +1099,11 @@ struct FusedBwdParams {
   int pad_;
   Plan p;
 };
+// dy, which is read once, is read with the non-temporal hint (load_dy) where more than 16 rows per lane hold the tensor, that is
+// above 32 MB of it: what a call of that size touches does not stay in the caches as a whole, and the hint leaves more of it to x.
+// Smaller ones are found there, and lines read with the hint are not, the next time: bf16 (1, 640, 128, 128), the same tensors
+// again and again, 15.2 us without it, 16.1 with.
+constexpr bool dy_streams(int nv) { return nv > 16; }
 // Statistics slots in LDS of a backward kernel: one per group of the chunk.  The kernels with parked rows need their LDS
 // for those and serve chunks of at most kBlock channels (the host checks), hence at most kBlock groups.
 constexpr int fused_bwd_stat_slots(int vec, int xl) { return xl > 0 ? kBlock : kBlock * vec; }
@@ -1131,6 +1144,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
   constexpr int NX = XW > 0 ? XW : NV;  // rows of x held at a time; row u lives in bx[u % NX]
   static_assert(XW >= 0 && XW <= NV, "window within the tile");
   typename LV::raw_t bx[NX], bd[NV];
+  constexpr bool kDyStreams = dy_streams(NV);
   auto row_offset = [&](int u) { return off + (int64_t)clamp_row(u, sfl.rows) * step; };
   // XW > 0: rows are requested all through the kernel, so their addresses must be cheap to form again: the tile's
   // (uniform) base plus a 32-bit byte offset per lane and row (the host admits only tiles below 2 GiB)
@@ -1181,7 +1195,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
     for (int u = 0; u < NB; ++u) {
       const int64_t o = row_offset(u);
       bx[u] = LV::load(x + o);
-      bd[u] = load_dy<T, VEC, DY16, true>(dy, o);
+      bd[u] = load_dy<T, VEC, DY16, kDyStreams>(dy, o);
     }
   } else {
     // the window of x first (row 0's arithmetic needs it), then all of dy; the rest of x follows row by row below
@@ -1189,7 +1203,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
 #pragma unroll
     for (int u = 0; u < NBX; ++u) bx[u] = LV::load(tile_row(x, t0, u));
 #pragma unroll
-    for (int u = 0; u < NBW; ++u) bd[u] = load_dy<T, VEC, DY16, true>(dy_row(t0, u), 0);
+    for (int u = 0; u < NBW; ++u) bd[u] = load_dy<T, VEC, DY16, kDyStreams>(dy_row(t0, u), 0);
   }
   commit_chunk_stats<A>(st, l, sm_mu, sm_rs);
   __builtin_amdgcn_s_setprio(2);  // towards the exchange: ahead of wavefronts that are already past theirs
@@ -1253,7 +1267,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
             issue_order_fence();  // in program order behind the row just consumed
             const int64_t o = row_offset(u + NB);
             bx[u + NB] = LV::load(x + o);
-            bd[u + NB] = load_dy<T, VEC, DY16, true>(dy, o);
+            bd[u + NB] = load_dy<T, VEC, DY16, kDyStreams>(dy, o);
           }
         }
         if constexpr (XW > 0) {
@@ -1270,7 +1284,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
             bx[(u + NBX) % NX] = LV::load(tile_row(x, t1, u + NBX));  // (its slot held row u + NBX - NX, consumed long ago)
           }
           if constexpr (NBW < NV) {
-            if (u + NBW < NV) bd[u + NBW] = load_dy<T, VEC, DY16, true>(dy_row(t1, u + NBW), 0);
+            if (u + NBW < NV) bd[u + NBW] = load_dy<T, VEC, DY16, kDyStreams>(dy_row(t1, u + NBW), 0);
           }
         }
       }

@@ -133,7 +133,7 @@ template <typename PT, typename A> __device__ __forceinline__ void store_param(v
 // The incoming gradient of a backward on float data may be stored in a 16-bit type (DY16; dydtype GN_F16 or GN_BF16: the
 // layer that produced it ran in half precision).  A lane vector of it is 8 bytes, carried in the first half of the raw
 // register vector until it is unpacked; widening happens in registers, no separate pass over dy.
-// LAST_USE: nobody reads this element again (the single-launch kernels, which read dy once).  Read with the non-temporal hint
+// LAST_USE: nobody reads this element again (single-launch kernels of large tensors: dy_streams, gn_fused.h).  Read with the non-temporal hint
 // it does not push out of the memory-side cache what others are about to read, the x of this call among it: bf16
 // (16, 320, 128, 128) forward + backward 169 -> 163 us, float32 (4, 256, 128, 128) 76 -> 66.  x itself is read plainly: with the
 // hint in the forward, the backward lost more than the forward gained (float32 (2, 256, 256, 256) 57.6 + 75.0 -> 54.2 + 89.3).
