@@ -226,10 +226,11 @@ int gnnhwc_bwd_nchw(const void *dy, const void *x, const void *weight, const voi
 /*
  * Kernel selection (no counterpart in the reference).  By default a problem whose tensors fit in the
  * register files of one launch is run by the single-launch kernels (x and dy are read from memory once;
- * workgroups exchange partial results while resident), and so is a larger forward as long as the workgroups
+ * workgroups exchange partial results while resident), and so is a larger forward or backward as long as the workgroups
  * that exchange with each other -- those on one 128-byte chunk of a sample's rows, or on the few chunks that a
  * group spans -- fit half of the device (up to 262144 rows where groups lie inside chunks) and
- * their records 32 MB; anything else is run by the multi-launch streaming kernels.  A single-launch kernel is
+ * their records 32 MB (a larger backward may also run as up to four such launches over groups of samples, where these fill
+ * the device well); anything else is run by the multi-launch streaming kernels.  A single-launch kernel is
  * fastest with the device to itself: calls of one process on different streams are ordered by the library (a call on another stream than the previous single-launch
  * call of the device first makes its stream wait, on the device, for what has been submitted to that
  * previous stream).  Where the device is shared all the same (launches recorded into graphs that are replayed
