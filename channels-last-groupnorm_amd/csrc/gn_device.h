@@ -70,6 +70,13 @@ __device__ __forceinline__ void issue_order_fence() { asm volatile("" ::: "memor
 // kept alive for the next, which doubles or triples the registers a 16-bit tile needs.
 template <typename R> __device__ __forceinline__ void pin(R &r) { asm volatile("" : "+v"(r)); }
 
+// A zero the compiler cannot see through (see lane_pos).
+__device__ __forceinline__ int opaque_zero() {
+  int z = 0;
+  asm volatile("" : "+s"(z));
+  return z;
+}
+
 template <> struct LaneVec<float, 4> {
   typedef f32x4 raw_t;
   static __device__ __forceinline__ raw_t load(const float *p) { return load_global<raw_t>(p); }

@@ -318,12 +318,6 @@ template <typename P> __device__ __forceinline__ P reread_kernel_args() {
   for (unsigned i = 0; i < sizeof(P) / 4; ++i) dst[i] = src[i];
   return a;
 }
-// A zero the compiler cannot see through (see lane_pos).
-__device__ __forceinline__ int opaque_zero() {
-  int z = 0;
-  asm volatile("" : "+s"(z));
-  return z;
-}
 __device__ __forceinline__ float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }

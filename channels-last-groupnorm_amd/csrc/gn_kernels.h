@@ -304,18 +304,21 @@ __device__ __forceinline__ void group_span(const Plan &p, const LanePos &l, int 
 // (Chan's update in pivot form; WelfordOps::reduce, src/gnnhwc/csrc/Welford.h:30-42, divides once per element): three
 // operations per element and four per channel and batch.
 // ---------------------------------------------------------------------------------------------
-template <typename T, int VEC, int U>
-__device__ __forceinline__ void fold_batch(const typename LaneVec<T, VEC>::raw_t (&raw)[U], int m, acc_t<T> &cnt,
-                                           acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
+// Row by row, each row's sums brought up to date before the next is unpacked (left alone, the scheduler unpacks a whole batch
+// ahead, which takes more registers than the rows); `refill(u)` may reuse the row's register.  The first batch's first row
+// has to be in `mean` already (begin_stats).
+template <typename T, int VEC, int U, typename REFILL>
+__device__ __forceinline__ void fold_batch(typename LaneVec<T, VEC>::raw_t (&raw)[U], int m, acc_t<T> &cnt, acc_t<T> (&mean)[VEC],
+                                           acc_t<T> (&m2)[VEC], REFILL &&refill) {
   using A = acc_t<T>;
   A s1[VEC], s2[VEC];
-  if (cnt == (A)0) LaneVec<T, VEC>::unpack(raw[0], mean);
 #pragma unroll
   for (int j = 0; j < VEC; ++j) { s1[j] = (A)0; s2[j] = (A)0; }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (u < m) {  // (m is U except in a lane's last batch)
       A v[VEC];
+      pin(raw[u]);
       LaneVec<T, VEC>::unpack(raw[u], v);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
@@ -323,7 +326,10 @@ __device__ __forceinline__ void fold_batch(const typename LaneVec<T, VEC>::raw_t
         s1[j] += d;
         s2[j] += d * d;
       }
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) { pin(s1[j]); pin(s2[j]); }
     }
+    refill(u);
   }
   cnt += (A)m;
   const A inv = fast_rcp(cnt);
@@ -364,10 +370,13 @@ __device__ __forceinline__ SweptRows sweep_rows(const Plan &p, const Sweep &sw, 
 // Bound: memory.  A tensor that exceeds that cache arrives at 6.0 TB/s by plain loads and at 6.9 by non-temporal ones, and
 // what non-temporal loads have read is not found there by a later pass (measured on a 537 MB read alone: 88 against 78 us; a
 // copy behind it, from the far end: 160 against 167).  float16 (1, 256, 1024, 1024): 103 us with tiles of neighbouring rows, plain
-// loads and the statistics in two passes over each batch (7.5 vector operations per element); 90 in this form.
+// loads and the statistics in two passes over each batch (7.5 vector operations per element); 86 in this form.
+// Small samples are bound by the chain from the first instruction to the last of a workgroup, and by how many are resident:
+// bf16 (70000, 64, 8, 8) 217 us in the former, 186 in this form with 95 registers.  (With two buffers of eight rows and the
+// scheduler left to itself, 230 registers and every row's offset formed ahead: 508; float64 (2, 320, 64, 64) 7.7, 7.3 and 12.)
 template <typename T, int VEC, int U>
 __device__ __forceinline__ void lane_stats(const T *__restrict__ x, const Plan &p, const LanePos &l, const Sweep &sw,
-                                           const SweptRows &s, acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
+                                           const SweptRows &s, int salt, acc_t<T> (&mean)[VEC], acc_t<T> (&m2)[VEC]) {
   using A = acc_t<T>;
   using LV = LaneVec<T, VEC>;
 #pragma unroll
@@ -375,45 +384,63 @@ __device__ __forceinline__ void lane_stats(const T *__restrict__ x, const Plan &
   A cnt = (A)0;
   const int rows = l.rows;
   if (rows == 0) return;
-  const T *base = x + ((l.n * p.R + l.row0 + l.ty) * p.C + (int64_t)l.cvi * VEC);
-  const int64_t step = (int64_t)p.rpi * p.C, sweep = (int64_t)p.tiles * sw.steps * step;
+  const T *src = x + ((l.n * p.R + l.row0 + l.ty) * p.C + (int64_t)l.cvi * VEC);  // the next row to request
+  const int64_t step = (int64_t)(p.rpi + salt) * p.C, to_next_batch = (int64_t)(p.tiles - 1) * sw.steps * step;
+  // (the address steps from row to row and the compiler must not see through it: the offsets of all rows of all loops,
+  // formed ahead in every workgroup, took 450 instructions before the first load)
+  auto advance = [&](int64_t elements) {
+    src += elements;
+    pin(src);
+  };
   // batches with all U rows for every lane: [0, keep) non-temporal, [keep, full) plain; no choice is left to the inside of
   // either loop, where a branch around the loads would make the waits behind it drain the queue
   const int full = sw.steps == U ? (s.last ? s.nb - 1 : s.nb) : 0;
   // (narrow lane vectors do without the first loop: tensors of that size and such a channel count are not worth its code)
   constexpr bool kSweepCold = VEC == vec_of<T>::value;
   const int keep = sw.keep_from < full ? sw.keep_from : full;
+  // one buffer of U rows, each refilled from the next batch as soon as it is folded: U loads in flight all the way
   auto sweep_batches = [&](auto streaming, int first, int end) {
     if (first >= end) return;
-    typename LV::raw_t buf0[U], buf1[U];
-    auto issue = [&](auto sel, int b) {
-      const T *src = base + (first + b) * sweep;
+    typename LV::raw_t buf[U];
+    auto request = [&](int u) {
+      if constexpr (decltype(streaming)::value) buf[u] = load_streaming<LV>(src);
+      else buf[u] = LV::load(src);
+      advance(step);
+    };
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        typename LV::raw_t &r = decltype(sel)::value == 0 ? buf0[u] : buf1[u];
-        if constexpr (decltype(streaming)::value) r = load_streaming<LV>(src + u * step);
-        else r = LV::load(src + u * step);
-      }
-      issue_order_fence();  // ahead of the rows consumed meanwhile
-    };
-    auto consume = [&](auto sel, int) {
-      if constexpr (decltype(sel)::value == 0) fold_batch<T, VEC, U>(buf0, U, cnt, mean, m2);
-      else fold_batch<T, VEC, U>(buf1, U, cnt, mean, m2);
-    };
-    issue(std::integral_constant<int, 0>{}, 0);
-    double_buffered(end - first, issue, consume);
+    for (int u = 0; u < U; ++u) request(u);
+    advance(to_next_batch);
+    issue_order_fence();
+    if (cnt == (A)0) LV::unpack(buf[0], mean);
+    for (int b = first + 1; b < end; ++b) {
+      fold_batch<T, VEC, U>(buf, U, cnt, mean, m2, [&](int u) {
+        issue_order_fence();
+        request(u);
+      });
+      advance(to_next_batch);
+    }
+    fold_batch<T, VEC, U>(buf, U, cnt, mean, m2, [](int) {});
   };
   if constexpr (kSweepCold) sweep_batches(std::true_type{}, 0, keep);
   sweep_batches(std::false_type{}, kSweepCold ? keep : 0, full);
-  // the rows of the one batch left: the sample's last, or that of a tile shorter than U rows per lane
-  constexpr int V = U < kUnrollFwd ? U : kUnrollFwd;
-  const T *src = base + full * sweep;
-  for (int m = rows - full * sw.steps; m > 0; m -= V, src += V * step) {
+  // the rows of the one batch left: the sample's last, or that of a tile shorter than U rows per lane; all requested at once
+  // (a lane without another row reads its last one again)
+  auto short_batch = [&](auto most, int m) {
+    constexpr int V = decltype(most)::value;
     typename LV::raw_t buf[V];
 #pragma unroll
-    for (int u = 0; u < V; ++u) buf[u] = LV::load(src + clamp_row(u, m) * step);
-    fold_batch<T, VEC, V>(buf, m < V ? m : V, cnt, mean, m2);
-  }
+    for (int u = 0; u < V; ++u) {
+      buf[u] = LV::load(src);
+      advance(u + 1 < m ? step : 0);
+    }
+    issue_order_fence();
+    if (cnt == (A)0) LV::unpack(buf[0], mean);
+    fold_batch<T, VEC, V>(buf, m, cnt, mean, m2, [](int) {});
+  };
+  const int left = rows - full * sw.steps;
+  if (left <= 0) return;
+  if (l.rows_base + (l.rows_rem > 0 ? 1 : 0) - full * sw.steps <= kUnrollFwd) short_batch(std::integral_constant<int, kUnrollFwd>{}, left);
+  else short_batch(std::integral_constant<int, U>{}, left);
 }
 
 // Sum of col[0], col[stride], ... (n entries) with eight reads in flight: the loop is latency bound otherwise.
@@ -603,7 +630,7 @@ __global__ __launch_bounds__(kBlock) void add_flat_kernel(const T *__restrict__ 
 //   part : 3 planes [N][nchunk][G][tiles]; only the groups a chunk intersects are written.
 // ---------------------------------------------------------------------------------------------
 template <typename T, int VEC>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void stats_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void stats_kernel(
     const T *__restrict__ x, acc_t<T> *__restrict__ part, Plan p, Sweep sw) {
   using A = acc_t<T>;
   __shared__ A sm_mean[kBlock * VEC];
@@ -611,10 +638,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
   const PartialGeo q = producer_geo(p);
   const int64_t plane = group_plane(q, p.G, p.N);
   for (int64_t n = blockIdx.z; n < p.N; n += gridDim.z) {
-    LanePos l = lane_pos(p, n, false);
+    const int salt = opaque_zero();  // (what a second sample would need again is not formed ahead for it)
+    LanePos l = lane_pos(p, n, false, salt);
     const SweptRows sweep = sweep_rows(p, sw, l);
     A mean[VEC], m2[VEC];
-    lane_stats<T, VEC, kUnrollStats>(x, p, l, sw, sweep, mean, m2);
+    lane_stats<T, VEC, kUnrollStats>(x, p, l, sw, sweep, salt, mean, m2);
     block_group_moments<A, VEC>(p, l, mean, m2, sm_mean, sm_m2, [&](int g, A cnt, A mu, A s2) {
       const int64_t slot = group_slot(q, p.G, n, l.tile, l.chunk, g);
       part[slot] = cnt;

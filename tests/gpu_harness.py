@@ -74,6 +74,16 @@ def cabi_bwd(dy_nrc, x_nrc, w, b, mean, rstd, G, act, dx=None, ws=None, want_dw=
     return dx, dw, db
 
 
+def far_from_zero(N, R, C, dtype, gen):
+    """N(m, 1) with one m for all channels, 1000 (bfloat16, whose spacing there would be the deviations': 200), and a first
+    row a tenth further off."""
+    far = 200.0 if dtype == torch.bfloat16 else 1000.0
+    x = torch.randn((N, R, C), generator=gen, device=gen.device).add_(far)
+    if R > 100000:  # (of few rows it would be the variance)
+        x[:, 0] *= 1.1
+    return x.to(dtype)
+
+
 def err(a, truth):
     """max_i |a_i - t_i| / (|t_i| + rms(t)): relative for elements of typical size, and relative to the
     tensor's scale for elements near zero (where a pure ratio is meaningless)."""

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from gnnhwc import _cabi
-from tests.gpu_harness import cabi_bwd, cabi_fwd, err
+from tests.gpu_harness import cabi_bwd, cabi_fwd, err, far_from_zero
 from tests.test_gpu_parity import FP32_TOL, _check_against_torch
 
 pytestmark = pytest.mark.gpu
@@ -69,31 +69,39 @@ def test_consumer_tiling(N, R, C, G, dtype, device):
     assert _cabi.last_launch() == "multi-launch"
 
 
-# The statistics pass takes every tiles-th batch of eight rows per lane: one batch and a part of one, as many batches as tiles, one row
-# more and less than whole batches, several samples; and tensors beyond what the memory-side cache is counted on to hold (the
-# last four), whose first batches and whose consumer use non-temporal loads.  Means of 30 standard deviations, which sums about
-# anything but a value of the data would lose.  FP32_TOL is the bar of all float32 results; y adds half a spacing of its type.
+# The statistics pass takes every tiles-th batch of eight rows per lane: fewer rows per lane than a batch (1, 2, 4, 5, 7), one batch
+# and a part of one, as many batches as tiles, one row more and less than whole batches, several samples, more samples than a
+# grid has layers; and tensors beyond what the memory-side cache is counted on to hold (the last four), whose first batches and
+# whose consumer use non-temporal loads.  One mean for all channels, many standard deviations away, and one row further off
+# still: sums about anything but a value of the data lose what test_oracle.py's test of lane sums shows.  FP32_TOL is the bar of
+# all float32 results; y = x a + c adds half a spacing of its type and, of x a, the roundings of a, of the mean and of c.
 @pytest.mark.parametrize("N,R,C,G,dtype", [
     (1, 1, 64, 8, torch.float32), (2, 255, 64, 8, torch.float32), (2, 257, 64, 8, torch.bfloat16), (1, 16384 * 12, 64, 2, torch.float32),
+    (300, 32, 64, 8, torch.bfloat16), (300, 64, 64, 8, torch.float16), (400, 128, 64, 8, torch.bfloat16), (500, 160, 64, 8, torch.float16),
+    (500, 225, 64, 8, torch.bfloat16), (65537, 33, 16, 2, torch.bfloat16),
     (1, 16384 * 12 + 1, 64, 2, torch.float16), (3, 16384 * 4 - 1, 64, 8, torch.float32), (1, 7919, 140, 4, torch.bfloat16),
     (2, 40007, 64, 8, torch.float64), (1, 940007, 64, 8, torch.float32), (3, 170003, 128, 16, torch.float32),
     (1, 524287, 256, 32, torch.float16), (2, 262145, 256, 8, torch.bfloat16)])
 def test_statistics_of_swept_rows(N, R, C, G, dtype, device):
     print("swept rows", N, R, C, G, dtype, flush=True)
     gen = torch.Generator(device=device).manual_seed(R + C)
-    x = torch.randn((N, R, C), generator=gen, device=device).add_(30.0 * torch.randn((C,), generator=gen, device=device)).to(dtype)
+    x = torch.empty((N, R, C), dtype=dtype, device=device)
+    for n in range(0, N, 4096):
+        x[n:n + 4096] = far_from_zero(min(4096, N - n), R, C, dtype, gen)
     w, b = torch.rand(C, generator=gen, device=device).to(dtype) + 0.5, torch.randn(C, generator=gen, device=device).to(dtype)
     y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 0)
     assert _cabi.last_launch() == "multi-launch"
     half = {torch.float32: 0.0, torch.float64: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
-    for n in range(N):
+    for n in range(N) if N < 8 else (0, 1, N // 2, N - 1):
         xd = x[n].double().view(R, G, C // G)
         mu, var = xd.mean(dim=(0, 2)), xd.var(dim=(0, 2), correction=0)
         rs = (var + 1e-5).rsqrt()
         assert err(mean[n], mu) <= FP32_TOL and err(rstd[n], rs) <= FP32_TOL, (err(mean[n], mu), err(rstd[n], rs))
-        want = ((xd - mu[:, None]) * rs[:, None]).view(R, C) * w.double() + b.double()
-        off = (y[n].double() - want).abs() / (want.abs() + want.square().mean().sqrt())
-        assert float(off.max()) <= FP32_TOL + half, float(off.max())
+        xa = xd * rs[:, None]
+        want = (xa - (mu * rs)[:, None]).view(R, C) * w.double() + b.double()
+        off = (y[n].double() - want).abs() / (want.abs() + want.square().mean().sqrt() + 1e-30)
+        lost = 4 * 2.0 ** -24 * float((xa.abs().view(R, C) * w.double()).max() / want.square().mean().sqrt())
+        assert float(off.max()) <= FP32_TOL + half + (0.0 if dtype == torch.float64 else lost), float(off.max())
 
 
 @pytest.mark.parametrize("want_dw,want_db", [(True, False), (False, True), (False, False)])

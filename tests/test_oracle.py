@@ -188,3 +188,39 @@ def test_oracle_float32_variant_tracks_float64():
         r32 = orc.fwd_bwd(x, w, b, dy, G, 1e-5, act, dtype=np.float32)
         for k in ("y", "mean", "rstd", "dx", "dw", "db"):
             assert rel(r32[k].astype(np.float64), r64[k]) < 2e-5, (act, k)
+
+
+@pytest.mark.parametrize("dtype,lanes", [(torch.float32, 16), (torch.float16, 32)])
+def test_lane_sums_need_a_pivot_of_the_data(dtype, lanes):
+    """The streaming statistics keep float32 sums per lane about a value of the data and merge the lanes.  On the data of
+    test_statistics_of_swept_rows such sums stay far within that test's bar, and sums about zero are far beyond it.
+    (bfloat16 has so few bits that squares and their sums are exact about zero, too.)"""
+    from tests.gpu_harness import far_from_zero
+    from tests.test_gpu_parity import FP32_TOL
+
+    R, C = 768 * lanes, 64
+    x = far_from_zero(1, R, C, dtype, torch.Generator().manual_seed(1))[0].float()
+    true = float((x.double().var(correction=0) + 1e-5).rsqrt())
+
+    def rstd(pivot):
+        mean = pivot.clone()
+        n, m2 = 0, torch.zeros_like(mean)
+        for batch in x.view(-1, 8, lanes, C):  # batches of eight rows per lane
+            s1 = torch.zeros_like(mean)
+            s2 = torch.zeros_like(mean)
+            for row in batch:
+                d = row - (mean if pivot.any() else 0.0)
+                s1, s2 = s1 + d, s2 + d * d
+            n += 8
+            if pivot.any():
+                t = s1 / n
+                mean, m2 = mean + t, m2 + (s2 - s1 * t)
+            else:
+                mean, m2 = mean + s1, m2 + s2
+        if not pivot.any():
+            mean, m2 = mean / n, m2 - mean * (mean / n)
+        total = m2.double().sum() + n * (mean.double() - mean.double().mean()).square().sum()
+        return float((total / (R * C) + 1e-5).rsqrt())
+
+    assert abs(rstd(x[:lanes]) / true - 1) <= 0.2 * FP32_TOL
+    assert not abs(rstd(torch.zeros(lanes, C)) / true - 1) <= 2 * FP32_TOL
