@@ -730,13 +730,17 @@ __device__ __forceinline__ void recover_bwd_tail(const T *x, const T *dy, int dy
 // ---------------------------------------------------------------------------------------------
 // Occupancy the register budget is sized for.  16 rows fit four workgroups per CU for every type because float gamma / beta are
 // requested behind the statistics (late_params; with them in front, those kernels took 131 - 135 registers, three workgroups):
-// bf16 (16, 320, 128, 128), float parameters, 76.5 -> 74.5 us; float32 (2, 256, 256, 256) 59.3 -> 56.9.
+// bf16 (16, 320, 128, 128), float parameters, 76.5 -> 74.5 us; float32 (2, 256, 256, 256) 59.3 -> 56.9.  With a channel addend,
+// float parameters and 16-bit data ten of 138 registers then pass through scratch memory, which costs less than the fourth
+// workgroup gives: bf16 (4 / 6, 320, 128, 128) 26.9 / 35.1 us at three workgroups without, 26.4 / 34.1 at four.
 // (with a residual: the tile plus a window of residual_window(nv) rows of the residual)
 constexpr int residual_window(int nv) { return nv <= 8 ? nv : 8; }
 constexpr int fused_fwd_waves(int nv, int add) {
   return add == kAddResidual ? (nv <= 4 ? 4 : nv <= 16 ? 3 : 2) : (nv <= 16 ? 4 : 2);
 }
-constexpr bool late_params(int nv, int param_bytes) { return nv >= 16 && param_bytes == 4; }
+// Kernels with additions have the addend's loads in front of the rows and request gamma / beta late whatever their size: bf16
+// (2, 640, 64, 64) 13.4 -> 13.1 us, (3, 320, 128, 128) 28.3 -> 27.9, (5, 320, 128, 128) 48.8 -> 47.2, all with a residual.
+constexpr bool late_params(int nv, int add, int param_bytes) { return add != kAddNone || (nv >= 16 && param_bytes == 4); }
 // TWO_LEVEL: the exchange of a launch with many row tiles per sample (two_level_exchange on the host).  A template
 // parameter, not a run-time switch: the code of the form a launch does not use would sit in the middle of the path every
 // workgroup executes once, and these kernels are sensitive to their own size.
@@ -793,9 +797,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
   // gamma / beta are needed only after the exchange, but they are requested first and without any branch: a load
   // under a branch makes the compiler drain every outstanding load where the branch joins, and then the statistics
   // below could not start on the first rows while the later ones are still arriving.  Where they would cost a fourth
-  // workgroup per CU (see fused_fwd_waves) they are requested behind the publication of the tile's moments instead, which
+  // workgroup per CU (see fused_fwd_waves) or follow an addend they are requested behind the publication of the tile's moments instead, which
   // takes a kernel that is not short of registers 0.2 - 0.6 us longer.
-  constexpr bool kLateParams = late_params(NV, (int)sizeof(PT));
+  constexpr bool kLateParams = late_params(NV, ADD, (int)sizeof(PT));
   A sa[VEC], sb[VEC];
   auto request_params = [&]() {
     const int cvi = l.cvi < p.cv ? l.cvi : p.cv - 1;
@@ -918,6 +922,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_fw
     request_params();
     issue_order_fence();
   }
+  // The stores of the sum are let out before the first look at the others' records: looks that queue behind them, on this CU and
+  // the others, come too early and have to be repeated.  bf16 with a residual (8 / 3, 320, 128, 128) 78.8 / 27.9 -> 76.8 / 26.0 us,
+  // (2, 640, 64, 64) 13.1 -> 12.9; with a channel addend (4 / 6, 320, 128, 128) 26.2 / 34.1 -> 25.3 / 33.1.
+  if constexpr (ADD != kAddNone) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // Each of the two phases that follow works on its own copy of the kernel's arguments, read again where the phase
   // begins: what the phases before it loaded need not stay in scalar registers (or be spilled and restored) all the way.
   const unsigned long long epoch = sync.epoch;
