@@ -567,7 +567,7 @@ __device__ __forceinline__ void recover_fwd(const T *x, T *y, const SyncArea &sy
 
 // The same for a backward workgroup, up to and including its rows of dx: the group sums of the chunk's groups from the
 // tile records (or from x and dy where they are missing) give the coefficients, then dx row by row from memory.
-template <typename T, typename PT, int VEC, int ACT, bool TWO_LEVEL, bool DY16>
+template <typename T, typename PT, int VEC, int ACT, bool TWO_LEVEL, bool DY16, bool EXACT>
 __device__ __forceinline__ void recover_bwd_dx(const T *x, const T *dy, T *dx, int dydtype, const void *mean, const void *rstd,
                                                int sdtype, const void *w, const void *b, const SyncArea &sync, const Plan &p,
                                                RecoveryLds &r, const float *sm_mu, const float *sm_rs, float *sm_k1,
@@ -618,9 +618,10 @@ __device__ __forceinline__ void recover_bwd_dx(const T *x, const T *dy, T *dx, i
       unpack_dy<T, VEC, DY16>(load_dy<T, VEC, DY16>(dy, off + (int64_t)u * step), vd, dydtype);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) vd[j] = vd[j] * act_bwd<ACT, float>(vx[j] * sa[j] + sb[j]);
-      // (g' passes through T as on the fast path, where it waits in registers in packed form)
-      const typename LV::raw_t gp = LV::pack(vd);
-      LV::unpack(gp, vd);
+      if constexpr (!EXACT) {  // g' passes through T as on the fast path, where it waits in registers in packed form
+        const typename LV::raw_t gp = LV::pack(vd);
+        LV::unpack(gp, vd);
+      }
 #pragma unroll
       for (int j = 0; j < VEC; ++j) vd[j] = sa[j] * vd[j] + (c1[j] * vx[j] + c2[j]);
       store_streaming<LV>(dx + off + (int64_t)u * step, LV::pack(vd));
@@ -1109,7 +1110,9 @@ constexpr bool dy_streams(int nv) { return nv > 16; }
 // Statistics slots in LDS of a backward kernel: one per group of the chunk.  The kernels with parked rows need their LDS
 // for those and serve chunks of at most kBlock channels (the host checks), hence at most kBlock groups.
 constexpr int fused_bwd_stat_slots(int vec, int xl) { return xl > 0 ? kBlock : kBlock * vec; }
-template <typename T, typename PT, int VEC, int ACT, int NV, bool TWO_LEVEL, int XW = 0, int XL = 0, bool DY16 = false>
+// EXACT (with XW > 0): dy itself is kept, not g', which is formed again in the second pass, in float, from the x that pass
+// reads anyway; for 16-bit data g' kept in between is rounded to the data type.
+template <typename T, typename PT, int VEC, int ACT, int NV, bool TWO_LEVEL, int XW = 0, int XL = 0, bool DY16 = false, bool EXACT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bwd_waves(NV, XW)))) void fused_bwd_kernel(
     const FusedBwdParams args) {
   using A = acc_t<T>;
@@ -1255,7 +1258,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
           s2[j] += g;
           vd[j] = g;
         }
-        bd[u] = LV::pack(vd);
+        if constexpr (!EXACT) bd[u] = LV::pack(vd);
         if constexpr (XW == 0 && NV > 16 && std::is_same<T, f16_t>::value) {
           // row by row here too (see the windowed form below): without it the conversions of float16, which the scheduler
           // takes further ahead than bfloat16's shifts, spilled up to 66 registers to memory.  float16 (2, 128, 400, 400)
@@ -1422,7 +1425,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
     const FusedBwdParams ka = reread_kernel_args<FusedBwdParams>();
     SyncArea ks = ka.sync;
     ks.epoch = epoch;
-    recover_bwd_dx<T, PT, VEC, ACT, TWO_LEVEL, DY16>((const T *)ka.x, (const T *)ka.dy, (T *)ka.dx, ka.dydtype, ka.mean, ka.rstd,
+    recover_bwd_dx<T, PT, VEC, ACT, TWO_LEVEL, DY16, EXACT>((const T *)ka.x, (const T *)ka.dy, (T *)ka.dx, ka.dydtype, ka.mean, ka.rstd,
                                                      ka.sdtype, ka.w, ka.b, ks, ka.p, recovery, sm_mu, sm_rs, sm1, sm2);
     if ((int)blockIdx.z == (ka.tail_last ? (int)gridDim.z - 1 : 0) && (ka.dw || ka.db))
       recover_bwd_tail<T, PT, ACT, DY16>((const T *)ka.x, (const T *)ka.dy, ka.dydtype, ka.w, ka.b, ka.mean_all, ka.rstd_all, ka.sdtype,
@@ -1483,9 +1486,20 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fused_bw
           LV::unpack(bx[u % NX], vx);
         }
         pin(bd[u]);
-        LV::unpack(bd[u], vd);  // g'
+        LV::unpack(bd[u], vd);  // g' (EXACT: dy)
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) vd[j] = sa[j] * vd[j] + (c1[j] * vx[j] + c2[j]);
+        for (int j = 0; j < VEC; ++j) {
+          if constexpr (EXACT) {
+            if (VEC >= 4 && j == VEC / 2) {  // half a row at a time, as in the first pass
+#pragma unroll
+              for (int i = 0; i < VEC / 2; ++i) pin(vd[i]);
+#pragma unroll
+              for (int i = VEC / 2; i < VEC; ++i) { pin(vx[i]); pin(vd[i]); }
+            }
+            vd[j] *= act_bwd<ACT, A>(vx[j] * sa[j] + sb[j]);
+          }
+          vd[j] = sa[j] * vd[j] + (c1[j] * vx[j] + c2[j]);
+        }
         if (u < rows) store_streaming<LV>((T *)tile_row(dx, t2, u), LV::pack(vd));
         if (u >= XW && u - XW >= XL) {
           issue_order_fence();

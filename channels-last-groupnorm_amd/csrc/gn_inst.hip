@@ -274,20 +274,23 @@ bool try_resident_fwd(const FwdArgs &a) {
 // float16 (1, 256, 400, 500) 87 / 66; bf16 (32, 320, 128, 128) 320 / 190.
 // (set by set with 16 or 22 rows of both tensors in registers: bf16 (16, 320, 128, 128) 128 and 101 us.)
 constexpr int kRolling = 0;  // in the place of a number of launches: one launch, set by set
-template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled);
-template <typename PT, int ACT, int NV, int XW = 0, int XL = 0> bool try_resident_bwd_nv(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
+template <typename PT, int ACT, int NV, int XW, int XL, bool EXACT, bool DY16>
+bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled);
+template <typename PT, int ACT, int NV, int XW = 0, int XL = 0, bool EXACT = false>
+bool try_resident_bwd_nv(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
   if (a.dydtype != GN_INST_DTYPE) {
-    if constexpr (kHasDy16) return try_resident_bwd_one<PT, ACT, NV, XW, XL, true>(a, records, batches, underfilled);
+    if constexpr (kHasDy16) return try_resident_bwd_one<PT, ACT, NV, XW, XL, EXACT, true>(a, records, batches, underfilled);
     else return false;
   }
-  return try_resident_bwd_one<PT, ACT, NV, XW, XL, false>(a, records, batches, underfilled);
+  return try_resident_bwd_one<PT, ACT, NV, XW, XL, EXACT, false>(a, records, batches, underfilled);
 }
-template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
+template <typename PT, int ACT, int NV, int XW, int XL, bool EXACT, bool DY16>
+bool try_resident_bwd_one(const BwdArgs &a, const BwdRecords &records, int batches, bool *underfilled) {
   if (NV < resident_min_rows()) return false;
   // (kernels that park rows of x in LDS have statistics slots for chunks of at most kBlock channels)
   if (XL > 0 && a.plan.lpr * a.plan.vec > kBlock) return false;
-  auto kernel_all = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, false, XW, XL, DY16>;
-  auto kernel_two = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, true, XW, XL, DY16>;
+  auto kernel_all = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, false, XW, XL, DY16, EXACT>;
+  auto kernel_two = fused_bwd_kernel<elem_t, PT, kVec, ACT, NV, true, XW, XL, DY16, EXACT>;
   static const int slots = std::min(resident_slots(kernel_all), resident_slots(kernel_two));
   const int64_t per = batches == kRolling ? a.plan.N : (a.plan.N + batches - 1) / batches;
   Plan p;
@@ -296,15 +299,15 @@ template <typename PT, int ACT, int NV, int XW, int XL, bool DY16> bool try_resi
   if (!resident_tiling(a.plan, per, NV, slots, p, rolling)) return false;
   if (rolling && tail_blocks_per_chunk(p, a.plan.N) > p.tiles) return false;  // (tail_blocks relies on it)
   const int64_t count = rolling ? 1 : (a.plan.N + per - 1) / per;  // launches
-  if (underfilled && a.plan.N * p.nchunk * p.tiles * 10 < count * slots * 8) {
-    *underfilled = true;
-    return false;
-  }
   // (the windowed form addresses the rows of a tile by 32-bit byte offsets from the tile's first row)
   if (XW > 0 && (int64_t)p.tile_rows * p.C * (int64_t)sizeof(elem_t) >= ((int64_t)1 << 31)) return false;
   // the channel records of every sample stay in the workspace until the last launch has summed them
   const size_t crec_need = (size_t)a.plan.N * p.tiles * a.plan.C * 16;
-  if (crec_need > records.crec) return false;
+  if (crec_need > (rolling ? records.crec : resident_crec_bytes((int64_t)p.lpr * p.vec))) return false;
+  if (underfilled && a.plan.N * p.nchunk * p.tiles * 10 < count * slots * 8) {
+    *underfilled = true;
+    return false;
+  }
   if (!resident_status()) return false;
   CapturedEpoch cap;
   if (!captured_epoch(a.stream, cap)) return false;
@@ -365,7 +368,20 @@ template <typename PT, int ACT> bool try_resident_bwd_act(const BwdArgs &a) {
   for (int b = 1; b <= most && !underfilled; ++b) {  // as few launches as it takes, each well filled ...
     if (launches(b, b > 1 ? &underfilled : nullptr)) return true;
   }
-  if (records.rolling && try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, records, kRolling, nullptr)) return true;
+  // Set by set.  Where launches that keep g' could serve the call, so may the set-by-set form that does.  Where only the streaming
+  // kernels could, which use g' in float, it is not rounded here either (EXACT; the identity's and relu's g', dy or 0, never is):
+  // relative error of dx (2-norm), bf16 silu, 1.66e-3 as in the streaming kernels, 2.35e-3 with g' rounded.  The second
+  // evaluation of the derivative, and a window that leaves it registers, cost bf16 (32, 320, 128, 128) 190 -> 218 us (streaming
+  // 321), (1, 640, 256, 256) 50.9 -> 57.4 (77).  (A window of 16 rows spills 46 registers, 226 and 59.5 us.)
+  constexpr bool rounds = sizeof(elem_t) == 2 && ACT != GN_ACT_IDENTITY && ACT != GN_ACT_RELU;
+  constexpr int exact_window = 12;
+  if (records.rolling && (underfilled || !rounds)) {
+    if (try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, records, kRolling, nullptr)) return true;
+  }
+  if constexpr (rounds) {
+    if (records.rolling && !underfilled && try_resident_bwd_nv<PT, ACT, 32, exact_window, parked, true>(a, records, kRolling, nullptr))
+      return true;
+  }
   for (int b = 2; b <= most && underfilled; ++b) {  // ... or filled as they may be
     if (launches(b, nullptr)) return true;
   }

@@ -163,7 +163,8 @@ def cabi_bwd_cast(dy, x, w, b, mean, rstd, G, act, dx=None, dtype_code=None, dy_
 
 
 @pytest.mark.parametrize("dy_dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape,G", SHAPES + [((5, 128 * 128, 320), 32)])  # the last: a backward in two launches
+# (the last two: a backward in two launches over groups of samples, and one that runs set by set)
+@pytest.mark.parametrize("shape,G", SHAPES + [((7, 128 * 128, 256), 32), ((5, 128 * 128, 320), 32)])
 def test_cast_backward_matches_widen_then_backward(family, shape, G, dy_dtype, device):
     act_name = ACTS[(shape[1] + shape[2] + 1) % 5]
     act = orc.ACT_CODES[act_name]
@@ -176,6 +177,8 @@ def test_cast_backward_matches_widen_then_backward(family, shape, G, dy_dtype, d
     rc, dx, dw, db = cabi_bwd_cast(dy16, x, w, b, mean, rstd, G, act)
     _cabi.check(rc, "gnnhwc_bwd_cast")
     torch.cuda.synchronize()
+    if shape[0] in (5, 7) and family == "resident":
+        assert _cabi.last_launch().endswith("parked=16 two_level=0 launches=%d" % (2 if shape[0] == 7 else 1)), _cabi.last_launch()
     for name, got, ref in (("dx", dx, want[0]), ("dweight", dw, want[1]), ("dbias", db, want[2])):
         assert torch.equal(got, ref), "%s differs from the backward on the widened gradient" % name
     # without parameters, and float32 dy through the same entry point (= gnnhwc_bwd)

@@ -420,7 +420,9 @@ def test_inference_in_place_without_statistics(family, shape, G, device):
     (2, 23 * 19, 64, 8, "silu", torch.bfloat16),
     (4, 128 * 128, 320, 32, "gelu", torch.bfloat16),
     (1, 150037, 192, 24, "silu", torch.bfloat16),      # the backward that keeps g' and streams x through a window
-    (6, 128 * 128, 320, 32, "relu", torch.float16),    # a backward in two launches over groups of samples
+    (6, 128 * 128, 320, 32, "relu", torch.float16),    # the same, several samples
+    (8, 128 * 128, 320, 32, "relu", torch.float16),    # a backward in two launches over groups of samples
+    (7, 128 * 128, 256, 32, "silu", torch.float32),    # the same, each launch with a window
     (3, 37 * 53, 96, 24, "gelu_tanh", torch.float32),
     (2, 1000, 30, 5, "silu", torch.float32),           # scalar kernels
 ])
@@ -452,8 +454,11 @@ RECOVERY_SHAPES = [
     (1, 64 * 64, 1280, 32, "silu", torch.bfloat16),
     (2, 9000, 40, 5, "relu", torch.float32),
     (1, 150037, 192, 24, "silu", torch.bfloat16),      # 58 MB: the windowed backward
-    (6, 128 * 128, 320, 32, "silu", torch.bfloat16),   # backward in two launches over groups of samples
+    (6, 128 * 128, 320, 32, "silu", torch.bfloat16),   # the same, several samples
+    (8, 128 * 128, 320, 32, "silu", torch.bfloat16),   # backward in two launches over groups of samples
+    (7, 128 * 128, 256, 32, "gelu", torch.float32),    # the same, each launch with a window
 ]
+IN_TWO_LAUNCHES = {(8, 320): "rows=22 window=0 parked=0 two_level=0 launches=2", (7, 256): "rows=32 window=12 parked=16 two_level=0 launches=2"}
 
 
 @pytest.mark.parametrize("N,R,C,G,act,dtype", RECOVERY_SHAPES)
@@ -515,6 +520,7 @@ def test_single_launch_kernels_recover_from_expired_waits(N, R, C, G, act, dtype
         dx2, dw2, db2 = cabi_bwd(dy, x, w, b, mean2, rstd2, G, code)
         torch.cuda.synchronize()
         _cabi.profile_enable(False)
+        assert _cabi.last_launch().endswith(IN_TWO_LAUNCHES.get((N, C), "launches=1")), _cabi.last_launch()
         launches = {k: v[0] for k, v in _cabi.profile_collect().items() if v[0]}
         assert set(launches) == {"fused_fwd", "fused_bwd"}, launches
         assert lib.gnnhwc_resident_status() == 0
