@@ -918,6 +918,18 @@ int gnnhwc_debug_consumer_plan(int64_t N, int64_t R, int64_t C, int64_t G, int d
   return GNNHWC_OK;
 }
 
+int gnnhwc_debug_backward_sets(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int64_t *out) {
+  Plan p;
+  const int rc = debug_producer_plan(N, R, C, G, dtype, 1, 1, out, p);
+  if (rc != GNNHWC_OK) return rc;
+  const BwdRecords r = dtype != GN_F64 ? resident_bwd_records(p) : BwdRecords{0, 0, 0, false};
+  p.tile_rows = kRollingBwdRows * p.rpi;
+  p.tiles = (int)((R + p.tile_rows - 1) / p.tile_rows);
+  out[0] = r.rolling ? 1 : 0; out[1] = (int64_t)r.crec; out[2] = (int64_t)r.rec; out[3] = (int64_t)r.frec;
+  out[4] = p.tiles; out[5] = p.nchunk; out[6] = tail_blocks_per_chunk(p, N); out[7] = exchange_chunks(p);
+  return GNNHWC_OK;
+}
+
 const char *gnnhwc_kernel_kind_name(int kind) {
   static const char *names[GNNHWC_NUM_KERNEL_KINDS] = {"fwd_stats", "fwd_stats_compact", "fwd_apply", "bwd_reduce",
                                                        "bwd_compact", "bwd_dx", "fused_fwd", "fused_bwd", "copy",

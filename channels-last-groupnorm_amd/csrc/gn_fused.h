@@ -1105,7 +1105,8 @@ struct FusedBwdParams {
 // dy, which is read once, is read with the non-temporal hint (load_dy) where more than 16 rows per lane hold the tensor, that is
 // above 32 MB of it: what a call of that size touches does not stay in the caches as a whole, and the hint leaves more of it to x.
 // Smaller ones are found there, and lines read with the hint are not, the next time: bf16 (1, 640, 128, 128), the same tensors
-// again and again, 15.2 us without it, 16.1 with.
+// again and again, 15.2 us without it, 16.1 with.  At 22 rows (32 - 46 MB) the backward takes the same with and without, bf16
+// (4, 320, 128, 128) 23.2 / 23.3, but in launches of 22 rows the hint keeps x for the next forward: (8, 320, 128, 128) 32.2 / 37.3.
 constexpr bool dy_streams(int nv) { return nv > 16; }
 // Statistics slots in LDS of a backward kernel: one per group of the chunk.  The kernels with parked rows need their LDS
 // for those and serve chunks of at most kBlock channels (the host checks), hence at most kBlock groups.

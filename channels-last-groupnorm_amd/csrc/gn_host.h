@@ -133,7 +133,7 @@ inline FwdRecords resident_fwd_records(const Plan &p) {
   FwdRecords r = {align_up(resident_rec_bytes(p.G), 256), align_up(resident_frec_bytes(p.G), 256), false};
   const int64_t rows = (int64_t)kRollingRows * p.rpi;
   const int64_t columns = p.N * p.nchunk, tiles = (p.R + rows - 1) / rows;
-  // full tiles only, and record indices within the kernels' 24-bit multiplies
+  // samples of a full tile or more, and record indices within the kernels' 24-bit multiplies
   if (p.N > 65535 || p.R < rows || columns * p.G >= (1 << 23) || tiles >= (1 << 23)) return r;
   const size_t rec = (size_t)16 * p.G * columns * tiles;
   if (rec > kRollingRecordBytes) return r;
@@ -172,15 +172,16 @@ struct BwdRecords {
   size_t crec, rec, frec;  // bytes of the channel records, of the tile records and of the final records
   bool rolling;            // a rolling launch is allowed
 };
+constexpr int kRollingBwdRows = 32;  // rows per lane of the one form that runs set by set
 inline BwdRecords resident_bwd_records(const Plan &p) {
   const int64_t cc = (int64_t)p.lpr * p.vec;
   BwdRecords r = {resident_crec_bytes(cc), align_up(resident_rec_bytes(p.G), 256), align_up(resident_frec_bytes(p.G), 256), false};
-  const int64_t rows = (int64_t)kRollingRows * p.rpi;
+  const int64_t rows = (int64_t)kRollingBwdRows * p.rpi;
   const int64_t columns = p.N * p.nchunk, tiles = (p.R + rows - 1) / rows;
-  // full tiles only, and record indices within the kernels' 24-bit multiplies
+  // samples of a full tile or more, and record indices within the kernels' 24-bit multiplies
   if (p.N > 65535 || p.R < rows || columns * p.G >= (1 << 23) || p.N * tiles >= (1 << 23) || p.C >= (1 << 23)) return r;
   const size_t rec = (size_t)16 * p.G * columns * tiles, crec = (size_t)16 * p.N * tiles * p.C;
-  if (rec > kRollingRecordBytes || crec > kRollingRecordBytes) return r;
+  if (rec > kRollingRecordBytes / 2 || crec > kRollingRecordBytes / 2) return r;
   r.rolling = true;
   if (crec > r.crec) r.crec = align_up(crec, 256);
   if (rec > r.rec) r.rec = align_up(rec, 256);
@@ -192,7 +193,9 @@ inline size_t resident_bwd_bytes(const Plan &p) {
   const BwdRecords r = resident_bwd_records(p);
   return kWorkspaceHeader + r.crec + r.rec + r.frec;
 }
-// Blocks of channels that the dgamma / dbeta stage of the single-launch backward cuts a chunk into (tail_blocks).
+// Blocks of channels that the dgamma / dbeta stage of the single-launch backward cuts a chunk into (tail_blocks).  Set by set, a
+// sample needs as many row tiles: 16 blocks for 16-bit data, 8 for float, from 64 (sample, tile) pairs on, i.e. samples of more
+// than 15 x 1024 or 7 x 1024 rows of 128 bytes.  Batches of smaller ones that four launches cannot hold stay on the streaming kernels.
 inline int tail_blocks_per_chunk(const Plan &p, int64_t samples) {
   const int64_t pairs = samples * p.tiles;
   const int cpp = kBlock / pow2_at_least(pairs < 64 ? (int)pairs : 64), cc = p.lpr * p.vec;

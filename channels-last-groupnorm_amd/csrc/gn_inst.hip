@@ -269,9 +269,10 @@ bool try_resident_fwd(const FwdArgs &a) {
 // (80 % of the workgroups that can be resident), else as one launch set by set, as the forward does (try_resident_fwd_nv), in the form
 // that holds the most rows per workgroup.  Full launches load, exchange and store in step and reach 5.6 TB/s; set by set, no
 // launch is left half empty and no gap lies between two.  Launches against set by set: bf16 (16, 320, 128, 128), 83 % full,
-// 89.5 / 96 us; (12, 320, 128, 128), 94 %, 80.5 / 89; float32 (2, 256, 256, 256), full, 73 / 76; but (3, 640, 200, 200), 78 %,
-// 97 / 88; (3, 640, 150, 160), 70 %, 50.9 / 49.7.  Where only the streaming kernels were left: float32 (1, 128, 512, 512) 107.9 / 73.7;
-// float16 (1, 256, 400, 500) 87 / 66; bf16 (32, 320, 128, 128) 320 / 190.
+// 89.5 / 96 us; (12, 320, 128, 128), 94 %, 80.5 / 89; float32 (2, 256, 256, 256), full, 73 / 76; at 78 % float32 (5, 320, 128, 128)
+// 58.0 / 58.6 and bf16 (3, 640, 200, 200) 97 / 88; at 70 % bf16 (3, 640, 150, 160) 51.0 / 49.7, (9, 320, 128, 128) 61.6 / 48.8; at
+// 68 % (5, 320, 140, 200) 60.7 / 49.3, (7, 320, 125, 160) 60.6 / 48.6.  Where only the streaming kernels were left: float32
+// (1, 128, 512, 512) 107.9 / 73.7; for 16-bit data see try_resident_bwd_act.
 // (set by set with 16 or 22 rows of both tensors in registers: bf16 (16, 320, 128, 128) 128 and 101 us.)
 constexpr int kRolling = 0;  // in the place of a number of launches: one launch, set by set
 template <typename PT, int ACT, int NV, int XW, int XL, bool EXACT, bool DY16>
@@ -376,10 +377,10 @@ template <typename PT, int ACT> bool try_resident_bwd_act(const BwdArgs &a) {
   constexpr bool rounds = sizeof(elem_t) == 2 && ACT != GN_ACT_IDENTITY && ACT != GN_ACT_RELU;
   constexpr int exact_window = 12;
   if (records.rolling && (underfilled || !rounds)) {
-    if (try_resident_bwd_nv<PT, ACT, 32, window, parked>(a, records, kRolling, nullptr)) return true;
+    if (try_resident_bwd_nv<PT, ACT, kRollingBwdRows, window, parked>(a, records, kRolling, nullptr)) return true;
   }
   if constexpr (rounds) {
-    if (records.rolling && !underfilled && try_resident_bwd_nv<PT, ACT, 32, exact_window, parked, true>(a, records, kRolling, nullptr))
+    if (records.rolling && !underfilled && try_resident_bwd_nv<PT, ACT, kRollingBwdRows, exact_window, parked, true>(a, records, kRolling, nullptr))
       return true;
   }
   for (int b = 2; b <= most && underfilled; ++b) {  // ... or filled as they may be

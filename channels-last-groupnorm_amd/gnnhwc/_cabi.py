@@ -41,6 +41,7 @@ SYMBOLS = (
     "gnnhwc_debug_read_trace",
     "gnnhwc_debug_plan",
     "gnnhwc_debug_consumer_plan",
+    "gnnhwc_debug_backward_sets",
     "gnnhwc_debug_last_launch",
     "gnnhwc_debug_load_tile",
 )
@@ -103,6 +104,8 @@ def _load():
     lib.gnnhwc_debug_plan.restype = ci
     lib.gnnhwc_debug_consumer_plan.argtypes = list(lib.gnnhwc_debug_plan.argtypes)
     lib.gnnhwc_debug_consumer_plan.restype = ci
+    lib.gnnhwc_debug_backward_sets.argtypes = [i64] * 4 + [ci, ctypes.POINTER(i64)]
+    lib.gnnhwc_debug_backward_sets.restype = ci
     lib.gnnhwc_debug_last_launch.argtypes = [ctypes.POINTER(i64)]
     lib.gnnhwc_debug_last_launch.restype = ci
     lib.gnnhwc_kernel_kind_name.argtypes = [ci]

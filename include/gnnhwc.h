@@ -230,7 +230,8 @@ int gnnhwc_bwd_nchw(const void *dy, const void *x, const void *weight, const voi
  * that exchange with each other -- those on one 128-byte chunk of a sample's rows, or on the few chunks that a
  * group spans -- fit half of the device (up to 262144 rows where groups lie inside chunks) and
  * their records 32 MB (a larger backward may also run as up to four such launches over groups of samples, where these fill
- * the device well); anything else is run by the multi-launch streaming kernels.  A single-launch kernel is
+ * the device well; set by set its records may take 16 MB each, and with 64 or more row tiles in the batch a sample needs
+ * more than 15360 rows of 128 bytes, 7168 for float data); anything else is run by the multi-launch streaming kernels.  A single-launch kernel is
  * fastest with the device to itself: calls of one process on different streams are ordered by the library (a call on another stream than the previous single-launch
  * call of the device first makes its stream wait, on the device, for what has been submitted to that
  * previous stream).  Where the device is shared all the same (launches recorded into graphs that are replayed
@@ -331,6 +332,13 @@ int gnnhwc_debug_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int
  */
 int gnnhwc_debug_consumer_plan(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int vector, int backward,
                                int64_t *out /* [11] */);
+/*
+ * The same for a backward run set by set (16-byte lane vectors).  out[8] receives: 1 if the record indices and the record
+ * memory allow such a launch, bytes of its channel records, tile records and final records (whether or not it is allowed),
+ * row tiles of a sample, chunks along C, blocks of channels per chunk of its dgamma / dbeta stage (it also needs as many row
+ * tiles), chunks of a set.
+ */
+int gnnhwc_debug_backward_sets(int64_t N, int64_t R, int64_t C, int64_t G, int dtype, int64_t *out /* [8] */);
 
 /*
  * In-kernel timeline of the single-launch kernels, for tuning (no counterpart in the reference; its

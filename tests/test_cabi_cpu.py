@@ -368,3 +368,58 @@ def test_records_of_forwards_run_set_by_set():
                 assert 16 * columns * G * tiles <= rec and 16 * N * G <= frec, ctx
             assert rec <= max(32 << 20, 16 * G * 1024 + 255), ctx
     assert allowed > 100, allowed
+
+
+def _backward_sets(N, R, C, G, dtype):
+    out = (ctypes.c_int64 * 8)()
+    assert _cabi.lib.gnnhwc_debug_backward_sets(N, R, C, G, dtype, out) == 0, _cabi.last_error()
+    return dict(zip(("rolling", "crec", "rec", "frec", "tiles", "nchunk", "blocks", "chunks"), (int(v) for v in out)))
+
+
+def test_records_and_order_of_backwards_run_set_by_set():
+    """Where such a launch is allowed: record indices stay below the kernels' 24-bit multiplies, the record memory holds every
+    (sample, tile, channel), (sample, chunk, group, tile) and (sample, group), the workspace query covers it, no sample is shorter
+    than a tile; and every block of the dgamma / dbeta stage goes to one workgroup of the last sample, in a chunk that is the
+    block's own or behind it: what that workgroup waits for was dispatched before it or belongs to its set."""
+    allowed = ordered = 0
+    shapes = [(16, 16384, 320, 32), (1, 262144, 256, 32), (7, 16385, 640, 32), (33, 16384, 272, 17), (65535, 1024, 64, 8), (65536, 1024, 64, 8),
+              (80, 15360, 128, 32), (80, 15361, 128, 32), (150, 7168, 64, 32), (150, 7169, 64, 32), (4, 1023, 65536, 32), (4, 1024, 65536, 32),
+              (200, 4096, 640, 32), (3, 30000, 1920, 32)]
+    for (N, R, C, G) in shapes + list(_sample_shapes(8, 600)):
+        for dtype in (0, 2, 3):
+            full = 16 // _ELEM[dtype]
+            if C % full:
+                continue
+            p, s = _plan(N, R, C, G, dtype, 1, 1), _backward_sets(N, R, C, G, dtype)
+            ctx = (N, R, C, G, dtype, p, s)
+            rows, width = 32 * p["rpi"], p["lpr"] * full
+            assert s["tiles"] == -(-R // rows) and s["nchunk"] == p["nchunk"], ctx
+            assert s["crec"] >= 16 * width * 1024 and s["rec"] >= 16 * G * 1024 and s["frec"] >= 16 * G * 1024, ctx  # one resident launch
+            assert 256 + s["crec"] + s["rec"] + s["frec"] <= _cabi.lib.gnnhwc_bwd_workspace_bytes(N, R, C, G, dtype), ctx
+            if not s["rolling"]:
+                continue
+            allowed += 1
+            columns, pairs = N * s["nchunk"], N * s["tiles"]
+            assert N <= 65535 and R >= rows and columns * G < 1 << 23 and pairs < 1 << 23 and C < 1 << 23, ctx
+            assert 16 * pairs * C <= s["crec"] and 16 * columns * G * s["tiles"] <= s["rec"] and 16 * N * G <= s["frec"], ctx
+            if p["lpr"] & (p["lpr"] - 1):
+                continue  # (no single-launch kernel takes such a chunk)
+            side = 256 // min(64, 1 << (pairs - 1).bit_length())  # channels a workgroup finishes at a time
+            assert s["blocks"] == max(1, width // side), ctx
+            if s["blocks"] > s["tiles"]:
+                continue  # refused
+            ordered += 1
+            total, workgroups = s["nchunk"] * s["blocks"], s["nchunk"] * s["tiles"]
+            taken = [w - (workgroups - total) for w in range(workgroups)]  # first block of each workgroup, in dispatch order
+            assert [b for b in taken if b >= 0] == list(range(total)), ctx
+            assert all(b < 0 or w // s["tiles"] >= b // s["blocks"] for w, b in enumerate(taken)), ctx
+    assert allowed > 100 and ordered > 50, (allowed, ordered)
+    # where the line lies, for 16-bit and for float data
+    for below, dtype in (((80, 15360, 128, 32), 3), ((150, 7168, 64, 32), 0)):
+        s = _backward_sets(*below, dtype)
+        assert s["rolling"] and s["blocks"] == s["tiles"] + 1, s
+        s = _backward_sets(below[0], below[1] + 1, *below[2:], dtype)
+        assert s["rolling"] and s["blocks"] == s["tiles"], s
+    assert not _backward_sets(4, 1023, 65536, 32, 3)["rolling"] and _backward_sets(4, 1024, 65536, 32, 3)["rolling"]
+    assert _cabi.lib.gnnhwc_debug_backward_sets(1, 16, 12, 4, 3, (ctypes.c_int64 * 8)()) == -1
+    assert _cabi.lib.gnnhwc_debug_backward_sets(1, 16, 16, 4, 3, None) == -1

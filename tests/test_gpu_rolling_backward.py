@@ -126,6 +126,24 @@ def test_every_activation_against_float64(N, R, C, G, few, act, dtype, params, d
         _against_float64(x, dy, w, b, G, dx, dw, db, 1, act)
 
 
+# Batches on both sides of the line that dgamma / dbeta draw (as many row tiles in a sample as blocks of channels in a chunk; chunks
+# of 128 bytes), with more sets than four launches hold.
+@pytest.mark.parametrize("N,R,C,G,dtype", [(80, 15360, 128, 32, torch.bfloat16), (150, 7168, 64, 32, torch.float32)])
+def test_samples_with_fewer_tiles_than_blocks_are_left_to_the_streaming_kernels(N, R, C, G, dtype, device):
+    print("rolling backward, bound", N, R, C, G, dtype, flush=True)
+    for rows in (R, R + 1):
+        gen = torch.Generator(device=device).manual_seed(rows)
+        x, dy = (torch.empty((N, rows, C), device=device, dtype=dtype).normal_(generator=gen) for _ in range(2))
+        w, b = torch.rand((C,), device=device, generator=gen) + 0.5, 0.1 * torch.randn((C,), device=device, generator=gen)
+        _, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
+        dx, dw, db = cabi_bwd(dy, x, w, b, mean, rstd, G, 2)
+        if rows == R:
+            assert _cabi.last_launch() == "multi-launch"
+        else:
+            assert _roundings(x, 2, _assert_set_by_set()) == 1
+        _against_float64(x, dy, w, b, G, dx, dw, db, 1)
+
+
 @pytest.mark.parametrize("N,R,C,G", [(7, 16385, 640, 32), (1, 262144, 256, 32)])
 @pytest.mark.parametrize("spins", [-2, 0, 2])
 def test_expired_waits_are_recovered(spins, N, R, C, G, device):
