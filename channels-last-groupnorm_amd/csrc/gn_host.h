@@ -150,11 +150,11 @@ inline size_t resident_fwd_bytes(const Plan &p) {
 // All-to-all or two-level exchange: records a workgroup would poll in the all-to-all form (tiles x chunks per group x
 // groups per chunk); beyond this bound the polling traffic of the whole launch rivals the tensor itself.
 constexpr int kTwoLevelRecords = 1024;
-inline bool two_level_exchange(const Plan &p) {
+inline int64_t exchange_records(const Plan &p) {
   const int chunk_channels = p.lpr * p.vec;
-  const int64_t per_group = (int64_t)p.tiles * ((p.D - 1) / chunk_channels + 2);
-  return per_group * p.gmax > kTwoLevelRecords && p.tiles > 1;
+  return (int64_t)p.tiles * ((p.D - 1) / chunk_channels + 2) * p.gmax;
 }
+inline bool two_level_exchange(const Plan &p) { return exchange_records(p) > kTwoLevelRecords && p.tiles > 1; }
 // chunk_channels = channels per workgroup (lpr * vec): N * tiles * C = workgroups * chunk_channels
 // A tensor of several samples that is too large for one single-launch kernel may still be run as up to
 // kMaxBatches such launches over consecutive groups of samples (samples share nothing but dgamma / dbeta).

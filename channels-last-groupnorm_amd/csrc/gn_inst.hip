@@ -204,9 +204,25 @@ bool try_resident_fwd_nv(const FwdArgs &a, const FwdRecords &records, bool rolli
   if (rolling && cooperative_launches()) return false;  // the runtime refuses a cooperative grid larger than the device
   if (!resident_tiling(a.plan, a.plan.N, NV, slots, p, rolling)) return false;
   // A rolling launch works with 16 rows per lane while a set is at most an eighth of what is resident -- several sets are
-  // then in every phase at any time -- and with 32 beyond that, where a set's exchange weighs more: bf16 (8, 320, 128, 128)
-  // 35.8 us with 16 rows against 38.2 with 32, (3, 640, 200, 200) 77.9 against 72.4, float32 (2, 256, 256, 256) 57.2 / 49.5.
-  if (rolling && NV < 32 && exchange_chunks(p) * p.tiles > slots / 8) return false;
+  // then in every phase at any time -- and with 32 beyond that, where a set's exchange weighs more.  Where every workgroup polls
+  // every tile, the exchange weighs more already: there a sample of 18 tiles or more keeps 16 rows only while the whole launch is at
+  // most 4/3 of what is resident.  16 / 32 rows, us: with 1.2 - 1.3 of it bf16 (8, 320, 128, 128) 32.0 / 34.3, (6, 320, 100, 215)
+  // 33.2 / 37.3, float32 (2, 256, 200, 210) 33.3 / 33.2; with 1.35 - 1.5 (2, 256, 200, 220) 37.2 / 34.5, (2, 256, 200, 250) 51.1 / 41.7,
+  // bf16 (2, 512, 200, 230) 41.8 / 39.6; with 2.2 and more float32 (4, 256, 200, 250) 106 / 86, bf16 (16, 320, 128, 128) 75.1 / 71.0,
+  // (20, 320, 96, 96) 54.0 / 48.1.  Shorter samples: bf16 (24, 320, 92, 92), 17 tiles, 55.9 / 62.4, (30, 640, 80, 80), 13, 99 / 102.  In
+  // two levels float32 (4, 128, 256, 256) 52.4 / 60.9.  (With a residual, three workgroups of 16 rows to a CU, the first line alone, and
+  // for 16-bit gelu, which the vector ALUs bound and which wants the wavefronts: (16, 320, 128, 128) 83.6 / 93.8; float32, half as many
+  // elements to a row, (2, 256, 200, 250) 53.7 / 46.9, and 16-bit gelu_tanh (16, 320, 128, 128) 78.0 / 75.7.)
+  const int64_t set = exchange_chunks(p) * p.tiles;
+  constexpr int kTallSample = 18, kManyRecords = 900;
+  constexpr bool alu_bound = sizeof(elem_t) == 2 && ACT == GN_ACT_GELU;
+  const bool polled_by_all = ADD != kAddResidual && !alu_bound && !two_level_exchange(p) && p.tiles >= kTallSample;
+  if (rolling && NV < 32 && (set > slots / 8 || (polled_by_all && p.nblocks * 3 > (int64_t)slots * 4))) return false;
+  // A launch that is resident as a whole: the fourth workgroup per CU is not worth it where all of them poll nearly as many records
+  // as are merged in two levels.  16 / 32 rows, us: float32 (1, 256, 200, 250), 980 records, 21.6 / 19.3, with a channel addend
+  // 31.0 / 27.0; bf16 (1, 512, 200, 250) 23.4 / 22.7; but float32 (1, 256, 250, 256) in groups of 16, 750 records, 24.5 / 23.9 and
+  // (1, 256, 256, 256) in groups of 32, 512, 23.1 / 23.5; bf16 (1, 512, 240, 250), two levels, 23.8 / 25.1.
+  if (!rolling && NV == 16 && polled_by_all && exchange_records(p) > kManyRecords && p.nblocks > 3 * (kMaxResidentBlocks / 4)) return false;
   if (!resident_status()) return false;
   CapturedEpoch cap;
   if (!captured_epoch(a.stream, cap)) return false;

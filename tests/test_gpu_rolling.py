@@ -47,8 +47,8 @@ def _assert_set_by_set(x, kernel="fused_fwd"):
     assert workgroups > (512 if rows == 32 else 1024), (rows, workgroups)
 
 
-def _against_float64(x, w, b, G, y, mean, rstd, eps=1e-5):
-    """y = silu(normalised x): within one rounding to its type of a value that meets the float32 bar (1e-5)."""
+def _against_float64(x, w, b, G, y, mean, rstd, eps=1e-5, act=2):
+    """y = silu (act 3: gelu) of normalised x: within one rounding to its type of a value that meets the float32 bar (1e-5)."""
     N, R, C = x.shape
     half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 0.0}[x.dtype]
     for n in range(N):
@@ -57,7 +57,8 @@ def _against_float64(x, w, b, G, y, mean, rstd, eps=1e-5):
         var = (t - mu).square().mean((0, 2), keepdim=True)
         rs = (var + eps).rsqrt()
         assert err(mean[n], mu) <= 1e-5 and err(rstd[n], rs) <= 1e-5
-        z = torch.nn.functional.silu(((t - mu) * rs).view(R, C) * w.double() + b.double())
+        f = torch.nn.functional.gelu if act == 3 else torch.nn.functional.silu
+        z = f(((t - mu) * rs).view(R, C) * w.double() + b.double())
         assert bool(((y[n].double() - z).abs() <= half * z.abs() * 1.001 + 1e-5 * (z.abs() + 1.0)).all())
 
 
@@ -85,6 +86,35 @@ def test_against_float64_and_the_streaming_kernels(N, R, C, G, dtype, device):
     _close(y, y0, mean, mean0, rstd, rstd0)
     inplace = cabi_fwd(x, w, b, G, 1e-5, 2, y=x)[0]
     assert torch.equal(inplace, y)
+
+
+# Both sides of the lines between 16 and 32 rows per lane (256 CUs): workgroups of 16 rows beyond 4/3 of the 1024 resident ones, where
+# all poll all; tiles of a sample below and from 18 on; groups that are merged in two levels whatever the workgroups; 16-bit gelu.
+@pytest.mark.parametrize("N,R,C,G,dtype,act,rows", [
+    (2, 43520, 256, 16, torch.float32, 2, 16), (2, 43521, 256, 16, torch.float32, 2, 32), (6, 21500, 320, 32, torch.bfloat16, 2, 16),
+    (16, 16384, 320, 32, torch.bfloat16, 2, 32), (24, 8704, 320, 32, torch.float16, 2, 16), (24, 8705, 320, 32, torch.float16, 2, 32),
+    (4, 65536, 128, 32, torch.float32, 2, 16), (16, 16384, 320, 32, torch.bfloat16, 3, 16), (2, 43521, 256, 16, torch.float32, 3, 32)])
+def test_rows_per_lane(N, R, C, G, dtype, act, rows, device):
+    print("rolling rows", N, R, C, G, dtype, act, flush=True)
+    x, w, b = _inputs(N, R, C, dtype, device)
+    y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, act)
+    _assert_set_by_set(x)
+    assert "rows=%d " % rows in _cabi.last_launch(), _cabi.last_launch()
+    _against_float64(x, w, b, G, y, mean, rstd, act=act)
+
+
+# The same for launches that are resident as a whole: more than 768 workgroups of 16 rows that all poll more than 900 records (980;
+# 588 in wider groups; 720 workgroups; two levels).
+@pytest.mark.parametrize("N,R,C,G,dtype,rows", [(1, 50000, 256, 32, torch.float32, 32), (1, 50000, 256, 16, torch.float32, 16),
+                                                (1, 46000, 256, 32, torch.float32, 16), (1, 60000, 512, 32, torch.bfloat16, 16)])
+def test_rows_per_lane_of_one_resident_launch(N, R, C, G, dtype, rows, device):
+    x, w, b = _inputs(N, R, C, dtype, device)
+    y, mean, rstd = cabi_fwd(x, w, b, G, 1e-5, 2)
+    assert _cabi.last_launch().startswith("fused_fwd rows=%d " % rows), _cabi.last_launch()
+    _against_float64(x, w, b, G, y, mean, rstd)
+    s, mean, rstd = (t for i, t in enumerate(cabi_fwd_add(x, None, torch.zeros(N, C, device=device, dtype=dtype), w, b, G, 1e-5, 2)) if i != 1)
+    assert _cabi.last_launch().startswith("fused_fwd_add rows=%d " % rows), _cabi.last_launch()
+    _against_float64(x, w, b, G, s, mean, rstd)
 
 
 def test_with_fused_additions(device):
